@@ -95,6 +95,11 @@ struct kah_ctx {
   bool ib_done = false;
   std::vector<int64_t> ib_of_pair;   // IB face of each pair, or -1
   DBuf d_ib_solid, d_ib_snoff, d_ib_snb, d_ib_faces, d_ib_img, d_ib_cut, d_ib_cutw, d_ib_ssdf;
+  // overlap map ids of the sources, the work items and their partial sums
+  DBuf d_ib_smap, d_ib_imap, d_ib_swork, d_ib_swoff, d_ib_spart, d_ib_fwork, d_ib_fwoff, d_ib_fpart;
+  std::vector<int32_t> ib_solid_h, ib_snoff_h, ib_snb_h, ib_img_h;   // until upload_ib
+  std::vector<IbFaceDesc> ib_faces_h;
+  int ib_nsw = 0, ib_nfw = 0;
   // velocity-space adaptation: the root lattice of the velocity grids (valid when vs_ok)
   VsArgs vsa{};
   bool vs_ok = false;
@@ -178,7 +183,8 @@ struct kah_ctx {
                           &d_ents, &d_recds, &d_bc, &d_sw, &d_poff, &d_pcnt, &d_vtb, &d_ovmap,
                           &d_moff, &d_cmid, &d_benc, &d_xcells, &d_xoff, &d_xbuf, &d_xfluid,
                           &d_ib_solid, &d_ib_snoff, &d_ib_snb, &d_ib_faces, &d_ib_img,
-                          &d_ib_cut, &d_ib_cutw, &d_ib_ssdf};
+                          &d_ib_cut, &d_ib_cutw, &d_ib_ssdf, &d_ib_smap, &d_ib_imap, &d_ib_swork,
+                          &d_ib_swoff, &d_ib_spart, &d_ib_fwork, &d_ib_fwoff, &d_ib_fpart};
     int64_t t = 0;
     for (const DBuf* b : bufs) t += int64_t(b->bytes);
     for (const LevelBin* b : bins) t += int64_t(b->items.bytes);
@@ -540,8 +546,9 @@ struct Builder {
   }
 };
 
-// Immersed-boundary arrays of the topology: checked, then uploaded as device descriptors.
-// Fills C->ib_of_pair for the descriptor builder.
+// Immersed-boundary arrays of the topology: checked and turned into descriptors (upload_ib sends
+// them to the device once the overlap maps are known). Fills C->ib_of_pair for the descriptor
+// builder.
 int setup_ib(kah_ctx* C, const kah_topology* T) {
   const int D = C->D, NW = C->NW;
   const int64_t nc = T->n_cells;
@@ -552,8 +559,16 @@ int setup_ib(kah_ctx* C, const kah_topology* T) {
   C->ib_done = false;
   C->ib_of_pair.clear();
   for (DBuf* b : {&C->d_ib_solid, &C->d_ib_snoff, &C->d_ib_snb, &C->d_ib_faces, &C->d_ib_img,
-                  &C->d_ib_cut, &C->d_ib_cutw, &C->d_ib_ssdf})
+                  &C->d_ib_cut, &C->d_ib_cutw, &C->d_ib_ssdf, &C->d_ib_smap, &C->d_ib_imap,
+                  &C->d_ib_swork, &C->d_ib_swoff, &C->d_ib_spart, &C->d_ib_fwork, &C->d_ib_fwoff,
+                  &C->d_ib_fpart})
     b->release();
+  C->ib_nsw = C->ib_nfw = 0;
+  C->ib_solid_h.clear();
+  C->ib_snoff_h.clear();
+  C->ib_snb_h.clear();
+  C->ib_img_h.clear();
+  C->ib_faces_h.clear();
   const int64_t ns = T->n_ib_solid, nf = T->n_ib_faces;
   if (ns == 0 && nf == 0) return 0;
   if (ns < 0 || nf < 0 || ns > nc || nf > T->n_pairs)
@@ -648,21 +663,66 @@ int setup_ib(kah_ctx* C, const kah_topology* T) {
   }
   C->ib_ns = int(ns);
   C->ib_nf = int(nf);
-  if (ns > 0) {
-    KAH_TRY(C->upload(C->d_ib_solid, sol.data(), sol.size(), "ib solid cells"));
-    KAH_TRY(C->upload(C->d_ib_snoff, soff.data(), soff.size(), "ib solid neighbour offsets"));
-    KAH_TRY(C->upload(C->d_ib_snb, snb.data(), snb.size(), "ib solid neighbours"));
-  }
   if (nf > 0 && C->P.marching == KAH_MARCH_CIP)   // the limited boundary slopes
     KAH_TRY(C->alloc(C->d_ib_ssdf, sizeof(double) * size_t(C->ib_rows) * size_t(C->NDF),
                      "ib boundary slopes"));
-  if (nf > 0) {
-    KAH_TRY(C->upload(C->d_ib_faces, fd.data(), fd.size(), "ib faces"));
-    KAH_TRY(C->upload(C->d_ib_img, img.data(), img.size(), "ib image cells"));
-    if (!cut.empty()) {
-      KAH_TRY(C->upload(C->d_ib_cut, cut.data(), cut.size(), "ib cut cells"));
-      KAH_TRY(C->upload(C->d_ib_cutw, cutw.data(), cutw.size(), "ib cut areas"));
+  if (!cut.empty()) {
+    KAH_TRY(C->upload(C->d_ib_cut, cut.data(), cut.size(), "ib cut cells"));
+    KAH_TRY(C->upload(C->d_ib_cutw, cutw.data(), cutw.size(), "ib cut areas"));
+  }
+  C->ib_solid_h.swap(sol);
+  C->ib_snoff_h.swap(soff);
+  C->ib_snb_h.swap(snb);
+  C->ib_img_h.swap(img);
+  C->ib_faces_h.swap(fd);
+  return 0;
+}
+
+// Uploads the immersed-boundary descriptors with the overlap map ids of their sources
+// (map(owner cell, source cell)) and the work items of the kernels.
+template <class Map>
+int upload_ib(kah_ctx* C, const int64_t* voff, Map&& map) {
+  auto chunks = [&](std::vector<int2>& work, std::vector<int32_t>& woff, int64_t cell) {
+    const int64_t n = voff[cell + 1] - voff[cell];
+    const int q = int(woff.size()) - 1;
+    for (int64_t k = 0; k * IB_CHUNK < n; ++k) work.push_back(make_int2(q, int(k)));
+    woff.push_back(int32_t(work.size()));
+  };
+  std::vector<int2> work;
+  std::vector<int32_t> woff(1, 0), ids;
+  if (C->ib_ns > 0) {
+    for (int q = 0; q < C->ib_ns; ++q) {
+      for (int32_t x = C->ib_snoff_h[q]; x < C->ib_snoff_h[q + 1]; ++x)
+        ids.push_back(map(C->ib_solid_h[q], C->ib_snb_h[x]));
+      chunks(work, woff, C->ib_solid_h[q]);
     }
+    C->ib_nsw = int(work.size());
+    KAH_TRY(C->upload(C->d_ib_solid, C->ib_solid_h.data(), C->ib_solid_h.size(), "ib solid cells"));
+    KAH_TRY(C->upload(C->d_ib_snoff, C->ib_snoff_h.data(), C->ib_snoff_h.size(),
+                      "ib solid neighbour offsets"));
+    KAH_TRY(C->upload(C->d_ib_snb, C->ib_snb_h.data(), C->ib_snb_h.size(), "ib solid neighbours"));
+    KAH_TRY(C->upload(C->d_ib_smap, ids.data(), ids.size(), "ib solid overlap maps"));
+    KAH_TRY(C->upload(C->d_ib_swork, work.data(), work.size(), "ib solid work items"));
+    KAH_TRY(C->upload(C->d_ib_swoff, woff.data(), woff.size(), "ib solid work offsets"));
+    KAH_TRY(C->alloc(C->d_ib_spart, sizeof(double) * work.size() * size_t(C->NW), "ib solid sums"));
+  }
+  if (C->ib_nf > 0) {
+    work.clear();
+    woff.assign(1, 0);
+    ids.assign(C->ib_img_h.size(), -1);
+    for (IbFaceDesc& F : C->ib_faces_h) {
+      for (int32_t x = F.img_beg; x < F.img_beg + F.img_cnt; ++x)
+        ids[size_t(x)] = map(F.donor, C->ib_img_h[size_t(x)]);
+      F.smap = map(F.donor, F.solid);
+      chunks(work, woff, F.donor);
+    }
+    C->ib_nfw = int(work.size());
+    KAH_TRY(C->upload(C->d_ib_faces, C->ib_faces_h.data(), C->ib_faces_h.size(), "ib faces"));
+    KAH_TRY(C->upload(C->d_ib_img, C->ib_img_h.data(), C->ib_img_h.size(), "ib image cells"));
+    KAH_TRY(C->upload(C->d_ib_imap, ids.data(), ids.size(), "ib image overlap maps"));
+    KAH_TRY(C->upload(C->d_ib_fwork, work.data(), work.size(), "ib face work items"));
+    KAH_TRY(C->upload(C->d_ib_fwoff, woff.data(), woff.size(), "ib face work offsets"));
+    KAH_TRY(C->alloc(C->d_ib_fpart, sizeof(double) * work.size() * 2, "ib face sums"));
   }
   return 0;
 }
@@ -1024,6 +1084,7 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
             (ed.oth_mode == MI_LIMITED || ed.oth_mode == MI_UNLIMITED || ed.oth_mode == MI_PLAIN))
           ed.map = assign(c, ed.oth_cell);
     }
+    KAH_TRY(upload_ib(C, T->vs_offset, assign));
     C->map_entries = next;
   }
   C->d_ovmap.release();
@@ -1218,7 +1279,11 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
     for (int h = hoff[c]; h < hoff[c + 1]; ++h)
       pcnt[halves[h].slot] = walled[c] ? 1 : nchunks(c);
   for (int64_t p = 0; p < int64_t(C->ib_of_pair.size()); ++p)
-    if (C->ib_of_pair[size_t(p)] >= 0) pcnt[size_t(2 * p + 1)] = 1;   // written by the IB kernel
+    if (C->ib_of_pair[size_t(p)] >= 0) {   // written by k_ib_wall, a row per work item
+      const int64_t h = T->pair_here[p];
+      pcnt[size_t(2 * p + 1)] =
+          int32_t((T->vs_offset[h + 1] - T->vs_offset[h] + IB_CHUNK - 1) / IB_CHUNK);
+    }
   int64_t rows = 0;
   for (size_t s = 0; s < poff.size(); ++s) {
     poff[s] = rows;
@@ -1477,12 +1542,29 @@ int run_slope(kah_ctx* C, const DevArgs& A) {
 // update_solid_cell! and update_solid_neighbor! (src/Flux/Flux.jl:461-482)
 int run_ib(kah_ctx* C, const DevArgs& A) {
   if (C->ib_ns == 0 && C->ib_nf == 0) return 0;
-  KAH_TRY(C->hip(launch_ib(A, C->D, C->uni, C->f32, C->ib_ns, C->d_ib_solid.as<int32_t>(),
-                           C->d_ib_snoff.as<int32_t>(), C->d_ib_snb.as<int32_t>(), C->ib_nf,
-                           C->d_ib_faces.as<IbFaceDesc>(), C->d_ib_img.as<int32_t>(),
-                           C->d_ib_cut.as<int32_t>(), C->d_ib_cutw.as<double2>(),
-                           C->d_cmid.as<double>(), C->d_df[C->cur].p, C->d_df[1 - C->cur].p,
-                           C->stream),
+  IbArgs B{};
+  B.ns = C->ib_ns;
+  B.nsw = C->ib_nsw;
+  B.nfw = C->ib_nfw;
+  B.solid = C->d_ib_solid.as<int32_t>();
+  B.snoff = C->d_ib_snoff.as<int32_t>();
+  B.snb = C->d_ib_snb.as<int32_t>();
+  B.smap = C->d_ib_smap.as<int32_t>();
+  B.swork = C->d_ib_swork.as<int2>();
+  B.swoff = C->d_ib_swoff.as<int32_t>();
+  B.spart = C->d_ib_spart.as<double>();
+  B.faces = C->d_ib_faces.as<IbFaceDesc>();
+  B.img = C->d_ib_img.as<int32_t>();
+  B.imap = C->d_ib_imap.as<int32_t>();
+  B.fwork = C->d_ib_fwork.as<int2>();
+  B.fwoff = C->d_ib_fwoff.as<int32_t>();
+  B.fpart = C->d_ib_fpart.as<double>();
+  B.cut_idx = C->d_ib_cut.as<int32_t>();
+  B.cut_w = C->d_ib_cutw.as<double2>();
+  B.cmid = C->d_cmid.as<double>();
+  B.df_a = C->d_df[C->cur].p;
+  B.df_b = C->d_df[1 - C->cur].p;
+  KAH_TRY(C->hip(launch_ib(A, C->D, C->uni, C->f32, B, C->stream),
                  "immersed-boundary kernel launch"));
   if (C->ib_nf > 0) C->ib_done = true;
   return 0;

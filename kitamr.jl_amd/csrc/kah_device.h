@@ -2554,14 +2554,18 @@ inline hipError_t launch_fr_d(const DevArgs& A, const int32_t* cells, int n, int
 
 // ------------------------------------------------------------------ immersed boundary
 // update_solid_cell! and update_solid_neighbor! (src/Boundary/Immersed_boundary.jl:122-148,
-// 367-483) between the slopes and the flux: one workgroup per solid cell or IB face, the
-// threads striding over the velocity cells of the target grid; sources on other grids are
-// read through their key-interval overlap. Arithmetic in FP64.
+// 367-483) between the slopes and the flux, in three launches over (solid cell or IB face, chunk
+// of IB_THREADS velocity cells) work items, one velocity cell per thread: the solid cells; the
+// extrapolated wall-side f with the partial sums of the wall density; the wall Maxwellian and
+// the there-half moments. Few solid cells and faces (tens) carry grids of up to ~3*10^4
+// velocity cells, so one workgroup per cell or face left most of the chip idle behind a serial
+// chain of dependent loads (1640 us per step on a 14^3 sphere, 24 faces, grids of 4.5k to 30k
+// cells; 85 us like this, bound by the latency of the three dependent launches); sources on
+// other grids are read through the overlap maps instead of a key search per source. Arithmetic
+// in FP64.
 
-// threads per workgroup of the immersed-boundary kernels: few workgroups (one per solid cell
-// or IB face) over grids of up to ~10^4 velocity cells, so each gets 8 waves (more would cap
-// the registers below what the 3D kernels need)
-constexpr int IB_THREADS = 512;
+// threads per workgroup of the immersed-boundary kernels = velocity cells per work item
+constexpr int IB_THREADS = IB_CHUNK;
 
 // sum of one value over the IB_THREADS-thread workgroup (every thread gets the sum; fixed
 // order: wave sums, then the waves' partials in index order)
@@ -2576,88 +2580,105 @@ __device__ inline double block_sum_ib(double v, double* sh) {
   return t;
 }
 
+// sum over the work items [w0, w1) of their partials part[w*stride]: every lane of the wave gets
+// it (lane l adds the items w0+l, w0+l+64, ..., then the fixed shuffle tree)
+__device__ inline double items_sum(const double* part, int w0, int w1, int stride) {
+  double t = 0.0;
+  for (int w = w0 + int(threadIdx.x & 63); w < w1; w += 64) t += part[int64_t(w) * stride];
+  return wave_sum(t);
+}
+
 // sum_j wn_j (f_j + sdf_j . (x - x_j)) over the listed cells at velocity cell i, with
 // wn_j = w_j / sum w, w_j = max(0, u.l_j/|u|)^2, l_j = (x - x_j)/|x - x_j| (1/N when the sum
 // is zero): vs_extrapolate! with the weights of update_solid_cell! / image_df (:24-47,
 // :122-141, :378-395). Sums of products in index order, as Julia's dot and norm.
 template <int D, int NDF, bool UNI, class FT>
-__device__ inline void ib_extrapolate(const DevArgs& A, const int32_t* cells, int N,
-                                      const double* cmid, const double* x, int i, int li,
-                                      uint32_t ki, const double (&u)[D], double (&out)[NDF]) {
+__device__ inline void ib_extrapolate(const DevArgs& A, const int32_t* cells, const int32_t* maps,
+                                      int N, const double* cmid, const double* x, int i, int li,
+                                      const uint32_t* kp, const double (&u)[D],
+                                      double (&out)[NDF]) {
   double nu = u[0] * u[0];
 #pragma unroll
   for (int t = 1; t < D; ++t) nu += u[t] * u[t];
   nu = sqrt(nu);
   double w[8], ws = 0.0;
-  for (int j = 0; j < N; ++j) {
-    const double* xj = &cmid[int64_t(cells[j]) * D];
-    double l[D];
 #pragma unroll
-    for (int t = 0; t < D; ++t) l[t] = x[t] - xj[t];
-    double nl = l[0] * l[0];
+  for (int j = 0; j < 8; ++j) {
+    w[j] = 0.0;
+    if (j < N) {
+      const double* xj = &cmid[int64_t(cells[j]) * D];
+      double l[D];
 #pragma unroll
-    for (int t = 1; t < D; ++t) nl += l[t] * l[t];
-    nl = sqrt(nl);
+      for (int t = 0; t < D; ++t) l[t] = x[t] - xj[t];
+      double nl = l[0] * l[0];
 #pragma unroll
-    for (int t = 0; t < D; ++t) l[t] = l[t] / nl;
-    double d = u[0] * l[0];
+      for (int t = 1; t < D; ++t) nl += l[t] * l[t];
+      nl = sqrt(nl);
 #pragma unroll
-    for (int t = 1; t < D; ++t) d += u[t] * l[t];
-    const double r = d / nu;
-    const double c = (r != r) ? r : (r > 0.0 ? r : 0.0);
-    w[j] = c * c;
-    ws = (j == 0) ? w[j] : ws + w[j];
+      for (int t = 0; t < D; ++t) l[t] = l[t] / nl;
+      double d = u[0] * l[0];
+#pragma unroll
+      for (int t = 1; t < D; ++t) d += u[t] * l[t];
+      const double r = d / nu;
+      const double c = (r != r) ? r : (r > 0.0 ? r : 0.0);
+      w[j] = c * c;
+      ws = (j == 0) ? w[j] : ws + w[j];
+    }
   }
 #pragma unroll
   for (int k = 0; k < NDF; ++k) out[k] = 0.0;
-  for (int j = 0; j < N; ++j) {
-    const double wn = ws == 0.0 ? 1.0 / double(N) : w[j] / ws;
-    const Grid<D, NDF, UNI, FT> G(A, cells[j]);
-    const double* xj = &cmid[int64_t(cells[j]) * D];
-    double dx[D];
 #pragma unroll
-    for (int t = 0; t < D; ++t) dx[t] = x[t] - xj[t];
-    // the source cells over target cell i: same level or coarser (injection) with factor 1,
-    // finer ones with 2^-D per level (vs_extrapolate!'s walk)
-    for_overlap<D, NDF, UNI, FT>(G, i, li, ki, A.lmax, [&](int jj, double den, double rden) {
+  for (int j = 0; j < 8; ++j) {
+    if (j < N) {
+      const double wn = ws == 0.0 ? 1.0 / double(N) : w[j] / ws;
+      const Grid<D, NDF, UNI, FT> G(A, cells[j]);
+      const double* xj = &cmid[int64_t(cells[j]) * D];
+      double dx[D];
 #pragma unroll
-      for (int k = 0; k < NDF; ++k) {
-        double ddf = G.s(jj, k, 0) * dx[0];
+      for (int t = 0; t < D; ++t) dx[t] = x[t] - xj[t];
+      // the source cells over target cell i: same level or coarser (injection) with factor 1,
+      // finer ones with 2^-D per level (vs_extrapolate!'s walk)
+      for_overlap_m<D, NDF, UNI, FT>(A, G, maps[j], i, li, kp,
+                                     [&](int jj, double den, double rden) {
 #pragma unroll
-        for (int t = 1; t < D; ++t) ddf += G.s(jj, k, t) * dx[t];
-        double v = G.f(jj, k) + ddf;
-        if (den != 1.0) v = v * rden;   // exact: den is a power of two
-        out[k] += v * wn;
-      }
-    });
+        for (int k = 0; k < NDF; ++k) {
+          double ddf = G.s(jj, k, 0) * dx[0];
+#pragma unroll
+          for (int t = 1; t < D; ++t) ddf += G.s(jj, k, t) * dx[t];
+          double v = G.f(jj, k) + ddf;
+          if (den != 1.0) v = v * rden;   // exact: den is a power of two
+          out[k] += v * wn;
+        }
+      });
+    }
   }
 }
 
-// update_solid_cell!: f of solid cell s from its fluid face neighbours, written to both
-// state buffers (this step's IB faces read it; the next step keeps it), then w and prim
+// update_solid_cell!: f of one chunk of solid cell s from its fluid face neighbours, written to
+// both state buffers (this step's IB faces read it; the next step keeps it), and the chunk's
+// partial moments; k_ib_wall forms w and prim from them
 template <int D, int NDF, bool UNI, class FT>
-__global__ __launch_bounds__(IB_THREADS) void k_ib_solid(DevArgs A, const int32_t* __restrict__ solid,
-                                                  const int32_t* __restrict__ nb_off,
-                                                  const int32_t* __restrict__ nb,
-                                                  const double* __restrict__ cmid, FT* df_a,
-                                                  FT* df_b) {
+__global__ __launch_bounds__(IB_THREADS) void k_ib_solid(DevArgs A, IbArgs B) {
   constexpr int NW = D + 2;
   __shared__ double red[IB_THREADS / 64];
-  const int q = blockIdx.x;
-  const int s = solid[q];
-  const int b = nb_off[q], N = nb_off[q + 1] - b;
+  const int2 wk = B.swork[blockIdx.x];
+  const int s = B.solid[wk.x];
+  const int b = B.snoff[wk.x], N = B.snoff[wk.x + 1] - b;
   const Grid<D, NDF, UNI, FT> G(A, s);
   const int n = G.n;
-  const double* xs = &cmid[int64_t(s) * D];
+  const int i = wk.y * IB_THREADS + int(threadIdx.x);
   double m[NW];
 #pragma unroll
   for (int r = 0; r < NW; ++r) m[r] = 0.0;
-  for (int i = threadIdx.x; i < n; i += IB_THREADS) {
+  if (i < n) {
+    FT* df_a = static_cast<FT*>(B.df_a);
+    FT* df_b = static_cast<FT*>(B.df_b);
     double u[D];
 #pragma unroll
     for (int t = 0; t < D; ++t) u[t] = G.u(i, t);
     double f[NDF];
-    ib_extrapolate<D, NDF, UNI, FT>(A, nb + b, N, cmid, xs, i, G.lev(i), G.key(i), u, f);
+    ib_extrapolate<D, NDF, UNI, FT>(A, B.snb + b, B.smap + b, N, B.cmid, &B.cmid[int64_t(s) * D],
+                                    i, G.lev(i), G.keyp(i), u, f);
     double fs[NDF];
 #pragma unroll
     for (int k = 0; k < NDF; ++k) {
@@ -2666,76 +2687,57 @@ __global__ __launch_bounds__(IB_THREADS) void k_ib_solid(DevArgs A, const int32_
       df_b[G.off * NDF + int64_t(k) * n + i] = v;
       fs[k] = double(v);
     }
-    double mt[NW];
-    moment_terms<D, NDF, double>(G.wt(i), u, fs, mt);
-#pragma unroll
-    for (int r = 0; r < NW; ++r) m[r] += mt[r];
+    moment_terms<D, NDF, double>(G.wt(i), u, fs, m);
   }
-  double w[NW];
 #pragma unroll
-  for (int r = 0; r < NW; ++r) w[r] = block_sum_ib(m[r], red);
-  w[NW - 1] = 0.5 * w[NW - 1];
-  if (threadIdx.x == 0) {
-    double p[NW];
-    get_prim<D>(w, A.gamma, p);
-#pragma unroll
-    for (int r = 0; r < NW; ++r) {
-      A.w[int64_t(s) * NW + r] = w[r];
-      A.prim[int64_t(s) * NW + r] = p[r];
-    }
+  for (int r = 0; r < NW; ++r) {
+    const double t = block_sum_ib(m[r], red);
+    if (threadIdx.x == 0) B.spart[int64_t(blockIdx.x) * NW + r] = t;
   }
 }
 
-// update_solid_neighbor! of one IB face: image_df, boundary_slope! and its positivity
-// scaling, the wall Maxwellian of zero net mass flux through the wall (cvc_Mu /
-// cvc_density) and the cut-cell mixing (cvc_correction!). The SolidNeighbor's df goes to
-// the pseudo cell's rows of both state buffers; the face's there half (df .* u[dir] over
-// rot*u[dir] > 0, calc_flux with a solid there side, src/Flux/CAIDVM.jl:110-112) goes to
-// its half_fw row, which the flux kernel sums like any other.
+// the cut-cell slot of velocity cell i of a face, or -1 (the face's list is ascending)
+__device__ inline int ib_cut_of(const int32_t* ci, int cnt, int i) {
+  int lo = 0, hi = cnt - 1;
+  while (lo <= hi) {
+    const int mid = (lo + hi) >> 1;
+    const int v = ci[mid];
+    if (v == i) return mid;
+    if (v < i) lo = mid + 1; else hi = mid - 1;
+  }
+  return -1;
+}
+
+// update_solid_neighbor! of one chunk of an IB face, first part: image_df, boundary_slope! and
+// its positivity scaling give the extrapolated df at the wall (to the pseudo cell's rows), and
+// the chunk's share of the two flux sums of the wall density
 template <int D, int NDF, bool UNI, class FT>
-__global__ __launch_bounds__(IB_THREADS) void k_ib_face(DevArgs A, const IbFaceDesc* __restrict__ faces,
-                                                 const int32_t* __restrict__ img,
-                                                 const int32_t* __restrict__ cut_idx,
-                                                 const double2* __restrict__ cut_w,
-                                                 const double* __restrict__ cmid, FT* df_a,
-                                                 FT* df_b) {
-  constexpr int NW = D + 2;
+__global__ __launch_bounds__(IB_THREADS) void k_ib_face(DevArgs A, IbArgs B) {
   __shared__ double red[IB_THREADS / 64];
-  const IbFaceDesc F = faces[blockIdx.x];
+  const int2 wk = B.fwork[blockIdx.x];
+  const IbFaceDesc F = B.faces[wk.x];
   const Grid<D, NDF, UNI, FT> G(A, F.donor);
   const Grid<D, NDF, UNI, FT> S(A, F.solid);
   const Grid<D, NDF, UNI, FT> PS(A, F.pseudo);   // the donor's grid, copied
   const int n = G.n;
-  FT* pa = df_a + PS.off * NDF;
-  FT* pb = df_b + PS.off * NDF;
-  FT* ps = reinterpret_cast<FT*>(A.sdf) + PS.off * NDF * D;
-  const int32_t* ci = cut_idx + F.cut_beg;
-  // the cut-cell slot of velocity cell i, or -1 (the list is ascending)
-  auto cut_of = [&](int i) {
-    int lo = 0, hi = F.cut_cnt - 1;
-    while (lo <= hi) {
-      const int mid = (lo + hi) >> 1;
-      const int v = ci[mid];
-      if (v == i) return mid;
-      if (v < i) lo = mid + 1; else hi = mid - 1;
-    }
-    return -1;
-  };
-  // pass 1: the extrapolated df at the wall, and the two flux sums of the wall density
+  const int i = wk.y * IB_THREADS + int(threadIdx.x);
   double sf = 0.0, mur = 0.0;
-  for (int i = threadIdx.x; i < n; i += IB_THREADS) {
+  if (i < n) {
+    FT* pa = static_cast<FT*>(B.df_a) + PS.off * NDF;
+    FT* ps = reinterpret_cast<FT*>(A.sdf) + PS.off * NDF * D;
     double u[D];
 #pragma unroll
     for (int t = 0; t < D; ++t) u[t] = G.u(i, t);
     const int li = G.lev(i);
-    const uint32_t ki = G.key(i);
+    const uint32_t* kp = G.keyp(i);
     double im[NDF];
-    ib_extrapolate<D, NDF, UNI, FT>(A, img + F.img_beg, F.img_cnt, cmid, F.ip, i, li, ki, u, im);
+    ib_extrapolate<D, NDF, UNI, FT>(A, B.img + F.img_beg, B.imap + F.img_beg, F.img_cnt, B.cmid,
+                                    F.ip, i, li, kp, u, im);
     // boundary_slope!'s one-sided difference with the solid cell, walked across the grids
     double sLv[NDF];
 #pragma unroll
     for (int k = 0; k < NDF; ++k) sLv[k] = 0.0;
-    for_overlap<D, NDF, UNI, FT>(S, i, li, ki, A.lmax, [&](int jj, double den, double rden) {
+    for_overlap_m<D, NDF, UNI, FT>(A, S, F.smap, i, li, kp, [&](int jj, double den, double rden) {
 #pragma unroll
       for (int k = 0; k < NDF; ++k) {
         double d = G.f(i, k) - S.f(jj, k);
@@ -2763,26 +2765,70 @@ __global__ __launch_bounds__(IB_THREADS) void k_ib_face(DevArgs A, const IbFaceD
     for (int t = 1; t < D; ++t) vn += u[t] * F.nrm[t];
     double M[2];
     maxwell<D>(u, F.bc, A.K, M);
-    const int j = cut_of(i);
+    const int j = ib_cut_of(B.cut_idx + F.cut_beg, F.cut_cnt, i);
     if (j >= 0) {
-      const double2 gw = cut_w[F.cut_beg + j];
-      mur += gw.y * vn * M[0];
-      sf += gw.x * vn * aux[0];
+      const double2 gw = B.cut_w[F.cut_beg + j];
+      mur = gw.y * vn * M[0];
+      sf = gw.x * vn * aux[0];
     } else if (vn >= 0.0) {
-      mur += G.wt(i) * vn * M[0];
+      mur = G.wt(i) * vn * M[0];
     } else {
-      sf += G.wt(i) * vn * aux[0];
+      sf = G.wt(i) * vn * aux[0];
     }
   }
-  const double SF = block_sum_ib(sf, red);
-  const double MuR = block_sum_ib(mur, red);
+  const double t0 = block_sum_ib(sf, red);
+  const double t1 = block_sum_ib(mur, red);
+  if (threadIdx.x == 0) {
+    B.fpart[int64_t(blockIdx.x) * 2] = t0;
+    B.fpart[int64_t(blockIdx.x) * 2 + 1] = t1;
+  }
+}
+
+// update_solid_neighbor! of one chunk, second part, after the face's flux sums are complete: the
+// wall Maxwellian of zero net mass flux (cvc_Mu / cvc_density) on u.n >= 0, the cut-cell mixing
+// (cvc_correction!) and the chunk's row of the face's there half (df .* u[dir] over
+// rot*u[dir] > 0, calc_flux with a solid there side, src/Flux/CAIDVM.jl:110-112), which the
+// flux kernel sums like any other. The SolidNeighbor's df goes to the pseudo cell's rows of both
+// state buffers. The workgroups after the faces' take one solid cell each: w and prim from the
+// partial moments of k_ib_solid.
+template <int D, int NDF, bool UNI, class FT>
+__global__ __launch_bounds__(IB_THREADS) void k_ib_wall(DevArgs A, IbArgs B) {
+  constexpr int NW = D + 2;
+  if (int(blockIdx.x) >= B.nfw) {
+    const int q = int(blockIdx.x) - B.nfw;
+    if (threadIdx.x >= 64) return;
+    double w[NW], p[NW];
+#pragma unroll
+    for (int r = 0; r < NW; ++r) w[r] = items_sum(B.spart + r, B.swoff[q], B.swoff[q + 1], NW);
+    w[NW - 1] = 0.5 * w[NW - 1];
+    if (threadIdx.x == 0) {
+      const int s = B.solid[q];
+      get_prim<D>(w, A.gamma, p);
+#pragma unroll
+      for (int r = 0; r < NW; ++r) {
+        A.w[int64_t(s) * NW + r] = w[r];
+        A.prim[int64_t(s) * NW + r] = p[r];
+      }
+    }
+    return;
+  }
+  __shared__ double red[IB_THREADS / 64];
+  const int2 wk = B.fwork[blockIdx.x];
+  const IbFaceDesc F = B.faces[wk.x];
+  const Grid<D, NDF, UNI, FT> G(A, F.donor);
+  const Grid<D, NDF, UNI, FT> PS(A, F.pseudo);
+  const int n = G.n;
+  const int w0 = B.fwoff[wk.x], w1 = B.fwoff[wk.x + 1];
+  const double SF = items_sum(B.fpart, w0, w1, 2);
+  const double MuR = items_sum(B.fpart + 1, w0, w1, 2);
   const double rho = -SF / MuR;
-  // pass 2: the wall Maxwellian on u.n >= 0, the cut-cell mix, the there-half moments. Each
-  // thread revisits the velocity cells it wrote in pass 1, so no barrier is needed here.
+  const int i = wk.y * IB_THREADS + int(threadIdx.x);
   double hm[NW];
 #pragma unroll
   for (int r = 0; r < NW; ++r) hm[r] = 0.0;
-  for (int i = threadIdx.x; i < n; i += IB_THREADS) {
+  if (i < n) {
+    FT* pa = static_cast<FT*>(B.df_a) + PS.off * NDF;
+    FT* pb = static_cast<FT*>(B.df_b) + PS.off * NDF;
     double u[D];
 #pragma unroll
     for (int t = 0; t < D; ++t) u[t] = G.u(i, t);
@@ -2791,21 +2837,18 @@ __global__ __launch_bounds__(IB_THREADS) void k_ib_face(DevArgs A, const IbFaceD
     for (int t = 1; t < D; ++t) vn += u[t] * F.nrm[t];
     double M[2];
     maxwell<D>(u, F.bc, A.K, M);
-    const int j = cut_of(i);
+    const int j = ib_cut_of(B.cut_idx + F.cut_beg, F.cut_cnt, i);
     double out[NDF];
 #pragma unroll
     for (int k = 0; k < NDF; ++k) {
       const double Mk = M[k] * rho;
       const double g = double(pa[k * n + i]);
       if (j >= 0) {
-        const double2 gw = cut_w[F.cut_beg + j];
+        const double2 gw = B.cut_w[F.cut_beg + j];
         out[k] = (gw.x * g + gw.y * Mk) / (gw.x + gw.y);
       } else {
         out[k] = vn >= 0.0 ? Mk : g;
       }
-    }
-#pragma unroll
-    for (int k = 0; k < NDF; ++k) {
       const FT v = FT(out[k]);
       pa[k * n + i] = v;
       pb[k * n + i] = v;
@@ -2813,38 +2856,34 @@ __global__ __launch_bounds__(IB_THREADS) void k_ib_face(DevArgs A, const IbFaceD
     }
     const double ud = pick<D>(u, F.dir);
     if (F.rot * ud > 0.0) {
-      double mic[NDF], mt[NW];
+      double mic[NDF];
 #pragma unroll
       for (int k = 0; k < NDF; ++k) mic[k] = out[k] * ud;
-      moment_terms<D, NDF, double>(G.wt(i), u, mic, mt);
-#pragma unroll
-      for (int r = 0; r < NW; ++r) hm[r] += mt[r];
+      moment_terms<D, NDF, double>(G.wt(i), u, mic, hm);
     }
   }
-  double tot[NW];
 #pragma unroll
-  for (int r = 0; r < NW; ++r) tot[r] = block_sum_ib(hm[r], red);
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int r = 0; r < NW; ++r) A.half_fw[A.part_off[F.slot] * NW + r] = tot[r];
+  for (int r = 0; r < NW; ++r) {
+    const double t = block_sum_ib(hm[r], red);
+    if (threadIdx.x == 0) A.half_fw[(A.part_off[F.slot] + wk.y) * NW + r] = t;
   }
 }
 
 template <int D, int NDF, bool UNI, class FT>
-inline hipError_t launch_ib_t(const DevArgs& A, int ns, const int32_t* solid,
-                              const int32_t* nb_off, const int32_t* nb, int nf,
-                              const IbFaceDesc* faces, const int32_t* img, const int32_t* cut_idx,
-                              const double2* cut_w, const double* cmid, void* df_a, void* df_b,
-                              hipStream_t st) {
-  if (ns > 0) {
-    hipLaunchKernelGGL((k_ib_solid<D, NDF, UNI, FT>), dim3(ns), dim3(IB_THREADS), 0, st, A, solid, nb_off, nb,
-                       cmid, static_cast<FT*>(df_a), static_cast<FT*>(df_b));
+inline hipError_t launch_ib_t(const DevArgs& A, const IbArgs& B, hipStream_t st) {
+  if (B.nsw > 0) {
+    hipLaunchKernelGGL((k_ib_solid<D, NDF, UNI, FT>), dim3(B.nsw), dim3(IB_THREADS), 0, st, A, B);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  if (nf > 0) {
-    hipLaunchKernelGGL((k_ib_face<D, NDF, UNI, FT>), dim3(nf), dim3(IB_THREADS), 0, st, A, faces, img, cut_idx,
-                       cut_w, cmid, static_cast<FT*>(df_a), static_cast<FT*>(df_b));
+  if (B.nfw > 0) {
+    hipLaunchKernelGGL((k_ib_face<D, NDF, UNI, FT>), dim3(B.nfw), dim3(IB_THREADS), 0, st, A, B);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (B.nfw + B.ns > 0) {
+    hipLaunchKernelGGL((k_ib_wall<D, NDF, UNI, FT>), dim3(B.nfw + B.ns), dim3(IB_THREADS), 0, st,
+                       A, B);
     return hipGetLastError();
   }
   return hipSuccess;

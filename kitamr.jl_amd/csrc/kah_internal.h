@@ -121,8 +121,8 @@ struct IbFaceDesc {     // one IB face (donor, SolidNeighbor), rebuilt every ste
   int32_t dir;
   int32_t img_beg, img_cnt;   // image stencil (fluid neighbours, then the donor)
   int32_t cut_beg, cut_cnt;   // cut velocity cells
-  int32_t slot;         // half_fw row of the face's there half (pair*2 + 1)
-  int32_t pad;
+  int32_t slot;         // half flux of the face's there half (pair*2 + 1)
+  int32_t smap;         // overlap map id of (donor's grid, solid cell's grid)
   int64_t row;          // first row of the face in the per-face velocity arrays (ib_ssdf)
   double apd;           // aux_point[dir]
   double rot;

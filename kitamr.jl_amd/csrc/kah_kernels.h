@@ -154,11 +154,33 @@ hipError_t launch_overlap_map(const DevArgs& A, int dim, const OvJob* jobs, int 
                               uint32_t* map, hipStream_t st);
 hipError_t launch_macro_slope(const DevArgs& A, int dim, bool uni, bool f32, const int32_t* cells,
                               int n, double* sw, hipStream_t st);
-// immersed boundary (shared or adapted velocity grids): the ns solid cells, then the nf IB faces;
-// both write f to the two state buffers df_a and df_b
-hipError_t launch_ib(const DevArgs& A, int dim, bool uni, bool f32, int ns, const int32_t* solid,
-                     const int32_t* nb_off, const int32_t* nb, int nf, const IbFaceDesc* faces,
-                     const int32_t* img, const int32_t* cut_idx, const double2* cut_w,
-                     const double* cmid, void* df_a, void* df_b, hipStream_t st);
+// Immersed boundary (shared or adapted velocity grids): ns solid cells and the IB faces, each as
+// work items of IB_CHUNK velocity cells (nsw, nfw of them; work[x] = (solid cell or face index,
+// chunk), the items of index q are [woff[q], woff[q+1])), with their overlap map ids and the
+// partial sums of each item. Both state buffers df_a (this step's) and df_b are written.
+constexpr int IB_CHUNK = 256;
+struct IbArgs {
+  int32_t ns, nsw, nfw;
+  const int32_t* solid;     // [ns] cells
+  const int32_t* snoff;     // [ns+1] first fluid neighbour of each
+  const int32_t* snb;       // fluid neighbours
+  const int32_t* smap;      // overlap map id of (solid cell's grid, neighbour's grid)
+  const int2* swork;
+  const int32_t* swoff;
+  double* spart;            // [nsw*(D+2)] moments
+  const IbFaceDesc* faces;
+  const int32_t* img;       // image stencils
+  const int32_t* imap;      // overlap map id of (donor's grid, image cell's grid)
+  const int2* fwork;
+  const int32_t* fwoff;
+  double* fpart;            // [nfw*2] the two flux sums of the wall density
+  const int32_t* cut_idx;
+  const double2* cut_w;
+  const double* cmid;
+  void* df_a;
+  void* df_b;
+};
+hipError_t launch_ib(const DevArgs& A, int dim, bool uni, bool f32, const IbArgs& B,
+                     hipStream_t st);
 
 }  // namespace kah

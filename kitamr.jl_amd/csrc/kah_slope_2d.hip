@@ -61,14 +61,9 @@ hipError_t launch_vs_project_2d(const DevArgs& A, bool uni, const int32_t* cells
              : launch_vs_project_t<2, 2, false, double>(A, cells, n, lds, scratch, dfw, st);
 }
 
-hipError_t launch_ib_2d(const DevArgs& A, bool uni, int ns, const int32_t* solid,
-                     const int32_t* nb_off, const int32_t* nb, int nf, const IbFaceDesc* faces,
-                     const int32_t* img, const int32_t* cut_idx, const double2* cut_w,
-                     const double* cmid, void* df_a, void* df_b, hipStream_t st) {
-  return uni ? launch_ib_t<2, 2, true, double>(A, ns, solid, nb_off, nb, nf, faces, img,
-                                                 cut_idx, cut_w, cmid, df_a, df_b, st)
-             : launch_ib_t<2, 2, false, double>(A, ns, solid, nb_off, nb, nf, faces, img,
-                                                  cut_idx, cut_w, cmid, df_a, df_b, st);
+hipError_t launch_ib_2d(const DevArgs& A, bool uni, const IbArgs& B, hipStream_t st) {
+  return uni ? launch_ib_t<2, 2, true, double>(A, B, st)
+             : launch_ib_t<2, 2, false, double>(A, B, st);
 }
 
 }  // namespace kah

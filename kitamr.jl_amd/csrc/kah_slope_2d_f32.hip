@@ -56,14 +56,9 @@ hipError_t launch_vs_project_2d_f32(const DevArgs& A, bool uni, const int32_t* c
              : launch_vs_project_t<2, 2, false, float>(A, cells, n, lds, scratch, dfw, st);
 }
 
-hipError_t launch_ib_2d_f32(const DevArgs& A, bool uni, int ns, const int32_t* solid,
-                     const int32_t* nb_off, const int32_t* nb, int nf, const IbFaceDesc* faces,
-                     const int32_t* img, const int32_t* cut_idx, const double2* cut_w,
-                     const double* cmid, void* df_a, void* df_b, hipStream_t st) {
-  return uni ? launch_ib_t<2, 2, true, float>(A, ns, solid, nb_off, nb, nf, faces, img,
-                                                 cut_idx, cut_w, cmid, df_a, df_b, st)
-             : launch_ib_t<2, 2, false, float>(A, ns, solid, nb_off, nb, nf, faces, img,
-                                                  cut_idx, cut_w, cmid, df_a, df_b, st);
+hipError_t launch_ib_2d_f32(const DevArgs& A, bool uni, const IbArgs& B, hipStream_t st) {
+  return uni ? launch_ib_t<2, 2, true, float>(A, B, st)
+             : launch_ib_t<2, 2, false, float>(A, B, st);
 }
 
 }  // namespace kah
