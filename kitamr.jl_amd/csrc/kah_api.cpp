@@ -81,7 +81,7 @@ struct kah_ctx {
   int64_t n_grids = 1, grid_cells = 0, map_entries = 0;   // distinct grids, their cells, map entries
   DBuf d_df[2], d_sdf, d_oflux, d_vflux, d_psflux, d_w, d_prim, d_qf, d_half, d_rho, d_res, d_scratch;
   DBuf d_cpre;   // per-cell prologue records of the fused step (k_cell_pre)
-  DBuf d_sl, d_slnb, d_hoff, d_halves, d_eoff, d_ents, d_recds, d_bc, d_sw, d_poff, d_pcnt;
+  DBuf d_sl, d_slnb, d_hoff, d_halves, d_eoff, d_ents, d_recds, d_bc, d_sw, d_poff;
   DBuf d_vtb, d_ovmap, d_moff;
   // ghost-exchange buffers: cell midpoints and bound_enc on the device, and the staging of
   // kah_pack_mirrors / kah_unpack_mirrors (grown on demand)
@@ -180,7 +180,7 @@ struct kah_ctx {
     const DBuf* bufs[] = {&d_fluid, &d_voff, &d_gu, &d_gw, &d_glev, &d_gkey, &d_gof, &d_df[0], &d_df[1],
                           &d_sdf, &d_oflux, &d_vflux, &d_psflux, &d_w, &d_prim, &d_qf, &d_half, &d_rho,
                           &d_res, &d_scratch, &d_cpre, &d_sl, &d_slnb, &d_hoff, &d_halves, &d_eoff,
-                          &d_ents, &d_recds, &d_bc, &d_sw, &d_poff, &d_pcnt, &d_vtb, &d_ovmap,
+                          &d_ents, &d_recds, &d_bc, &d_sw, &d_poff, &d_vtb, &d_ovmap,
                           &d_moff, &d_cmid, &d_benc, &d_xcells, &d_xoff, &d_xbuf, &d_xfluid,
                           &d_ib_solid, &d_ib_snoff, &d_ib_snb, &d_ib_faces, &d_ib_img,
                           &d_ib_cut, &d_ib_cutw, &d_ib_ssdf, &d_ib_smap, &d_ib_imap, &d_ib_swork,
@@ -1132,7 +1132,6 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
   KAH_TRY(C->upload(C->d_hoff, hoff.data(), hoff.size(), "half offsets"));
   KAH_TRY(C->upload(C->d_halves, halves.data(), halves.size(), "half descriptors"));
   KAH_TRY(C->upload(C->d_eoff, eoff.data(), eoff.size(), "entry offsets"));
-  KAH_TRY(C->upload(C->d_ents, ents.data(), ents.size(), "entry descriptors"));
   KAH_TRY(C->upload(C->d_recds, T->cell_ds, size_t(nc * D), "cell ds"));
   KAH_TRY(C->upload(C->d_cmid, T->cell_mid, size_t(nc * D), "cell midpoints"));
   KAH_TRY(C->upload(C->d_benc, T->bound_enc, size_t(nc), "bound_enc"));
@@ -1291,7 +1290,12 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
   }
   C->part_rows = rows;
   KAH_TRY(C->upload(C->d_poff, poff.data(), poff.size(), "partial offsets"));
-  KAH_TRY(C->upload(C->d_pcnt, pcnt.data(), pcnt.size(), "partial counts"));
+  for (EntryDesc& e : ents)
+    for (int sd = 0; sd < 2; ++sd) {
+      e.row[sd] = poff[size_t(2 * e.pair + sd)];
+      e.rows[sd] = pcnt[size_t(2 * e.pair + sd)];
+    }
+  KAH_TRY(C->upload(C->d_ents, ents.data(), ents.size(), "entry descriptors"));
 
   // state buffers
   const int64_t NDF = C->NDF, NW = C->NW;
@@ -1429,7 +1433,6 @@ DevArgs make_args(kah_ctx* C, double dt) {
   A.qf = C->d_qf.as<double>();
   A.half_fw = C->d_half.as<double>();
   A.part_off = C->d_poff.as<int64_t>();
-  A.part_cnt = C->d_pcnt.as<int32_t>();
   A.rho_w = C->d_rho.as<double>();
   A.res = C->d_res.as<double>();
   A.cpre = C->d_cpre.p ? C->d_cpre.as<double>() : nullptr;

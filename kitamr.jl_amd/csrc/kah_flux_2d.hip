@@ -10,9 +10,7 @@ hipError_t launch_flux_relax_2d(const DevArgs& A, bool uni, const int32_t* cells
 }
 
 hipError_t launch_cell_pre_2d(const DevArgs& A, const int32_t* cells, int n, hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_cell_pre<2>, dim3((n + 255) / 256), dim3(256), 0, st, A, cells, n);
-  return hipGetLastError();
+  return launch_cell_pre_t<2>(A, cells, n, st);
 }
 
 }  // namespace kah

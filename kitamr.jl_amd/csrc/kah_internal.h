@@ -96,7 +96,7 @@ struct HalfDesc {       // one half flux computed by its owner cell in K1
 };
 
 struct EntryDesc {      // one face side of a fluid cell, gathered in K2
-  int32_t pair;         // half fluxes at half_fw[pair*2 + 0/1]
+  int32_t pair;
   int32_t oth_cell;     // data cell of the other side (-1 for domain faces)
   int32_t side;         // 0: the cell is "here" (adds), 1: "there" (subtracts)
   int32_t own_mode;     // MI_* of the cell's own upwind set
@@ -106,6 +106,8 @@ struct EntryDesc {      // one face side of a fluid cell, gathered in K2
   int32_t map;          // overlap map id of (owner grid, other grid), MAP_SAME, or -1
   double rot;
   double area;          // signed face area, rot*A (or rot*A/2^(DIM-1))
+  int64_t row[2];       // first partial row in half_fw of the face's here / there half flux
+  int32_t rows[2];      // their row counts
   double fmid[3];
   double xown[3], dsown[3];
   double xoth[3], dsoth[3];

@@ -39,7 +39,6 @@ struct DevArgs {
   double* qf;
   double* half_fw;          // partial half-flux sums: row part_off[slot]+chunk, D+2 each
   const int64_t* part_off;  // [npairs*2] first partial row of each half flux
-  const int32_t* part_cnt;  // [npairs*2] number of partial rows (velocity chunks)
   double* rho_w;            // [npairs]
   double* res;              // [nc*2*(D+2)] residual terms of the last iterate
   // per-cell prologue of the fused step (k_cell_pre), cpre_len(D) doubles per cell:
