@@ -28,10 +28,64 @@
 namespace kah {
 
 // ------------------------------------------------------------------ reductions
-__device__ inline double wave_sum(double v) {
+// Lane exchanges of the reductions without LDS: the gfx950 row swaps for lane bits 5 and 4, DPP
+// moves for the lower four (a shuffle through LDS costs a round trip of some hundred cycles and
+// two selects per 32 bits). xor_lane<O> is the value of lane ^ O.
+template <int O>
+__device__ inline uint32_t xor_lane32(uint32_t x) {
+  static_assert(O == 8 || O == 4 || O == 2 || O == 1, "within a row of 16 lanes");
+  if constexpr (O == 8) return __builtin_amdgcn_update_dpp(0u, x, 0x128, 0xf, 0xf, true);
+  if constexpr (O == 4) {   // lanes with bit 2 clear read lane + 4, the others lane - 4
+    const uint32_t t = __builtin_amdgcn_update_dpp(0u, x, 0x104, 0xf, 0x5, false);
+    return __builtin_amdgcn_update_dpp(t, x, 0x114, 0xf, 0xa, false);
+  }
+  if constexpr (O == 2) return __builtin_amdgcn_update_dpp(0u, x, 0x4e, 0xf, 0xf, true);
+  return __builtin_amdgcn_update_dpp(0u, x, 0xb1, 0xf, 0xf, true);
+}
+template <int O>
+__device__ inline double xor_lane(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = xor_lane32<O>(uint32_t(b)), hi = xor_lane32<O>(uint32_t(b >> 32));
+  return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
+}
+// a and b with the upper lanes of a (lane bit O set) exchanged for the lower lanes of b: a lane
+// with the bit clear ends with its own a and its partner's a, one with the bit set with its
+// partner's b and its own b
+template <int O>
+__device__ inline void swap_halves(double& a, double& b) {
+  static_assert(O == 32 || O == 16, "row swaps");
+  const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+  uint32_t r[2][2];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t p = uint32_t(x >> (32 * h)), q = uint32_t(y >> (32 * h));
+    if constexpr (O == 32) {
+      const auto t = __builtin_amdgcn_permlane32_swap(p, q, false, false);
+      r[0][h] = t[0];
+      r[1][h] = t[1];
+    } else {
+      const auto t = __builtin_amdgcn_permlane16_swap(p, q, false, false);
+      r[0][h] = t[0];
+      r[1][h] = t[1];
+    }
+  }
+  a = __builtin_bit_cast(double, (uint64_t(r[0][1]) << 32) | r[0][0]);
+  b = __builtin_bit_cast(double, (uint64_t(r[1][1]) << 32) | r[1][0]);
+}
+// (own, partner) values of v across lane bit O, in either order: for symmetric operations
+template <int O>
+__device__ inline void both_lanes(double v, double& a, double& b) {
+  a = b = v;
+  if constexpr (O >= 16) swap_halves<O>(a, b);
+  else b = xor_lane<O>(v);
+}
+
+template <int O = 32>
+__device__ inline double wave_sum(double v) {
+  double a, b;
+  both_lanes<O>(v, a, b);
+  if constexpr (O == 1) return a + b;
+  else return wave_sum<O / 2>(a + b);
 }
 
 // Workgroup sum of the first cnt of CNT per-thread partials. out[q] (LDS) receives the
@@ -51,17 +105,18 @@ __device__ inline double two_sum(double a, double b, double& err) {
   return s;
 }
 
-// Sum over the 64 lanes of a wave of (s, e) pairs (a value and its running error): an xor
-// butterfly whose every level adds with two_sum and carries the errors, so every lane ends
-// with the same compensated total s + e.
+// Sum over the lanes that share the lane bits above O of (s, e) pairs (a value and its running
+// error): an xor butterfly whose every level adds with two_sum and carries the errors, so every
+// lane ends with the same compensated total s + e.
+template <int O = 32>
 __device__ inline void wave_sum2(double& s, double& e) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const double so = __shfl_xor(s, o, 64);
-    const double eo = __shfl_xor(e, o, 64);
-    double err;
-    s = two_sum(s, so, err);
-    e = (e + eo) + err;
+  if constexpr (O >= 1) {
+    double sa, sb, ea, eb, err;
+    both_lanes<O>(s, sa, sb);
+    both_lanes<O>(e, ea, eb);
+    s = two_sum(sa, sb, err);
+    e = (ea + eb) + err;
+    wave_sum2<O / 2>(s, e);
   }
 }
 
@@ -81,43 +136,52 @@ constexpr int red_stride(int cnt) { return pow2_at_least(cnt) <= 64 ? pow2_at_le
 // bits finishes it. P/2 + P/4 + ... + 1 + log2(64/P) exchanges instead of P*6.
 // The levels are one template instance per value count M, each writing fresh arrays of M/2,
 // so that every index is a compile-time constant: a loop over the levels, left to the
-// unroller, stays rolled for 32 values and puts the arrays in scratch memory.
-template <int M>
+// unroller, stays rolled for 32 values and puts the arrays in scratch memory. At the levels of
+// lane bits 5 and 4 one row swap per 32 bits both selects and exchanges. FIRST: all errors 0.
+// With LDS shuffles and selects a third of the slope kernel's instructions were here; measured
+// with them and without: the CIP flux kernel (a sum of 14 values per Newton step) 108 -> 69 us
+// on 40^2 leaves with 24^2 velocity cells, a 3D cell's 80 sums 175 -> 158 us, 2D kernels 1-3 %.
+template <int M, int O, bool FIRST>
 __device__ inline void scatter_levels(const double (&v)[M], const double (&e)[M], double& s0,
-                                      double& e0, int lane, int o) {
+                                      double& e0, int lane) {
   if constexpr (M == 1) {
     s0 = v[0];
     e0 = e[0];
   } else {
-    const bool up = (lane & o) != 0;
     double nv[M / 2], ne[M / 2];
 #pragma unroll
     for (int j = 0; j < M / 2; ++j) {
-      const double lo = v[j], hi = v[M / 2 + j], loe = e[j], hie = e[M / 2 + j];
-      const double keep = up ? hi : lo, ke = up ? hie : loe;
-      const double send = up ? lo : hi, se = up ? loe : hie;
-      const double recv = __shfl_xor(send, o, 64), re = __shfl_xor(se, o, 64);
+      double a = v[j], b = v[M / 2 + j], ea = 0.0, eb = 0.0;
+      if constexpr (!FIRST) {
+        ea = e[j];
+        eb = e[M / 2 + j];
+      }
+      if constexpr (O >= 16) {
+        swap_halves<O>(a, b);
+        if constexpr (!FIRST) swap_halves<O>(ea, eb);
+      } else {
+        const bool up = (lane & O) != 0;
+        const double send = up ? a : b, se = up ? ea : eb;
+        a = up ? b : a;
+        ea = up ? eb : ea;
+        b = xor_lane<O>(send);
+        eb = xor_lane<O>(se);
+      }
       double err;
-      nv[j] = two_sum(keep, recv, err);
-      ne[j] = (ke + re) + err;
+      nv[j] = two_sum(a, b, err);
+      ne[j] = FIRST ? err : (ea + eb) + err;
     }
-    scatter_levels<M / 2>(nv, ne, s0, e0, lane, o >> 1);
+    scatter_levels<M / 2, O / 2, false>(nv, ne, s0, e0, lane);
   }
 }
 
+// v: the values of each lane (errors 0); v[0], e[0] receive the sum described above
 template <int P>
 __device__ inline void wave_scatter2(double (&v)[P], double (&e)[P]) {
   static_assert(P >= 1 && P <= 64 && (P & (P - 1)) == 0, "power of two up to 64");
-  const int lane = threadIdx.x & 63;
   double s0, e0;
-  scatter_levels<P>(v, e, s0, e0, lane, 32);
-#pragma unroll
-  for (int o = 32 / P; o > 0; o >>= 1) {
-    const double so = __shfl_xor(s0, o, 64), eo = __shfl_xor(e0, o, 64);
-    double err;
-    s0 = two_sum(s0, so, err);
-    e0 = (e0 + eo) + err;
-  }
+  scatter_levels<P, 32, true>(v, e, s0, e0, threadIdx.x & 63);
+  wave_sum2<32 / P>(s0, e0);
   v[0] = s0;
   e[0] = e0;
 }
@@ -150,7 +214,7 @@ __device__ inline double block_totals(const double (&vals)[CNT], int cnt, double
     for (int q = 0; q < CNT; ++q) {
       if (q < cnt) {
         double v = vals[q], e = 0.0;
-        wave_sum2(v, e);
+        wave_sum2<>(v, e);
         if (lane == 0) {
           red[(wv * CNT + q) * 2] = v;
           red[(wv * CNT + q) * 2 + 1] = e;
@@ -2611,7 +2675,7 @@ constexpr int IB_THREADS = IB_CHUNK;
 // sum of one value over the IB_THREADS-thread workgroup (every thread gets the sum; fixed
 // order: wave sums, then the waves' partials in index order)
 __device__ inline double block_sum_ib(double v, double* sh) {
-  v = wave_sum(v);
+  v = wave_sum<>(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -2626,7 +2690,7 @@ __device__ inline double block_sum_ib(double v, double* sh) {
 __device__ inline double items_sum(const double* part, int w0, int w1, int stride) {
   double t = 0.0;
   for (int w = w0 + int(threadIdx.x & 63); w < w1; w += 64) t += part[int64_t(w) * stride];
-  return wave_sum(t);
+  return wave_sum<>(t);
 }
 
 // sum_j wn_j (f_j + sdf_j . (x - x_j)) over the listed cells at velocity cell i, with
