@@ -45,9 +45,9 @@ struct DBuf {
 
 struct LevelBin {
   int level;
-  int maxh;
-  int wpi = 4;    // chunked kernel: waves per workgroup (3 or 4)
-  int n;          // work items: cells (per-cell kernel) or (cell, chunk) pairs
+  int maxh;       // per-cell kernel: half fluxes; chunked kernel: its kind
+  int waves = 4;  // chunked kernel: waves per workgroup
+  int n;          // work items: cells (per-cell kernel) or chunks
   bool chunked;
   DBuf items;
 };
@@ -82,7 +82,7 @@ struct kah_ctx {
   DBuf d_df[2], d_sdf, d_oflux, d_vflux, d_psflux, d_w, d_prim, d_qf, d_half, d_rho, d_res, d_scratch;
   DBuf d_cpre;   // per-cell prologue records of the fused step (k_cell_pre)
   DBuf d_sl, d_slnb, d_hoff, d_halves, d_eoff, d_ents, d_recds, d_bc, d_sw, d_poff;
-  DBuf d_vtb, d_ovmap, d_moff;
+  DBuf d_vtb, d_ovmap, d_moff, d_regs;
   // ghost-exchange buffers: cell midpoints and bound_enc on the device, and the staging of
   // kah_pack_mirrors / kah_unpack_mirrors (grown on demand)
   std::vector<int64_t> voff_h;
@@ -95,8 +95,8 @@ struct kah_ctx {
   bool ib_done = false;
   std::vector<int64_t> ib_of_pair;   // IB face of each pair, or -1
   DBuf d_ib_solid, d_ib_snoff, d_ib_snb, d_ib_faces, d_ib_img, d_ib_cut, d_ib_cutw, d_ib_ssdf;
-  // overlap map ids of the sources, the work items and their partial sums
-  DBuf d_ib_smap, d_ib_imap, d_ib_swork, d_ib_swoff, d_ib_spart, d_ib_fwork, d_ib_fwoff, d_ib_fpart;
+  // overlap map ids of the sources, the work items, the wall density and its terms
+  DBuf d_ib_smap, d_ib_imap, d_ib_swork, d_ib_fwork, d_ib_term, d_ib_rho;
   std::vector<int32_t> ib_solid_h, ib_snoff_h, ib_snb_h, ib_img_h;   // until upload_ib
   std::vector<IbFaceDesc> ib_faces_h;
   int ib_nsw = 0, ib_nfw = 0;
@@ -115,8 +115,13 @@ struct kah_ctx {
   // whose LDS already limits residency, the 3D grids (8 waves: -14 % on the sphere's flux
   // phase against 4) and the other forms run 8 waves.
   int fr_waves = 0;
-  int flux_waves(size_t lds) const {
+  // In the FP64 form a small launch of irregular cells with larger grids runs 16 waves: too few
+  // workgroups to fill the GPU, its time is one workgroup's (75^2 adapted cylinder 0.459 -> 0.435
+  // ms per step; grids of 640 cells and fewer gain nothing).
+  int flux_waves(size_t lds, int64_t n, bool irregular, size_t cells) const {
     if (fr_waves) return fr_waves;
+    if (!f32 && !uni && irregular && cells < 1024 && n > 640 && P.marching == KAH_MARCH_CAIDVM)
+      return 16;
     if (D != 2 || !f32 || uni || lds == 0) return 8;   // 3D grids (4.5k cells and up): 8 waves
     if (lds <= 8 * 1024) return 2;
     return lds <= 40 * 1024 ? 4 : 8;
@@ -128,7 +133,7 @@ struct kah_ctx {
     int n = 0;
     size_t lds = 0;
     int waves = 8;          // waves per workgroup
-    int reg_class = 0;      // fused step through the gather of regular cells (1, 2) or not
+    int reg_class = 0;      // fused step through the stored gathers (1, 2: regular cells, 3) or not
   };
   int reg_mode = 1;   // KAH_OPT_REGULAR: 0 every cell through the general slope and gather
   // KAH_OPT_BRANCHES: independent launches of one phase (the slope bins of one projection
@@ -181,10 +186,10 @@ struct kah_ctx {
                           &d_sdf, &d_oflux, &d_vflux, &d_psflux, &d_w, &d_prim, &d_qf, &d_half, &d_rho,
                           &d_res, &d_scratch, &d_cpre, &d_sl, &d_slnb, &d_hoff, &d_halves, &d_eoff,
                           &d_ents, &d_recds, &d_bc, &d_sw, &d_poff, &d_vtb, &d_ovmap,
-                          &d_moff, &d_cmid, &d_benc, &d_xcells, &d_xoff, &d_xbuf, &d_xfluid,
+                          &d_moff, &d_regs, &d_cmid, &d_benc, &d_xcells, &d_xoff, &d_xbuf, &d_xfluid,
                           &d_ib_solid, &d_ib_snoff, &d_ib_snb, &d_ib_faces, &d_ib_img,
                           &d_ib_cut, &d_ib_cutw, &d_ib_ssdf, &d_ib_smap, &d_ib_imap, &d_ib_swork,
-                          &d_ib_swoff, &d_ib_spart, &d_ib_fwork, &d_ib_fwoff, &d_ib_fpart};
+                          &d_ib_fwork, &d_ib_term, &d_ib_rho};
     int64_t t = 0;
     for (const DBuf* b : bufs) t += int64_t(b->bytes);
     for (const LevelBin* b : bins) t += int64_t(b->items.bytes);
@@ -560,8 +565,7 @@ int setup_ib(kah_ctx* C, const kah_topology* T) {
   C->ib_of_pair.clear();
   for (DBuf* b : {&C->d_ib_solid, &C->d_ib_snoff, &C->d_ib_snb, &C->d_ib_faces, &C->d_ib_img,
                   &C->d_ib_cut, &C->d_ib_cutw, &C->d_ib_ssdf, &C->d_ib_smap, &C->d_ib_imap,
-                  &C->d_ib_swork, &C->d_ib_swoff, &C->d_ib_spart, &C->d_ib_fwork, &C->d_ib_fwoff,
-                  &C->d_ib_fpart})
+                  &C->d_ib_swork, &C->d_ib_fwork, &C->d_ib_term, &C->d_ib_rho})
     b->release();
   C->ib_nsw = C->ib_nfw = 0;
   C->ib_solid_h.clear();
@@ -682,19 +686,17 @@ int setup_ib(kah_ctx* C, const kah_topology* T) {
 // (map(owner cell, source cell)) and the work items of the kernels.
 template <class Map>
 int upload_ib(kah_ctx* C, const int64_t* voff, Map&& map) {
-  auto chunks = [&](std::vector<int2>& work, std::vector<int32_t>& woff, int64_t cell) {
-    const int64_t n = voff[cell + 1] - voff[cell];
-    const int q = int(woff.size()) - 1;
-    for (int64_t k = 0; k * IB_CHUNK < n; ++k) work.push_back(make_int2(q, int(k)));
-    woff.push_back(int32_t(work.size()));
-  };
   std::vector<int2> work;
-  std::vector<int32_t> woff(1, 0), ids;
+  std::vector<int32_t> ids;
+  auto chunks = [&](int q, int64_t cell) {
+    for (int64_t k = 0; k * IB_CHUNK < voff[cell + 1] - voff[cell]; ++k)
+      work.push_back(make_int2(q, int(k)));
+  };
   if (C->ib_ns > 0) {
     for (int q = 0; q < C->ib_ns; ++q) {
       for (int32_t x = C->ib_snoff_h[q]; x < C->ib_snoff_h[q + 1]; ++x)
         ids.push_back(map(C->ib_solid_h[q], C->ib_snb_h[x]));
-      chunks(work, woff, C->ib_solid_h[q]);
+      chunks(q, C->ib_solid_h[q]);
     }
     C->ib_nsw = int(work.size());
     KAH_TRY(C->upload(C->d_ib_solid, C->ib_solid_h.data(), C->ib_solid_h.size(), "ib solid cells"));
@@ -703,27 +705,154 @@ int upload_ib(kah_ctx* C, const int64_t* voff, Map&& map) {
     KAH_TRY(C->upload(C->d_ib_snb, C->ib_snb_h.data(), C->ib_snb_h.size(), "ib solid neighbours"));
     KAH_TRY(C->upload(C->d_ib_smap, ids.data(), ids.size(), "ib solid overlap maps"));
     KAH_TRY(C->upload(C->d_ib_swork, work.data(), work.size(), "ib solid work items"));
-    KAH_TRY(C->upload(C->d_ib_swoff, woff.data(), woff.size(), "ib solid work offsets"));
-    KAH_TRY(C->alloc(C->d_ib_spart, sizeof(double) * work.size() * size_t(C->NW), "ib solid sums"));
   }
   if (C->ib_nf > 0) {
     work.clear();
-    woff.assign(1, 0);
     ids.assign(C->ib_img_h.size(), -1);
+    int q = 0;
     for (IbFaceDesc& F : C->ib_faces_h) {
       for (int32_t x = F.img_beg; x < F.img_beg + F.img_cnt; ++x)
         ids[size_t(x)] = map(F.donor, C->ib_img_h[size_t(x)]);
       F.smap = map(F.donor, F.solid);
-      chunks(work, woff, F.donor);
+      chunks(q++, F.donor);
     }
     C->ib_nfw = int(work.size());
     KAH_TRY(C->upload(C->d_ib_faces, C->ib_faces_h.data(), C->ib_faces_h.size(), "ib faces"));
     KAH_TRY(C->upload(C->d_ib_img, C->ib_img_h.data(), C->ib_img_h.size(), "ib image cells"));
     KAH_TRY(C->upload(C->d_ib_imap, ids.data(), ids.size(), "ib image overlap maps"));
     KAH_TRY(C->upload(C->d_ib_fwork, work.data(), work.size(), "ib face work items"));
-    KAH_TRY(C->upload(C->d_ib_fwoff, woff.data(), woff.size(), "ib face work offsets"));
-    KAH_TRY(C->alloc(C->d_ib_fpart, sizeof(double) * work.size() * 2, "ib face sums"));
+    KAH_TRY(C->alloc(C->d_ib_term, sizeof(double) * 2 * size_t(C->ib_rows), "ib wall density terms"));
+    KAH_TRY(C->alloc(C->d_ib_rho, sizeof(double) * size_t(C->ib_nf), "ib wall densities"));
   }
+  return 0;
+}
+
+}  // namespace
+
+namespace {
+
+// The slope launches of kah_set_topology.
+struct SlopeTables {
+  const kah_topology* T;
+  const Builder* B;
+  const std::vector<int32_t>* hoff;
+  const std::vector<HalfDesc>* halves;
+  const std::vector<int64_t>*poff, *mbase, *voff, *gof;   // gof null: a shared grid
+};
+
+// The record of a regular cell of the slope kernel: every direction SL_INNER with one neighbour
+// per side and no transverse projection, and its 2*D half fluxes its own limited
+// reconstructions, one out of either side of each direction, from one reconstruction point and
+// cell size, the two faces of a direction differing along it alone. Returns 0 (not regular),
+// 1 (every neighbour on the cell's velocity grid) or 2 (some on other grids).
+template <int D>
+int slope_record(const kah_ctx* C, const SlopeTables& t, int32_t c, RegCell<D>& r) {
+  const int hb = (*t.hoff)[size_t(c)], he = (*t.hoff)[size_t(c) + 1];
+  if (he - hb != 2 * D) return 0;
+  auto grid = [&](int64_t cell) { return t.gof ? (*t.gof)[size_t(cell)] : int64_t(0); };
+  r = RegCell<D>{};
+  r.off = (*t.voff)[size_t(c)];
+  r.n = int32_t((*t.voff)[size_t(c) + 1] - r.off);
+  r.g = grid(c);
+  int cls = 1;
+  for (int d = 0; d < D; ++d) {
+    const SlopeDesc& sd = t.B->sl[size_t(c) * D + d];
+    if (sd.mode != SL_INNER || sd.nb_cnt[0] != 1 || sd.nb_cnt[1] != 1) return 0;
+    for (int sx = 0; sx < 2; ++sx) {
+      const SlopeNb& nb = t.B->slnb[size_t(sd.nb_beg[sx])];
+      if (nb.proj) return 0;
+      if (!C->uni && nb.map != MAP_SAME) cls = 2;
+      RegSide& S = r.s[d][sx];
+      S.off = (*t.voff)[size_t(nb.cell)];
+      S.n = int32_t((*t.voff)[size_t(nb.cell) + 1] - S.off);
+      S.g = grid(nb.cell);
+      S.map = C->uni ? MAP_SAME : nb.map;
+      S.mbase = nb.map >= 0 ? (*t.mbase)[size_t(nb.map)] : -1;
+      S.ds = sd.ds[sx];
+      S.rds = sd.rds[sx];
+      S.rds_f = sd.rds_f[sx];
+      S.row = -1;
+    }
+  }
+  for (int h = hb; h < he; ++h) {
+    const HalfDesc& hd = (*t.halves)[size_t(h)];
+    if (hd.data_cell != c || hd.mode != MI_LIMITED || hd.rot == 0.0) return 0;
+    const int d = hd.dir, sx = (hd.rot > 0.0) == (hd.sel != 0) ? 1 : 0;   // out of the upper face
+    RegSide& S = r.s[d][sx];
+    if (S.row >= 0) return 0;
+    S.row = (*t.poff)[size_t(hd.slot)];
+    S.fm = hd.fmid[d];
+    S.dx_f = hd.dx_f[d];
+    const bool other = r.s[d][1 - sx].row >= 0;
+    for (int e = 0; e < D; ++e) {
+      if (h == hb) {
+        r.x[e] = hd.xrec[e];
+        r.dsr[e] = hd.dsrec[e];
+        r.dsr_f[e] = hd.ds_f[e];
+      } else if (r.x[e] != hd.xrec[e] || r.dsr[e] != hd.dsrec[e]) {
+        return 0;
+      }
+      if (e == d) continue;
+      if (other && r.fmt[d][e] != hd.fmid[e]) return 0;
+      r.fmt[d][e] = hd.fmid[e];
+      r.dxt_f[d][e] = hd.dx_f[e];
+    }
+  }
+  return cls;
+}
+
+template <int D, class ChunksOf>
+int slope_bins(kah_ctx* C, const SlopeTables& t, const std::vector<char>& walled,
+               const std::vector<int>& depth, int Dmax, ChunksOf&& chunks_of) {
+  std::vector<RegCell<D>> regs;
+  for (int L = 0; L <= Dmax; ++L) {
+    std::map<int, std::vector<int32_t>> lists;   // walled cells by half-flux count
+    std::map<int, std::vector<int4>> works;      // 8*kind + waves
+    for (int32_t c : C->fluid) {
+      if (depth[size_t(c)] != L) continue;
+      if (walled[size_t(c)]) {
+        const int nh = (*t.hoff)[size_t(c) + 1] - (*t.hoff)[size_t(c)];
+        lists[nh <= 4 ? 4 : (nh <= 8 ? 8 : (nh <= 16 ? 16 : 24))].push_back(c);
+        continue;
+      }
+      RegCell<D> r;
+      const int kind = C->reg_mode ? slope_record<D>(C, t, c, r) : 0;
+      int32_t idx = c;
+      if (kind) {
+        idx = int32_t(regs.size());
+        regs.push_back(r);
+      }
+      const int64_t n = (*t.voff)[size_t(c) + 1] - (*t.voff)[size_t(c)];
+      const auto ck = chunks_of(c);
+      auto& wl = works[8 * kind + ck.waves];
+      for (int k = 0; k < ck.count; ++k)
+        wl.push_back(make_int4(idx, k, int(k * ck.cells), int(std::min(n, (k + 1) * ck.cells))));
+    }
+    // the few irregular cells first: a launch that waits for room behind the bulk ends after it
+    for (int kind : {0, 2, 1})
+      for (int w : {3, 4}) {
+        const auto it = works.find(8 * kind + w);
+        if (it == works.end()) continue;
+        LevelBin* lb = new LevelBin();
+        C->bins.push_back(lb);
+        lb->level = L;
+        lb->maxh = kind;
+        lb->waves = w;
+        lb->n = int(it->second.size());
+        lb->chunked = true;
+        KAH_TRY(C->upload(lb->items, it->second.data(), it->second.size(), "slope work items"));
+      }
+    for (auto& kv : lists) {
+      LevelBin* lb = new LevelBin();
+      C->bins.push_back(lb);
+      lb->level = L;
+      lb->maxh = kv.first;
+      lb->n = int(kv.second.size());
+      lb->chunked = false;
+      KAH_TRY(C->upload(lb->items, kv.second.data(), kv.second.size(), "level cells"));
+    }
+  }
+  if (!regs.empty()) KAH_TRY(C->upload(C->d_regs, regs.data(), regs.size(), "regular cells"));
   return 0;
 }
 
@@ -1125,12 +1254,16 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
       sd.rds_f[k] = float(sd.rds[k]);
       sd.inv_cnt_f[k] = float(sd.inv_cnt[k]);
     }
-  for (auto& e : B.slnb)
+  for (auto& e : B.slnb) {
     for (int t = 0; t < 3; ++t) e.dm_f[t] = float(e.dm[t]);
+    e.off = voff[size_t(e.cell)];
+    e.n = int32_t(voff[size_t(e.cell) + 1] - e.off);
+    e.g = C->uni ? 0 : gof[size_t(e.cell)];
+    e.mbase = e.map >= 0 ? mbase[size_t(e.map)] : -1;
+  }
   KAH_TRY(C->upload(C->d_sl, B.sl.data(), B.sl.size(), "slope descriptors"));
   KAH_TRY(C->upload(C->d_slnb, B.slnb.data(), B.slnb.size(), "slope neighbours"));
   KAH_TRY(C->upload(C->d_hoff, hoff.data(), hoff.size(), "half offsets"));
-  KAH_TRY(C->upload(C->d_halves, halves.data(), halves.size(), "half descriptors"));
   KAH_TRY(C->upload(C->d_eoff, eoff.data(), eoff.size(), "entry offsets"));
   KAH_TRY(C->upload(C->d_recds, T->cell_ds, size_t(nc * D), "cell ds"));
   KAH_TRY(C->upload(C->d_cmid, T->cell_mid, size_t(nc * D), "cell midpoints"));
@@ -1162,20 +1295,29 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
     if (eoff[c + 1] - eoff[c] > MAX_ENTRIES)
       return C->fail(KAH_EUNSUPPORTED, "cell " + std::to_string(c) + " has more than " +
                                            std::to_string(MAX_ENTRIES) + " face sides");
-  // Chunks of the slope kernel: 3-wave or 4-wave workgroups (64*VPT velocity cells per wave),
-  // whichever pads the cell's grid least (a 568-cell grid fills one 3-wave chunk of 576 at
-  // VPT 3; ties go to 4 waves).
-  auto wpi_of = [&](int64_t c) {
-    const int64_t n = T->vs_offset[c + 1] - T->vs_offset[c];
-    auto padded = [&](int64_t w) {
-      const int64_t cv = w * 64 * C->slope_vpt;
-      return (n + cv - 1) / cv * cv;
-    };
-    return padded(3) < padded(4) ? 3 : 4;
+  // Chunks of the slope kernel, by grid size alone (alike for regular and general cells, whose
+  // sums so run in the same order). FP64 form: 4-wave workgroups, as many chunks as come nearest
+  // to slope_vpt velocity cells per thread, cut evenly at multiples of 64 (784 cells: one chunk
+  // of 13 wave passes; 1.01 against 1.11 ms per step on 22k refined leaves with 28^2 grids, 0.29
+  // against 0.33 on 3D leaves with 12^3). FP32 form: slope_vpt per thread of a 3-wave or 4-wave
+  // workgroup, whichever pads the grid least (a 568-cell grid fills one 3-wave chunk of 576 at 3
+  // cells per thread; ties go to 4 waves): the even cut is no faster on its adapted grids, and
+  // a thread's plain FP64 sum of slope_vpt terms is what a chunk's bits depend on, which over
+  // some hundred steps of float rounding decide the last digits of every f.
+  struct Chunks {
+    int waves, count;
+    int64_t cells;
   };
-  auto nchunks = [&](int64_t c) {
-    const int64_t cv = int64_t(C->slope_vpt) * 64 * wpi_of(c);
-    return int((T->vs_offset[c + 1] - T->vs_offset[c] + cv - 1) / cv);
+  auto chunks_of = [&](int64_t c) {
+    const int64_t n = T->vs_offset[c + 1] - T->vs_offset[c], w = 64 * C->slope_vpt;
+    if (!C->f32) {
+      const int64_t k = std::max<int64_t>(1, (2 * n + 4 * w) / (8 * w));
+      const int64_t cells = ((n + 63) / 64 + k - 1) / k * 64;
+      return Chunks{4, int((n + cells - 1) / cells), cells};
+    }
+    auto count = [&](int64_t v) { return (n + v * w - 1) / (v * w); };
+    const int64_t v = 3 * count(3) < 4 * count(4) ? 3 : 4;
+    return Chunks{int(v), int(count(v)), v * w};
   };
   // Launch order of the slopes: the reference sweeps coarse to fine levels because the
   // transverse projection (update_slope_transverse_level!, src/Flux/Slope.jl:849-945) reads
@@ -1209,91 +1351,86 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
       for (int32_t c : C->fluid) depth[size_t(c)] = T->ps_level[c] - Lmin;
     for (int32_t c : C->fluid) Dmax = std::max(Dmax, depth[size_t(c)]);
   }
-  // Regular cells of the slope kernel: every direction SL_INNER with one neighbour per side,
-  // no transverse projection, and 2*D half fluxes that are the cell's own limited or
-  // plain-slope reconstructions.
-  // Returns 0 (not regular), 1 (both neighbours of every direction on the cell's velocity
-  // grid) or 2 (some on other grids).
-  auto slope_regular = [&](int32_t c) {
-    if (!C->reg_mode || hoff[c + 1] - hoff[c] != 2 * D) return 0;
-    int cls = 1;
-    for (int d = 0; d < D; ++d) {
-      const SlopeDesc& sd = B.sl[size_t(c) * D + d];
-      if (sd.mode != SL_INNER || sd.nb_cnt[0] != 1 || sd.nb_cnt[1] != 1) return 0;
-      for (int sx = 0; sx < 2; ++sx) {
-        const SlopeNb& nbr = B.slnb[size_t(sd.nb_beg[sx])];
-        if (nbr.proj) return 0;
-        if (!C->uni && nbr.map != MAP_SAME) cls = 2;
-      }
-    }
+  // Stored micro fluxes: a half flux that is its owner's own reconstruction through an inner face
+  // or a reconstructing domain face keeps it for the gathers, in the owner's block of the face's
+  // direction when it is alone on its side of the cell, else (a coarse side of hanging faces) in a
+  // block of its own after the cells'.
+  const int64_t prow = C->np + C->ib_rows;   // the cells' rows, then the SolidNeighbors'
+  int64_t of_elems = prow * C->NDF * D;
+  std::vector<int64_t> of_slot(size_t(std::max<int64_t>(C->npairs, 1) * 2), -1);
+  for (int64_t c = 0; c < nc; ++c) {
+    const int64_t n = voff[size_t(c) + 1] - voff[size_t(c)];
+    int on_side[6] = {};
+    auto side_of = [&](const HalfDesc& hd) {
+      return 2 * hd.dir + ((hd.rot > 0.0) == (hd.sel != 0) ? 1 : 0);
+    };
+    auto kept = [&](const HalfDesc& hd) {
+      return hd.data_cell == c && (hd.mode == MI_LIMITED || hd.mode == MI_UNLIMITED);
+    };
+    for (int h = hoff[c]; h < hoff[c + 1]; ++h)
+      if (kept(halves[h])) ++on_side[side_of(halves[h])];
     for (int h = hoff[c]; h < hoff[c + 1]; ++h) {
-      const HalfDesc& hd = halves[size_t(h)];
-      if (hd.data_cell != c || (hd.mode != MI_LIMITED && hd.mode != MI_UNLIMITED)) return 0;
-    }
-    return cls;
-  };
-  for (int L = 0; L <= Dmax; ++L) {
-    // half-count bins: the per-thread accumulators of K1 are MAXH*(dim+2) doubles, so a bin
-    // sized to the common counts (4: 2D interior, 6: 3D interior) keeps registers low
-    // bins 5 and 6: regular cells (the slopes and half fluxes of slope_regular /
-    // half_regular), with every neighbour on the cell's grid, or some on other grids
-    const int caps[7] = {4, 6, 8, 16, 24, -1, -2};
-    std::vector<int32_t> lists[7];
-    std::vector<int2> works[7][2];   // [bin][3-wave items, 4-wave items]
-    for (int32_t c : C->fluid) {
-      if (depth[size_t(c)] != L) continue;
-      int nh = hoff[c + 1] - hoff[c];
-      int b = nh <= 4 ? 0 : (nh <= 6 ? 1 : (nh <= 8 ? 2 : (nh <= 16 ? 3 : 4)));
-      if (walled[c]) {
-        lists[b].push_back(c);
+      HalfDesc& hd = halves[h];
+      hd.ofb = -1;
+      if (!kept(hd)) continue;
+      if (on_side[side_of(hd)] == 1) {
+        hd.ofb = voff[size_t(c)] * C->NDF * D + int64_t(hd.dir) * C->NDF * n;
       } else {
-        const int rc = slope_regular(c);
-        if (rc) b = 4 + rc;
-        auto& wl = works[b][wpi_of(c) == 3 ? 0 : 1];
-        for (int ch = 0; ch < nchunks(c); ++ch) wl.push_back(make_int2(c, ch));
+        hd.ofb = of_elems;
+        of_elems += C->NDF * n;
       }
-    }
-    for (int b = 0; b < 7; ++b) {
-      for (int kind = 0; kind < 3; ++kind) {   // per-cell kernel, 3-wave items, 4-wave items
-        const size_t cnt = kind ? works[b][kind - 1].size() : lists[b].size();
-        if (cnt == 0) continue;
-        LevelBin* lb = new LevelBin();
-        lb->level = L;
-        lb->maxh = caps[b];
-        lb->n = int(cnt);
-        lb->chunked = kind > 0;
-        lb->wpi = kind == 1 ? 3 : 4;
-        C->bins.push_back(lb);
-        if (kind) KAH_TRY(C->upload(lb->items, works[b][kind - 1].data(), cnt, "slope work items"));
-        else KAH_TRY(C->upload(lb->items, lists[b].data(), cnt, "level cells"));
-      }
+      of_slot[size_t(hd.slot)] = hd.ofb;
     }
   }
-  KAH_TRY(C->upload(C->d_fluid, C->fluid.data(), C->fluid.size(), "fluid cells"));
-
+  KAH_TRY(C->upload(C->d_halves, halves.data(), halves.size(), "half descriptors"));
   // partial rows of every half flux
   std::vector<int64_t> poff(size_t(std::max<int64_t>(C->npairs, 1) * 2), 0);
   std::vector<int32_t> pcnt(poff.size(), 0);
   for (int64_t c = 0; c < nc; ++c)
     for (int h = hoff[c]; h < hoff[c + 1]; ++h)
-      pcnt[halves[h].slot] = walled[c] ? 1 : nchunks(c);
+      pcnt[halves[h].slot] = walled[c] ? 1 : chunks_of(c).count;
   for (int64_t p = 0; p < int64_t(C->ib_of_pair.size()); ++p)
-    if (C->ib_of_pair[size_t(p)] >= 0) {   // written by k_ib_wall, a row per work item
-      const int64_t h = T->pair_here[p];
-      pcnt[size_t(2 * p + 1)] =
-          int32_t((T->vs_offset[h + 1] - T->vs_offset[h] + IB_CHUNK - 1) / IB_CHUNK);
-    }
+    if (C->ib_of_pair[size_t(p)] >= 0) pcnt[size_t(2 * p + 1)] = 1;   // written by the IB kernel
   int64_t rows = 0;
   for (size_t s = 0; s < poff.size(); ++s) {
     poff[s] = rows;
     rows += pcnt[s];
   }
   C->part_rows = rows;
+  // the slope launches: regular cells (slope_record) apart from the general ones
+  C->d_regs.release();
+  const SlopeTables tab{T, &B, &hoff, &halves, &poff, &mbase, &voff, C->uni ? nullptr : &gof};
+  KAH_TRY(D == 2 ? slope_bins<2>(C, tab, walled, depth, Dmax, chunks_of)
+                 : slope_bins<3>(C, tab, walled, depth, Dmax, chunks_of));
+  KAH_TRY(C->upload(C->d_fluid, C->fluid.data(), C->fluid.size(), "fluid cells"));
+
   KAH_TRY(C->upload(C->d_poff, poff.data(), poff.size(), "partial offsets"));
-  for (EntryDesc& e : ents)
+  for (EntryDesc& e : ents) {
     for (int sd = 0; sd < 2; ++sd) {
       e.row[sd] = poff[size_t(2 * e.pair + sd)];
       e.rows[sd] = pcnt[size_t(2 * e.pair + sd)];
+    }
+    e.mbase = e.map >= 0 ? mbase[size_t(e.map)] : -1;
+    if (e.oth_cell < 0) continue;
+    e.oth_off = voff[size_t(e.oth_cell)];
+    e.oth_n = int32_t(voff[size_t(e.oth_cell) + 1] - e.oth_off);
+    e.oth_g = C->uni ? 0 : gof[size_t(e.oth_cell)];
+  }
+  for (int64_t c = 0; c < nc; ++c)
+    for (int x = eoff[c]; x < eoff[c + 1]; ++x) {
+      EntryDesc& e = ents[size_t(x)];
+      e.own_ofb = of_slot[size_t(2 * e.pair + e.side)];
+      e.oth_ofb = of_slot[size_t(2 * e.pair + 1 - e.side)];
+      e.kind = -1;   // no stored form
+      const bool same = C->uni || e.map == MAP_SAME;
+      if (e.oth_cell < 0) {
+        if (e.oth_mode == MI_SELF_PLAIN && e.own_mode == MI_PLAIN) e.kind = EK_SELF;
+        else if ((e.oth_mode == MI_MAXWELL || e.oth_mode == MI_WALL) && e.own_ofb >= 0)
+          e.kind = EK_MAXWELL;
+      } else if (e.own_ofb >= 0) {
+        if (e.oth_mode == MI_PLAIN && same) e.kind = EK_PLAIN;
+        else if (e.oth_mode != MI_PLAIN && e.oth_ofb >= 0) e.kind = EK_STORED;
+      }
     }
   KAH_TRY(C->upload(C->d_ents, ents.data(), ents.size(), "entry descriptors"));
 
@@ -1301,7 +1438,6 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
   const int64_t NDF = C->NDF, NW = C->NW;
   const size_t fs = C->fsize();
   // the state buffers hold the SolidNeighbor rows of the IB faces after the cells' rows
-  const int64_t prow = C->np + C->ib_rows;
   KAH_TRY(C->alloc(C->d_df[0], fs * prow * NDF, "df"));
   KAH_TRY(C->alloc(C->d_df[1], fs * prow * NDF, "df"));
   if (C->ib_nf > 0) {
@@ -1309,7 +1445,7 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
     KAH_TRY(C->zero(C->d_df[1]));
   }
   KAH_TRY(C->alloc(C->d_sdf, fs * prow * NDF * D, "sdf"));   // + the SolidNeighbors' slopes
-  KAH_TRY(C->alloc(C->d_oflux, fs * prow * NDF * D, "outgoing micro fluxes"));
+  KAH_TRY(C->alloc(C->d_oflux, fs * size_t(of_elems), "outgoing micro fluxes"));
   KAH_TRY(C->alloc(C->d_psflux, sizeof(double) * nc * NW, "flux"));
   KAH_TRY(C->alloc(C->d_w, sizeof(double) * nc * NW, "w"));
   KAH_TRY(C->alloc(C->d_prim, sizeof(double) * nc * NW, "prim"));
@@ -1336,31 +1472,35 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
   for (auto* b : C->frbins) delete b;
   C->frbins.clear();
   {
-    // the regular gather reads the outgoing micro fluxes the slope kernel stores while it
-    // forms the half fluxes (CAIDVM only), so neither side may be a cell whose slope kernel
-    // forms them in another arithmetic (the per-cell kernel of walled cells; in the FP32 form
-    // CIP_Marching gathers in FP64 while the slope kernel reconstructs in FP32)
+    // the stored gathers read the micro fluxes the slope kernels keep while they form the half
+    // fluxes (CAIDVM only), so neither side may be a cell whose slope kernel forms them in another
+    // arithmetic (in the FP32 form: the per-cell kernel of walled cells, and CIP_Marching, which
+    // gathers in FP64 while the slope kernel reconstructs in FP32)
     const bool caidvm = C->P.flux_kind == KAH_FLUX_CAIDVM;
     const bool same_arith = !(C->f32 && C->P.marching == KAH_MARCH_CIP);
-    // 0: not regular; 1: every neighbour on the cell's velocity grid; 2: some on other grids
-    auto regular = [&](int32_t c) {
-      if (!C->reg_mode || !caidvm || !same_arith || walled[c] || eoff[c + 1] - eoff[c] != 2 * D)
-        return 0;
+    // 0: not regular; 1: every neighbour on the cell's velocity grid; 2: some on other grids;
+    // 3: any other cell that gathers from stored micro fluxes
+    auto fr_class = [&](int32_t c) {
+      if (!caidvm || !same_arith) return 0;
+      const bool wall = C->f32 && walled[c];
+      bool reg = !walled[c] && eoff[c + 1] - eoff[c] == 2 * D, stored = !wall;
       int cls = 1;
       for (int e = eoff[c]; e < eoff[c + 1]; ++e) {
         const EntryDesc& ed = ents[size_t(e)];
-        if (ed.oth_cell < 0 || ed.oth_cell >= nc || T->bound_enc[ed.oth_cell] < 0) return 0;
+        const bool inner = ed.oth_cell >= 0 && ed.oth_cell < nc && T->bound_enc[ed.oth_cell] >= 0;
+        if (ed.kind < 0 || (C->f32 && inner && walled[ed.oth_cell])) stored = false;
         // a neighbour on another level shares a hanging face: its side holds more than one
-        // face, each with its own reconstruction, so one stored outgoing flux cannot serve
-        if (walled[ed.oth_cell] || T->ps_level[ed.oth_cell] != T->ps_level[c]) return 0;
-        if (!C->uni && ed.map != MAP_SAME) cls = 2;
-        if ((ed.own_mode != MI_LIMITED && ed.own_mode != MI_UNLIMITED) ||
+        // face, each with its own reconstruction
+        if (!inner || walled[ed.oth_cell] || T->ps_level[ed.oth_cell] != T->ps_level[c] ||
+            (ed.own_mode != MI_LIMITED && ed.own_mode != MI_UNLIMITED) ||
             (ed.oth_mode != MI_LIMITED && ed.oth_mode != MI_UNLIMITED))
-          return 0;
+          reg = false;
+        if (!C->uni && ed.map != MAP_SAME) cls = 2;
       }
-      return cls;
+      return reg ? cls : (stored ? 3 : 0);
     };
-    // keys: 3*size bin + regular class
+    // keys: whether the cell is a regular one (alike whatever path it takes), size bin, path; the
+    // irregular ones are launched first, as in the slope phase
     std::map<int, std::vector<int32_t>> lists;
     std::map<int, int64_t> bmax;
     for (int32_t c : C->fluid) {
@@ -1368,7 +1508,8 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
       int b = 0;
       if (!C->uni)
         while ((int64_t(640) << b) < n) ++b;
-      const int key = 3 * b + regular(c);
+      const int cls = fr_class(c), bulk = cls == 1 || cls == 2;
+      const int key = (64 * bulk + 63 - b) * 4 + (C->reg_mode ? cls : 0);   // large grids first
       lists[key].push_back(c);
       bmax[key] = std::max(bmax[key], n);
     }
@@ -1378,14 +1519,14 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
       auto* fb = new kah_ctx::FrBin();
       C->frbins.push_back(fb);
       fb->n = int(kv.second.size());
-      fb->reg_class = key % 3;
+      fb->reg_class = key % 4;
       // LDS and workgroup size from the size class, so that a cell gets the same launch shape
       // (and the same order of its sums) whether it is regular or not
-      const int64_t cap = C->uni ? int64_t(C->n0) : std::min<int64_t>(int64_t(640) << (key / 3),
+      const int64_t cap = C->uni ? int64_t(C->n0) : std::min<int64_t>(int64_t(640) << (63 - key / 4 % 64),
                                                                        int64_t(C->max_n));
       fb->lds = sc_elem * size_t(NDF + 1) * size_t(std::max(cap, bmax[key]));
       if (fb->lds > C->lds_limit) fb->lds = 0;
-      fb->waves = C->flux_waves(fb->lds);
+      fb->waves = C->flux_waves(fb->lds, std::max(cap, bmax[key]), key < 256, kv.second.size());
       need_scratch |= fb->lds == 0;
       KAH_TRY(C->upload(fb->cells, kv.second.data(), kv.second.size(), "flux cells"));
     }
@@ -1527,8 +1668,8 @@ int run_slope(kah_ctx* C, const DevArgs& A) {
       const LevelBin* b = C->bins[j];
       hipStream_t st = branch_stream(C, int(j - b0) % nb);
       if (b->chunked)
-        KAH_TRY(C->hip(launch_slope_chunk(A, C->D, C->uni, C->f32, b->items.as<int2>(), b->n,
-                                          b->maxh, C->slope_vpt, b->wpi, st),
+        KAH_TRY(C->hip(launch_slope_chunk(A, C->D, C->uni, C->f32, C->d_regs.p,
+                                          b->items.as<int4>(), b->n, b->maxh, b->waves, st),
                        "slope kernel launch"));
       else
         KAH_TRY(C->hip(launch_slope(A, C->D, C->uni, C->f32, b->items.as<int32_t>(), b->n,
@@ -1548,20 +1689,19 @@ int run_ib(kah_ctx* C, const DevArgs& A) {
   IbArgs B{};
   B.ns = C->ib_ns;
   B.nsw = C->ib_nsw;
+  B.nf = C->ib_nf;
   B.nfw = C->ib_nfw;
   B.solid = C->d_ib_solid.as<int32_t>();
   B.snoff = C->d_ib_snoff.as<int32_t>();
   B.snb = C->d_ib_snb.as<int32_t>();
   B.smap = C->d_ib_smap.as<int32_t>();
   B.swork = C->d_ib_swork.as<int2>();
-  B.swoff = C->d_ib_swoff.as<int32_t>();
-  B.spart = C->d_ib_spart.as<double>();
   B.faces = C->d_ib_faces.as<IbFaceDesc>();
   B.img = C->d_ib_img.as<int32_t>();
   B.imap = C->d_ib_imap.as<int32_t>();
   B.fwork = C->d_ib_fwork.as<int2>();
-  B.fwoff = C->d_ib_fwoff.as<int32_t>();
-  B.fpart = C->d_ib_fpart.as<double>();
+  B.term = C->d_ib_term.as<double2>();
+  B.rho = C->d_ib_rho.as<double>();
   B.cut_idx = C->d_ib_cut.as<int32_t>();
   B.cut_w = C->d_ib_cutw.as<double2>();
   B.cmid = C->d_cmid.as<double>();
@@ -1587,8 +1727,8 @@ int run_flux_relax(kah_ctx* C, const DevArgs& A, int mode) {
   KAH_TRY(fork_branches(C, nb));
   for (size_t j = 0; j < C->frbins.size(); ++j) {
     const kah_ctx::FrBin* b = C->frbins[j];
-    const int m = (mode != MODE_FUSED || b->reg_class == 0) ? mode
-                  : (b->reg_class == 1 ? MODE_FUSED_REG : MODE_FUSED_REGX);
+    constexpr int fused[4] = {MODE_FUSED, MODE_FUSED_REG, MODE_FUSED_REGX, MODE_FUSED_ST};
+    const int m = mode == MODE_FUSED ? fused[b->reg_class] : mode;
     KAH_TRY(C->hip(launch_flux_relax(A, C->D, C->uni, C->f32, b->cells.as<int32_t>(), b->n, m,
                                      march, b->lds, C->fr_waves ? C->fr_waves : b->waves,
                                      branch_stream(C, int(j) % nb)),

@@ -343,7 +343,8 @@ struct Grid {
   // shared tensor-product grid (the 64 positions of a wave form one tile). Any bijection of
   // [0, n) gives the same per-cell results; the order only makes the upwind branches
   // uniform per wave.
-  __device__ int vi(int p) const {
+  __device__ int vi(int p) const { return tile_vi(A, p); }
+  static __device__ int tile_vi(const DevArgs& A, int p) {
     if constexpr (UNI) {
       if (A.vt_mode != 0) {
         const int T = __builtin_amdgcn_readfirstlane(p >> 6);
@@ -448,6 +449,33 @@ __device__ inline void for_overlap_m(const DevArgs& A, const Grid<D, NDF, UNI, F
   }
 }
 
+// The velocity cells of a neighbour grid that overlap velocity cell i (level li, key *kp) of the
+// owner grid: cell j alone, as coarse as i or coarser, when cnt is 0, else the cnt finer cells
+// from j on (for_overlap's pairing). From the overlap map when there is one, else by the search.
+struct Overlap {
+  int j, cnt;
+};
+__device__ inline Overlap overlap_of(const DevArgs& A, int64_t mbase, int64_t g, int n, int dim,
+                                     int i, int li, const uint32_t* kp) {
+  if (mbase >= 0) {
+    const uint32_t code = A.ovmap[mbase + i];
+    return Overlap{int(code >> 8), int(code & 255u)};
+  }
+  const uint32_t* key = A.gkey + g;
+  const uint32_t ki = *kp;
+  int lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (key[mid] <= ki) lo = mid; else hi = mid - 1;
+  }
+  Overlap o{lo, 0};
+  if (int(A.glev[g + lo]) > li) {
+    const uint32_t end = ki + (1u << (dim * (A.lmax - li)));
+    for (int t = lo; t < n && key[t] < end; ++t) ++o.cnt;
+  }
+  return o;
+}
+
 // Overlap map of one (owner grid, neighbour grid) job, one velocity cell of the owner per
 // thread (the search of for_overlap, done once per topology).
 template <int D, int NDF>
@@ -485,6 +513,29 @@ inline hipError_t launch_overlap_map_t(const DevArgs& A, const OvJob* jobs, int 
   return hipGetLastError();
 }
 
+// positivity_preserving_reconstruct (src/Flux/CAIDVM.jl:127-141) times the normal velocity, from
+// the offset dx = face midpoint - u dt - reconstruction point and the cell size ds
+template <int D, int NDF, class T>
+__device__ inline void limited_recon(const T (&f)[NDF], const T (&s)[D][NDF], const T (&dx)[D],
+                                     const T (&ds)[D], T vn, T (&out)[NDF]) {
+#pragma unroll
+  for (int k = 0; k < NDF; ++k) {
+    T s_dx = dx[0] * s[0][k];
+    T s_abs = ds[0] * fabs(s[0][k]);
+#pragma unroll
+    for (int t = 1; t < D; ++t) {
+      s_dx = s_dx + dx[t] * s[t][k];
+      s_abs = s_abs + ds[t] * fabs(s[t][k]);
+    }
+    const T a = f[k] - T(MACH_EPS), b = T(0.5) * s_abs + T(EPS);
+    // b >= EPS > 0, so |a| >= b with b finite means |a/b| >= 1 and the limiter is 1
+    // exactly; the quotient is only formed where it can be below 1 (or NaN)
+    T lim = T(1);
+    if (!(fabs(a) >= b && b < T(HUGE_VAL))) lim = jl_min(T(fabs(a / b)), T(1));
+    out[k] = (f[k] + lim * s_dx) * vn;
+  }
+}
+
 // Micro flux of one velocity cell: value times the normal velocity.
 // LIMITED is positivity_preserving_reconstruct (src/Flux/CAIDVM.jl:127-141); UNLIMITED the
 // plain reconstruction used next to solid cells and at domain walls/inflow (CAIDVM.jl:13-14,
@@ -510,24 +561,19 @@ __device__ inline void micro_recon(int mode, const T (&f)[NDF], const T (&s)[D][
     if constexpr (sizeof(T) == 8) dx[t] = fmid[t] - u[t] * dt - xrec[t];
     else dx[t] = dxf[t] - u[t] * dt;
   }
+  if (mode == MI_LIMITED) {
+    T ds[D];
+#pragma unroll
+    for (int t = 0; t < D; ++t) ds[t] = desc_val<T>(dsrec[t], dsf[t]);
+    limited_recon<D, NDF, T>(f, s, dx, ds, vn, out);
+    return;
+  }
 #pragma unroll
   for (int k = 0; k < NDF; ++k) {
     T s_dx = dx[0] * s[0][k];
 #pragma unroll
     for (int t = 1; t < D; ++t) s_dx = s_dx + dx[t] * s[t][k];
-    if (mode == MI_LIMITED) {
-      T s_abs = desc_val<T>(dsrec[0], dsf[0]) * fabs(s[0][k]);
-#pragma unroll
-      for (int t = 1; t < D; ++t) s_abs = s_abs + desc_val<T>(dsrec[t], dsf[t]) * fabs(s[t][k]);
-      const T a = f[k] - T(MACH_EPS), b = T(0.5) * s_abs + T(EPS);
-      // b >= EPS > 0, so |a| >= b with b finite means |a/b| >= 1 and the limiter is 1
-      // exactly; the quotient is only formed where it can be below 1 (or NaN)
-      T lim = T(1);
-      if (!(fabs(a) >= b && b < T(HUGE_VAL))) lim = jl_min(T(fabs(a / b)), T(1));
-      out[k] = (f[k] + lim * s_dx) * vn;
-    } else {
-      out[k] = (f[k] + s_dx) * vn;
-    }
+    out[k] = (f[k] + s_dx) * vn;
   }
 }
 
@@ -595,25 +641,32 @@ template <int D, int NDF, bool UNI, class FT, class T>
 __device__ inline void side_sum(const DevArgs& A, int c, int n_own, int beg, int cnt,
                                 double dsx, double rdsx, float rdsx_f, int i, int li,
                                 const uint32_t* kp, const T (&f)[NDF], T (&a)[NDF]) {
+  using GR = Grid<D, NDF, UNI, FT>;
 #pragma unroll
   for (int k = 0; k < NDF; ++k) a[k] = T(0);
   for (int e = 0; e < cnt; ++e) {
-    const SlopeNb nb = A.slnb[beg + e];
-    const Grid<D, NDF, UNI, FT> N(A, nb.cell);
-    for_overlap_m<D, NDF, UNI, FT>(A, N, nb.map, i, li, kp,
-                                   [&](int j, double den, double rden) {
+    const SlopeNb& nb = A.slnb[beg + e];
+    const FT* nf = reinterpret_cast<const FT*>(A.df) + nb.off * NDF;
+    const FT* ns = reinterpret_cast<const FT*>(A.sdf_r) + nb.off * (NDF * D);
+    Overlap ov{i, 0};
+    if constexpr (!UNI)
+      if (nb.map != MAP_SAME) ov = overlap_of(A, nb.mbase, nb.g, nb.n, D, i, li, kp);
+    int x = 0;
+    do {
+      const int j = ov.j + x;
+      T rden = T(1);
+      if (ov.cnt) rden = T(ldexp(1.0, -D * (int(A.glev[nb.g + j]) - li)));
 #pragma unroll
       for (int k = 0; k < NDF; ++k) {
-        T pj = T(N.f(j, k));
+        T pj = T(GR::at(nf, k * nb.n + j));
         if (nb.proj) {
 #pragma unroll
-          for (int t = 0; t < D; ++t) pj += desc_val<T>(nb.dm[t], nb.dm_f[t]) * T(N.s(j, k, t));
+          for (int t = 0; t < D; ++t)
+            pj += desc_val<T>(nb.dm[t], nb.dm_f[t]) * T(GR::at(ns, (t * NDF + k) * nb.n + j));
         }
-        T term = f[k] - pj;
-        if (den != 1.0) term = term * T(rden);
-        a[k] += div_ds(term, dsx, rdsx, rdsx_f);
+        a[k] += div_ds(T((f[k] - pj) * rden), dsx, rdsx, rdsx_f);   // rden: a power of two
       }
-    });
+    } while (++x < ov.cnt);
   }
 }
 
@@ -704,11 +757,11 @@ __device__ inline void half_terms(const DevArgs& A, const Grid<D, NDF, UNI, FT>&
   } else if (hd.data_cell == c) {
     micro_recon<D, NDF>(hd.mode, f, s, u, T(A.dt), hd.xrec, hd.dsrec, hd.fmid, hd.dx_f, hd.ds_f,
                         hd.dir, mic);
-    // the cell's own outgoing flux through an inner face (a domain face's second half is the
-    // ghost side: the cell's data flowing in)
-    if (hd.bc < 0) {
+    // the cell's own outgoing flux, for the gathers that read it
+    if (hd.ofb >= 0) {
+      FT* of = reinterpret_cast<FT*>(A.oflux) + hd.ofb;
 #pragma unroll
-      for (int k = 0; k < NDF; ++k) G.set_of(i, k, hd.dir, mic[k]);
+      for (int k = 0; k < NDF; ++k) Grid<D, NDF, UNI, FT>::at(of, k * G.n + i) = FT(mic[k]);
     }
   } else {
     // the there side of a face whose other cell is solid: f of that cell * vn (shared
@@ -717,72 +770,6 @@ __device__ inline void half_terms(const DevArgs& A, const Grid<D, NDF, UNI, FT>&
 #pragma unroll
     for (int k = 0; k < NDF; ++k) mic[k] = T(S.f(i, k)) * ud;
   }
-  moment_terms<D, NDF, T>(wt, u, mic, m);
-}
-
-// slope_dir of a regular cell (SL_INNER with one neighbour per side, no transverse
-// projection): the neighbours' velocity cells that overlap i (cell i itself on the same grid);
-// the same operations in the same order as slope_dir.
-// SAME: both neighbours on the cell's velocity grid (or a shared grid): velocity cell i.
-template <int D, int NDF, bool UNI, class FT, class T, bool SAME>
-__device__ inline void slope_regular(const DevArgs& A, const Grid<D, NDF, UNI, FT>& G, int c,
-                                     int d, int i, int li, const uint32_t* kp,
-                                     const T (&f)[NDF], T (&s)[NDF]) {
-  const SlopeDesc sd = A.sl[c * D + d];
-  T a[2][NDF];
-#pragma unroll
-  for (int side = 0; side < 2; ++side) {
-    const SlopeNb nb = A.slnb[sd.nb_beg[side]];
-#pragma unroll
-    for (int k = 0; k < NDF; ++k) a[side][k] = T(0);
-    if constexpr (SAME) {
-      const int64_t no = UNI ? int64_t(nb.cell) * G.n : A.voff[nb.cell];
-      const FT* nf = reinterpret_cast<const FT*>(A.df) + no * NDF;
-#pragma unroll
-      for (int k = 0; k < NDF; ++k) {
-        const T term = f[k] - T(double(Grid<D, NDF, UNI, FT>::at(nf, k * G.n + i)));
-        a[side][k] += div_ds(term, sd.ds[side], sd.rds[side], sd.rds_f[side]);
-      }
-    } else {
-      const Grid<D, NDF, UNI, FT> N(A, nb.cell);
-      for_overlap_m<D, NDF, UNI, FT>(A, N, nb.map, i, li, kp, [&](int j, double den, double rden) {
-#pragma unroll
-        for (int k = 0; k < NDF; ++k) {
-          T term = f[k] - T(N.f(j, k));
-          if (den != 1.0) term = term * T(rden);
-          a[side][k] += div_ds(term, sd.ds[side], sd.rds[side], sd.rds_f[side]);
-        }
-      });
-    }
-  }
-  const T ic0 = desc_val<T>(sd.inv_cnt[0], sd.inv_cnt_f[0]);
-  const T ic1 = desc_val<T>(sd.inv_cnt[1], sd.inv_cnt_f[1]);
-#pragma unroll
-  for (int k = 0; k < NDF; ++k) {
-    s[k] = minmod_sel(a[0][k] * ic0, a[1][k] * ic1);
-    s[k] = T(G.stored(s[k]));
-    G.set_s(i, k, d, s[k]);
-  }
-}
-
-// half_terms of a regular cell: every half flux it owns is its own limited or plain-slope
-// upwind reconstruction.
-template <int D, int NDF, bool UNI, class FT, class T>
-__device__ inline void half_regular(const DevArgs& A, const Grid<D, NDF, UNI, FT>& G,
-                                    const HalfDesc& hd, int i, const T (&u)[D],
-                                    const T (&f)[NDF], const T (&s)[D][NDF], T wt,
-                                    double (&m)[D + 2]) {
-#pragma unroll
-  for (int q = 0; q < D + 2; ++q) m[q] = 0.0;
-  const T ud = pick<D>(u, hd.dir);
-  const T ru = desc_val<T>(hd.rot, hd.rot_f) * ud;
-  const bool in = hd.sel ? (ru > T(0)) : (ru <= T(0));
-  if (!in) return;
-  T mic[NDF];
-  micro_recon<D, NDF>(hd.mode, f, s, u, T(A.dt), hd.xrec, hd.dsrec, hd.fmid, hd.dx_f, hd.ds_f,
-                      hd.dir, mic);
-#pragma unroll
-  for (int k = 0; k < NDF; ++k) G.set_of(i, k, hd.dir, mic[k]);
   moment_terms<D, NDF, T>(wt, u, mic, m);
 }
 
@@ -886,140 +873,216 @@ __global__ __launch_bounds__(NWV * 64) void k_slope(DevArgs A0, const int32_t* _
   }
 }
 
-// VPT velocity cells per thread, one (cell, chunk) work item per workgroup: the same
-// per-cell work as k_slope without the loop over the grid, for cells without wall faces.
-// Each workgroup writes its partial sums of the cell's half fluxes to row
-// part_off[slot]+chunk; k_flux_relax adds the rows in chunk order.
-template <int D, int NDF, bool UNI, class FT, int MAXH, int VPT, int REG = 0, int WPI = 4>
-__global__ __launch_bounds__(WPI * 64) void k_slope_chunk(DevArgs A0,
-                                                          const int2* __restrict__ work,
+// One (cell, chunk) work item per workgroup of NWV waves: the same per-cell work as k_slope, for
+// cells without wall faces; a thread takes the velocity cells p0 + tid, + 64*NWV, ... of the
+// chunk. Each workgroup writes its partial sums of the cell's half fluxes to row
+// part_off[slot]+chunk; k_cell_pre adds the rows in chunk order.
+// A general cell owns up to 24 half fluxes (hanging faces): the slopes come first, then the half
+// fluxes HB at a time from the chunk's f and the slopes just written, so that only HB*(D+2)
+// FP64 accumulators are live: 105 -> 78 us for the 3D cells of 6 to 8 half fluxes, whose 40
+// accumulators left two waves per SIMD; in 2D the same as one pass with all of them.
+template <int D, int NDF, bool UNI, class FT, int NWV>
+__global__ __launch_bounds__(NWV * 64) void k_slope_chunk(DevArgs A0, const int4* __restrict__ work,
                                                           int nwork, KAH_RO_PARAMS) {
-  // WPI waves (3 or 4) per workgroup, 64*WPI*VPT velocity cells per chunk; the host picks
-  // WPI per cell so that the chunks pad its grid least (a 568-cell grid fills one 3-wave
-  // chunk of 576 where a 4-wave chunk would hold 768).
-  static_assert(WPI == 3 || WPI == 4, "three or four waves per work item");
-  constexpr int NW = D + 2;
-  constexpr int CNT = MAXH * NW;
-  constexpr int CH = 64 * WPI;   // threads per item
+  constexpr int NW = D + 2, BS = NWV * 64, HB = 4, CNT = HB * NW;
+  using CT = typename Arith<FT>::type;
   DevArgs A = A0;
   KAH_RO_BIND(A);
-  const int2 wk = work[xcd_remap(blockIdx.x, nwork)];
+  const int4 wk = work[xcd_remap(blockIdx.x, nwork)];
   const int c = wk.x, ch = wk.y;
-  const int tid = threadIdx.x;
   const Grid<D, NDF, UNI, FT> G(A, c);
   const int hb = A.half_off[c];
   const int nh = A.half_off[c + 1] - hb;
-  if constexpr (MAXH > 8) {
-    // Cells with many half fluxes (hanging faces): the velocity cells' slopes stay in
-    // registers and the half fluxes are summed one at a time (NW values per thread instead
-    // of MAXH*NW), each with a per-wave reduce-scatter; one barrier, then the waves in order.
-    using CT = typename Arith<FT>::type;
-    constexpr int P = pow2_at_least(NW);
-    constexpr int SH = (P == 4) ? 4 : 3;   // lanes per value after the reduce-scatter
-    __shared__ double redh[2 * WPI * MAXH * P];
-    CT u[VPT][D], f[VPT][NDF], s[VPT][D][NDF], wt[VPT];
-    int iv[VPT];
+  __shared__ double red[2 * NWV * red_stride(CNT)];
+  for (int p = wk.z + int(threadIdx.x); p < wk.w; p += BS) {
+    const int i = G.vi(p);
+    CT f[NDF], s[NDF];
 #pragma unroll
-    for (int r = 0; r < VPT; ++r) {
-      const int p = (ch * VPT + r) * CH + tid;
-      iv[r] = -1;
-      if (p < G.n) {
-        const int i = G.vi(p);
-        iv[r] = i;
+    for (int k = 0; k < NDF; ++k) f[k] = CT(G.f(i, k));
+    const int li = G.lev(i);
+    const uint32_t* kp = G.keyp(i);
 #pragma unroll
-        for (int d = 0; d < D; ++d) u[r][d] = CT(G.u(i, d));
-#pragma unroll
-        for (int k = 0; k < NDF; ++k) f[r][k] = CT(G.f(i, k));
-        const int li = G.lev(i);
-        const uint32_t* kp = G.keyp(i);
-#pragma unroll
-        for (int d = 0; d < D; ++d)
-          slope_dir<D, NDF, UNI, FT, CT>(A, G, c, d, i, li, kp, f[r], s[r][d]);
-        wt[r] = CT(G.wt(i));
-      }
-    }
-    const int lane = tid & 63, wv = tid >> 6;
-    for (int h = 0; h < nh; ++h) {
-      const HalfDesc hd = A.halves[hb + h];
-      double v[P], e[P];
-#pragma unroll
-      for (int q = 0; q < P; ++q) v[q] = e[q] = 0.0;
-#pragma unroll
-      for (int r = 0; r < VPT; ++r) {
-        if (iv[r] >= 0) {
-          double m[NW];
-          half_terms<D, NDF, UNI, FT, CT>(A, G, c, hd, iv[r], u[r], f[r], s[r], wt[r], m);
-#pragma unroll
-          for (int q = 0; q < NW; ++q) v[q] = (r == 0) ? m[q] : v[q] + m[q];
-        }
-      }
-      wave_scatter2<P>(v, e);
-      if ((lane & ((1 << SH) - 1)) == 0) {
-        const int q = lane >> SH;
-        redh[((wv * MAXH + h) * P + q) * 2] = v[0];
-        redh[((wv * MAXH + h) * P + q) * 2 + 1] = e[0];
-      }
-    }
-    __syncthreads();
-    for (int t = tid; t < nh * NW; t += CH) {
-      const int h = t / NW, q = t % NW;
-      double S = redh[(h * P + q) * 2], E = redh[(h * P + q) * 2 + 1];
-      for (int w = 1; w < WPI; ++w) {
-        double err;
-        S = two_sum(S, redh[((w * MAXH + h) * P + q) * 2], err);
-        E = (E + redh[((w * MAXH + h) * P + q) * 2 + 1]) + err;
-      }
-      A.half_fw[(A.part_off[A.halves[hb + h].slot] + ch) * NW + q] = S + E;
-    }
-    return;
+    for (int d = 0; d < D; ++d) slope_dir<D, NDF, UNI, FT, CT>(A, G, c, d, i, li, kp, f, s);
   }
-  __shared__ double red[2 * WPI * red_stride(CNT)];
-
-  // Per-thread partials (VPT <= 4 terms each) in FP64; the sum over the item's threads is
-  // compensated (two_sum butterflies, then the waves in order).
-  double acc[CNT];
+  for (int h0 = 0; h0 < nh; h0 += HB) {
+    const int m0 = nh - h0 < HB ? nh - h0 : HB;
+    // per-thread partials in FP64; the sum over the workgroup is compensated
+    double acc[CNT];
 #pragma unroll
-  for (int q = 0; q < CNT; ++q) acc[q] = 0.0;
-  // velocity cells (ch*VPT + r)*CH + tid, r < VPT
-#pragma unroll
-  for (int r = 0; r < VPT; ++r) {
-    const int p = (ch * VPT + r) * CH + tid;
-    if (p < G.n) {
-      using CT = typename Arith<FT>::type;
+    for (int q = 0; q < CNT; ++q) acc[q] = 0.0;
+    for (int p = wk.z + int(threadIdx.x); p < wk.w; p += BS) {
       const int i = G.vi(p);
       CT u[D], f[NDF], s[D][NDF];
 #pragma unroll
       for (int d = 0; d < D; ++d) u[d] = CT(G.u(i, d));
 #pragma unroll
-      for (int k = 0; k < NDF; ++k) f[k] = CT(G.f(i, k));
-      // REG 1: regular cell, neighbours on its grid; 2: regular cell, neighbours on any grid
-      const int li = REG == 1 ? 0 : G.lev(i);
-      const uint32_t* kp = REG == 1 ? nullptr : G.keyp(i);
-      if constexpr (REG != 0) {
+      for (int k = 0; k < NDF; ++k) {
+        f[k] = CT(G.f(i, k));
 #pragma unroll
-        for (int d = 0; d < D; ++d)
-          slope_regular<D, NDF, UNI, FT, CT, REG == 1>(A, G, c, d, i, li, kp, f, s[d]);
-      } else {
-#pragma unroll
-        for (int d = 0; d < D; ++d) slope_dir<D, NDF, UNI, FT, CT>(A, G, c, d, i, li, kp, f, s[d]);
+        for (int d = 0; d < D; ++d) s[d][k] = CT(G.s(i, k, d));
       }
       const CT wt = CT(G.wt(i));
 #pragma unroll
-      for (int h = 0; h < MAXH; ++h) {
-        if (h < nh) {
+      for (int h = 0; h < HB; ++h) {
+        if (h < m0) {
           double m[NW];
-          if constexpr (REG) half_regular<D, NDF, UNI, FT, CT>(A, G, A.halves[hb + h], i, u, f, s, wt, m);
-          else half_terms<D, NDF, UNI, FT, CT>(A, G, c, A.halves[hb + h], i, u, f, s, wt, m);
+          half_terms<D, NDF, UNI, FT, CT>(A, G, c, A.halves[hb + h0 + h], i, u, f, s, wt, m);
 #pragma unroll
-          for (int q = 0; q < NW; ++q) acc[h * NW + q] = (r == 0) ? m[q] : acc[h * NW + q] + m[q];
+          for (int q = 0; q < NW; ++q) acc[h * NW + q] += m[q];
         }
       }
     }
+    const double tot = block_totals<CNT, NWV>(acc, m0 * NW, red);
+    if (int(threadIdx.x) < m0 * NW) {
+      const int h = threadIdx.x / NW, q = threadIdx.x % NW;
+      A.half_fw[(A.part_off[A.halves[hb + h0 + h].slot] + ch) * NW + q] = tot;
+    }
   }
-  const double tot = block_totals<CNT, WPI>(acc, nh * NW, red);
-  if (tid < nh * NW) {
-    const int h = tid / NW, q = tid % NW;
-    A.half_fw[(A.part_off[A.halves[hb + h].slot] + ch) * NW + q] = tot;
+}
+
+// The neighbour's values over velocity cell i as the slope reads them: a += (f - f_j)*share/ds
+// over its velocity cells j that overlap i, from the first value (already loaded).
+template <int D, int NDF, class FT, class T>
+__device__ inline void reg_side(const DevArgs& A, const RegSide& S, const FT* nf, const Overlap& ov,
+                                int li, const T (&f)[NDF], const T (&v)[NDF], T (&a)[NDF]) {
+  if (ov.cnt == 0) {
+#pragma unroll
+    for (int k = 0; k < NDF; ++k) a[k] = T(0) + div_ds(T(f[k] - v[k]), S.ds, S.rds, S.rds_f);
+    return;
+  }
+#pragma unroll
+  for (int k = 0; k < NDF; ++k) a[k] = T(0);
+  for (int x = 0; x < ov.cnt; ++x) {
+    const int j = ov.j + x;
+    const T rden = T(ldexp(1.0, -D * (int(A.glev[S.g + j]) - li)));
+#pragma unroll
+    for (int k = 0; k < NDF; ++k) {
+      const T w = x == 0 ? v[k] : T(nf[k * S.n + j]);
+      a[k] += div_ds(T((f[k] - w) * rden), S.ds, S.rds, S.rds_f);
+    }
+  }
+}
+
+// K1 of a regular cell (every direction with one same-level neighbour per side, no transverse
+// projection, its 2*D half fluxes its own limited reconstructions): the same operations per
+// velocity cell as k_slope_chunk's, with what bounds it taken out. Everything the cell needs is
+// in one record (RegCell), so a workgroup waits for its work item, its record and then its
+// values instead of a chain of descriptor lookups per direction; all values of a velocity cell
+// (2*D neighbours, f, velocities, weight) are loaded before the first is used; and a velocity
+// cell leaves through one face per direction, so one reconstruction with the face picked per
+// lane serves both sides' half fluxes: 103 -> 72 us on 64^2 leaves with 28^2 velocity cells and
+// 547 -> 388 us on 22k leaves (FP64, 3.2 TB/s of f, slopes and micro fluxes; 5 waves per SIMD,
+// the wait for memory bounds it), 107 -> 44 us on 3D leaves with 12^3.
+// SAME: every neighbour on the cell's velocity grid (or a shared grid).
+template <int D, int NDF, bool UNI, class FT, bool SAME, int NWV>
+__global__ __launch_bounds__(NWV * 64) void k_slope_chunk_reg(DevArgs A0,
+                                                              const RegCell<D>* __restrict__ recs,
+                                                              const int4* __restrict__ work,
+                                                              int nwork, KAH_RO_PARAMS) {
+  constexpr int NW = D + 2, BS = NWV * 64, CNT = 2 * D * NW;
+  using CT = typename Arith<FT>::type;
+  DevArgs A = A0;
+  KAH_RO_BIND(A);
+  const int4 wk = work[xcd_remap(blockIdx.x, nwork)];
+  const RegCell<D>& R = recs[wk.x];
+  const int ch = wk.y, n = R.n;
+  const FT* df = reinterpret_cast<const FT*>(A.df);
+  const FT* fb = df + R.off * NDF;
+  FT* sw = reinterpret_cast<FT*>(A.sdf) + R.off * (NDF * D);
+  FT* of = reinterpret_cast<FT*>(A.oflux) + R.off * (NDF * D);
+  const double* gu = A.gu + R.g * D;
+  const double* gw = A.gw + R.g;
+  const CT dt = CT(A.dt);
+  using GR = Grid<D, NDF, UNI, FT>;
+  __shared__ double red[2 * NWV * red_stride(CNT)];
+  double acc[CNT];
+#pragma unroll
+  for (int q = 0; q < CNT; ++q) acc[q] = 0.0;
+  for (int p = wk.z + int(threadIdx.x); p < wk.w; p += BS) {
+    const int i = GR::tile_vi(A, p);
+    int li = 0;
+    Overlap ov[D][2];
+    if constexpr (!SAME) {
+      li = int(A.glev[R.g + i]);
+#pragma unroll
+      for (int d = 0; d < D; ++d)
+#pragma unroll
+        for (int sd = 0; sd < 2; ++sd) {
+          const RegSide& S = R.s[d][sd];
+          ov[d][sd] = Overlap{i, 0};
+          if (S.map != MAP_SAME)
+            ov[d][sd] = overlap_of(A, S.mbase, S.g, S.n, D, i, li, A.gkey + R.g + i);
+        }
+    }
+    CT u[D], f[NDF], v[D][2][NDF];
+#pragma unroll
+    for (int k = 0; k < NDF; ++k) f[k] = CT(GR::at(fb, k * n + i));
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+#pragma unroll
+      for (int sd = 0; sd < 2; ++sd) {
+        const RegSide& S = R.s[d][sd];
+        const FT* nf = df + S.off * NDF;
+#pragma unroll
+        for (int k = 0; k < NDF; ++k)
+          v[d][sd][k] = CT(SAME ? GR::at(nf, k * n + i) : GR::at(nf, k * S.n + ov[d][sd].j));
+      }
+#pragma unroll
+    for (int d = 0; d < D; ++d) u[d] = CT(GR::at(gu, d * n + i));
+    const CT wt = CT(GR::at(gw, i));
+    CT s[D][NDF];
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      CT a[2][NDF];
+#pragma unroll
+      for (int sd = 0; sd < 2; ++sd) {
+        const RegSide& S = R.s[d][sd];
+        if constexpr (SAME) {
+#pragma unroll
+          for (int k = 0; k < NDF; ++k)
+            a[sd][k] = CT(0) + div_ds(CT(f[k] - v[d][sd][k]), S.ds, S.rds, S.rds_f);
+        } else {
+          reg_side<D, NDF, FT, CT>(A, S, df + S.off * NDF, ov[d][sd], li, f, v[d][sd], a[sd]);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < NDF; ++k) {
+        s[d][k] = CT(GR::stored(minmod_sel(a[0][k], a[1][k])));
+        GR::at(sw, (d * NDF + k) * n + i) = FT(s[d][k]);
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const bool pos = u[d] > CT(0);   // leaves through the upper face of direction d
+      CT dx[D], ds[D], mic[NDF];
+#pragma unroll
+      for (int t = 0; t < D; ++t) {
+        ds[t] = desc_val<CT>(R.dsr[t], R.dsr_f[t]);
+        if constexpr (sizeof(CT) == 8) {
+          const double fm = t == d ? (pos ? R.s[d][1].fm : R.s[d][0].fm) : R.fmt[d][t];
+          dx[t] = fm - u[t] * dt - R.x[t];
+        } else {
+          const float o = t == d ? (pos ? R.s[d][1].dx_f : R.s[d][0].dx_f) : R.dxt_f[d][t];
+          dx[t] = o - u[t] * dt;
+        }
+      }
+      limited_recon<D, NDF, CT>(f, s, dx, ds, u[d], mic);
+#pragma unroll
+      for (int k = 0; k < NDF; ++k) GR::at(of, (d * NDF + k) * n + i) = FT(mic[k]);
+      // selects, not a branch: the two sides' sums would be folded into one indexed array
+      CT m[NW];
+      moment_terms<D, NDF, CT>(wt, u, mic, m);
+#pragma unroll
+      for (int q = 0; q < NW; ++q) {
+        acc[2 * d * NW + q] += double(pos ? CT(0) : m[q]);
+        acc[(2 * d + 1) * NW + q] += double(pos ? m[q] : CT(0));
+      }
+    }
+  }
+  const double tot = block_totals<CNT, NWV>(acc, CNT, red);
+  if (int(threadIdx.x) < CNT) {
+    const int h = threadIdx.x / NW, q = threadIdx.x % NW;
+    A.half_fw[(R.s[h >> 1][h & 1].row + ch) * NW + q] = tot;
   }
 }
 
@@ -1107,46 +1170,158 @@ __device__ inline void gather_flux(const DevArgs& A, int c, int n_own, int eb, i
 // grids through the overlap map, with the 2^(-DIM*dl) factors): the same terms in the same
 // order as gather_flux, so the same result, without slopes, neighbour velocities or
 // reconstruction.
+// The upwind side differs from lane to lane, so it picks the address, not the code path: all
+// map words, then all 2*DIM*NDF values are loaded at once, and the sums follow. With a branch
+// per side every face waited for its own loads: cells with neighbours on other grids 219 -> 169 us
+// on the 160^2 adapted cylinder (FP32 form); on one grid the compiler had done so already.
 // SAME: every neighbour on the cell's velocity grid (or a shared grid): velocity cell i.
 template <int D, int NDF, bool UNI, class FT, class T, bool SAME>
 __device__ inline void gather_regular(const DevArgs& A, const Grid<D, NDF, UNI, FT>& G, int eb,
                                       int i, int li, const uint32_t* kp, const T (&u)[D],
                                       T (&fl)[NDF]) {
   const FT* of = reinterpret_cast<const FT*>(A.oflux);
+  bool own[2 * D];
+  Overlap ov[2 * D];
+  T v[2 * D][NDF];
 #pragma unroll
   for (int e = 0; e < 2 * D; ++e) {
     const EntryDesc& ed = A.ents[eb + e];
-    const T ud = pick<D>(u, ed.dir);
-    const T ru = desc_val<T>(ed.rot, ed.rot_f) * ud;
-    const bool own = ed.side ? (ru > T(0)) : (ru <= T(0));
-    const T area = desc_val<T>(ed.area, ed.area_f);
-    if (own) {
-      const FT* b = of + G.off * (NDF * D);
-#pragma unroll
-      for (int k = 0; k < NDF; ++k) {
-        const T t = area * T(Grid<D, NDF, UNI, FT>::at(b, (ed.dir * NDF + k) * G.n + i));
-        fl[k] += ed.side ? -t : t;
+    const T ru = desc_val<T>(ed.rot, ed.rot_f) * pick<D>(u, ed.dir);
+    own[e] = ed.side ? (ru > T(0)) : (ru <= T(0));
+    ov[e] = Overlap{i, 0};
+    if constexpr (!SAME) {
+      if (ed.map != MAP_SAME) {
+        ov[e] = overlap_of(A, ed.mbase, ed.oth_g, ed.oth_n, D, i, li, kp);
+        if (own[e]) ov[e] = Overlap{i, 0};
       }
-    } else if constexpr (SAME) {
-      const int64_t no = UNI ? int64_t(ed.oth_cell) * G.n : A.voff[ed.oth_cell];
-      const FT* b = of + no * (NDF * D);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 2 * D; ++e) {
+    const EntryDesc& ed = A.ents[eb + e];
+    const FT* b = of + (own[e] ? G.off : ed.oth_off) * (NDF * D);
+    const int n = SAME || own[e] ? G.n : ed.oth_n;
+#pragma unroll
+    for (int k = 0; k < NDF; ++k)
+      v[e][k] = T(Grid<D, NDF, UNI, FT>::at(b, (ed.dir * NDF + k) * n + ov[e].j));
+  }
+#pragma unroll
+  for (int e = 0; e < 2 * D; ++e) {
+    const EntryDesc& ed = A.ents[eb + e];
+    const T area = desc_val<T>(ed.area, ed.area_f);
+    if (SAME || ov[e].cnt == 0) {
 #pragma unroll
       for (int k = 0; k < NDF; ++k) {
-        const T t = area * T(Grid<D, NDF, UNI, FT>::at(b, (ed.dir * NDF + k) * G.n + i));
+        const T t = area * v[e][k];
         fl[k] += ed.side ? -t : t;
       }
     } else {
-      const Grid<D, NDF, UNI, FT> N(A, ed.oth_cell);
-      const FT* b = of + N.off * (NDF * D);
-      for_overlap_m<D, NDF, UNI, FT>(A, N, ed.map, i, li, kp,
-                                     [&](int j, double den, double rden) {
+      const FT* b = of + ed.oth_off * (NDF * D);
+      for (int x = 0; x < ov[e].cnt; ++x) {
+        const int j = ov[e].j + x;
+        const T rden = T(ldexp(1.0, -D * (int(A.glev[ed.oth_g + j]) - li)));
 #pragma unroll
         for (int k = 0; k < NDF; ++k) {
-          T t = area * T(Grid<D, NDF, UNI, FT>::at(b, (ed.dir * NDF + k) * N.n + j));
-          if (den != 1.0) t = t * T(rden);   // exact: den is a power of two
+          const T w = x == 0 ? v[e][k]
+                             : T(Grid<D, NDF, UNI, FT>::at(b, (ed.dir * NDF + k) * ed.oth_n + j));
+          const T t = area * w * rden;   // exact scaling: a power of two
           fl[k] += ed.side ? -t : t;
         }
-      });
+      }
+    }
+  }
+}
+
+// gather_flux from stored micro fluxes for any cell of the CAIDVM flux whose sides the slope
+// kernels stored in this arithmetic: hanging faces (each sub-face of a coarse side has a block
+// of its own), domain faces and immersed-boundary faces beside plain ones, up to MAX_ENTRIES
+// face sides. The same terms in the same order as gather_flux, so the same result; four faces'
+// values are loaded at once, without slopes, neighbour velocities or reconstruction (gather_flux
+// waits for each face's map word, then its f and slopes): 107 -> 30 us for the irregular cells of
+// a 20^2 Riemann mesh refined in both spaces, 115 -> 87 us for those of 22k refined leaves.
+template <int D, int NDF, bool UNI, class FT, class T>
+__device__ inline void gather_stored(const DevArgs& A, const Grid<D, NDF, UNI, FT>& G, int eb,
+                                     int ne, int i, int li, const uint32_t* kp, const T (&u)[D],
+                                     const T (&f)[NDF], T (&fl)[NDF]) {
+  using GR = Grid<D, NDF, UNI, FT>;
+  constexpr int B = 4;
+  const FT* of = reinterpret_cast<const FT*>(A.oflux);
+  const FT* df = reinterpret_cast<const FT*>(A.df);
+  for (int e0 = 0; e0 < ne; e0 += B) {
+    bool own[B];
+    Overlap ov[B];
+    T v[B][NDF];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      own[b] = true;
+      ov[b] = Overlap{i, 0};
+      if (e0 + b < ne) {
+        const EntryDesc& ed = A.ents[eb + e0 + b];
+        const T ru = desc_val<T>(ed.rot, ed.rot_f) * pick<D>(u, ed.dir);
+        own[b] = ed.side ? (ru > T(0)) : (ru <= T(0));
+        if constexpr (!UNI) {
+          if (ed.kind == EK_STORED && ed.map != MAP_SAME) {
+            ov[b] = overlap_of(A, ed.mbase, ed.oth_g, ed.oth_n, D, i, li, kp);
+            if (own[b]) ov[b] = Overlap{i, 0};
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+#pragma unroll
+      for (int k = 0; k < NDF; ++k) v[b][k] = T(0);
+      if (e0 + b < ne) {
+        const EntryDesc& ed = A.ents[eb + e0 + b];
+        if (ed.kind != EK_SELF) {
+          // the incoming set of a boundary Maxwellian reads nothing: any address of its own
+          const bool self = own[b] || ed.kind == EK_MAXWELL;
+          const FT* q = self ? of + ed.own_ofb
+                             : (ed.kind == EK_PLAIN ? df + ed.oth_off * NDF : of + ed.oth_ofb);
+          const int n = self ? G.n : ed.oth_n;
+#pragma unroll
+          for (int k = 0; k < NDF; ++k) v[b][k] = T(GR::at(q, k * n + ov[b].j));
+        }
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      if (e0 + b < ne) {
+        const EntryDesc& ed = A.ents[eb + e0 + b];
+        const T area = desc_val<T>(ed.area, ed.area_f);
+        const T ud = pick<D>(u, ed.dir);
+        if (ed.kind == EK_SELF) {
+#pragma unroll
+          for (int k = 0; k < NDF; ++k) fl[k] += area * (f[k] * ud);
+        } else if (own[b] || (ed.kind == EK_STORED && ov[b].cnt == 0)) {
+#pragma unroll
+          for (int k = 0; k < NDF; ++k) {
+            const T t = area * v[b][k];
+            fl[k] += ed.side ? -t : t;
+          }
+        } else if (ed.kind == EK_PLAIN) {
+#pragma unroll
+          for (int k = 0; k < NDF; ++k) fl[k] += area * (v[b][k] * ud);
+        } else if (ed.kind == EK_MAXWELL) {
+          T mic[NDF];
+          micro_maxwell<D, NDF>(&A.bc_prim[ed.bc * (D + 2)], A.rho_w_r[ed.pair],
+                                ed.oth_mode == MI_WALL, u, A.K, ed.dir, mic);
+#pragma unroll
+          for (int k = 0; k < NDF; ++k) fl[k] += area * mic[k];
+        } else {
+          const FT* q = of + ed.oth_ofb;
+          for (int x = 0; x < ov[b].cnt; ++x) {
+            const int j = ov[b].j + x;
+            const T rden = T(ldexp(1.0, -D * (int(A.glev[ed.oth_g + j]) - li)));
+#pragma unroll
+            for (int k = 0; k < NDF; ++k) {
+              const T w = x == 0 ? v[b][k] : T(GR::at(q, k * ed.oth_n + j));
+              const T t = area * w * rden;   // exact scaling: a power of two
+              fl[k] += ed.side ? -t : t;
+            }
+          }
+        }
+      }
     }
   }
 }
@@ -1655,7 +1830,8 @@ __global__ __launch_bounds__(NWV * 64) void k_flux_relax(DevArgs A0,
 
   // half flux = sum of its partial rows in chunk order (micro_to_macro's 1/2 on the energy
   // row applied after the sum), one thread per (entry, side, component)
-  constexpr bool FUSED = (MODE == MODE_FUSED || MODE == MODE_FUSED_REG || MODE == MODE_FUSED_REGX);
+  constexpr bool FUSED = (MODE == MODE_FUSED || MODE == MODE_FUSED_REG ||
+                          MODE == MODE_FUSED_REGX || MODE == MODE_FUSED_ST);
   // the record of k_cell_pre (fused CAIDVM_Marching / Euler steps, which the host always
   // precedes by it): copied to LDS below
   constexpr bool pre = FUSED && MARCH != MARCH_CIP;
@@ -1814,6 +1990,10 @@ __global__ __launch_bounds__(NWV * 64) void k_flux_relax(DevArgs A0,
           gather_regular<D, NDF, UNI, FT, CT, true>(A, G, eb, i, 0, nullptr, u, fl);
         else
           gather_regular<D, NDF, UNI, FT, CT, false>(A, G, eb, i, G.lev(i), G.keyp(i), u, fl);
+      } else if constexpr (MODE == MODE_FUSED_ST) {
+#pragma unroll
+        for (int k = 0; k < NDF; ++k) fl[k] = CT(0);
+        gather_stored<D, NDF, UNI, FT, CT>(A, G, eb, ne, i, UNI ? 0 : G.lev(i), G.keyp(i), u, f, fl);
       } else if (FUSED) {
         CT s[D][NDF];
 #pragma unroll
@@ -2548,52 +2728,30 @@ inline hipError_t launch_slope_t(const DevArgs& A, const int32_t* cells, int n, 
   return hipGetLastError();
 }
 
-template <int D, int NDF, bool UNI, class FT, int VPT, int WPI>
-inline hipError_t launch_slope_chunk_w(const DevArgs& A, const int2* work, int n, int maxh,
-                                       hipStream_t st) {
-  const dim3 grid(n), block(WPI * 64);
-  if (maxh == -1)   // regular cells, neighbours on the cell's grid: 2*D half fluxes
-    hipLaunchKernelGGL((k_slope_chunk<D, NDF, UNI, FT, 2 * D, VPT, 1, WPI>), grid, block, 0,
-                       st, A, work, n, KAH_RO_ARGS(A));
-  else if (maxh == -2)   // regular cells, neighbours on other grids
-    hipLaunchKernelGGL((k_slope_chunk<D, NDF, UNI, FT, 2 * D, VPT, 2, WPI>), grid, block, 0,
-                       st, A, work, n, KAH_RO_ARGS(A));
-  else if (maxh <= 4)
-    hipLaunchKernelGGL((k_slope_chunk<D, NDF, UNI, FT, 4, VPT, 0, WPI>), grid, block, 0, st,
-                       A, work, n, KAH_RO_ARGS(A));
-  else if (maxh <= 6)
-    hipLaunchKernelGGL((k_slope_chunk<D, NDF, UNI, FT, 6, VPT, 0, WPI>), grid, block, 0, st,
-                       A, work, n, KAH_RO_ARGS(A));
-  else if (maxh <= 8)
-    hipLaunchKernelGGL((k_slope_chunk<D, NDF, UNI, FT, 8, VPT, 0, WPI>), grid, block, 0, st,
-                       A, work, n, KAH_RO_ARGS(A));
-  else if (maxh <= 16)
-    hipLaunchKernelGGL((k_slope_chunk<D, NDF, UNI, FT, 16, VPT, 0, WPI>), grid, block, 0, st,
-                       A, work, n, KAH_RO_ARGS(A));
-  else
-    hipLaunchKernelGGL((k_slope_chunk<D, NDF, UNI, FT, 24, VPT, 0, WPI>), grid, block, 0, st,
-                       A, work, n, KAH_RO_ARGS(A));
+template <int D, int NDF, bool UNI, class FT, int NWV>
+inline hipError_t launch_slope_chunk_w(const DevArgs& A, const void* recs, const int4* work, int n,
+                                       int kind, hipStream_t st) {
+  const dim3 grid(n), block(NWV * 64);
+  const RegCell<D>* r = static_cast<const RegCell<D>*>(recs);
+  if (kind == 0)
+    hipLaunchKernelGGL((k_slope_chunk<D, NDF, UNI, FT, NWV>), grid, block, 0, st, A, work, n,
+                       KAH_RO_ARGS(A));
+  else if (kind == 1 || UNI)
+    hipLaunchKernelGGL((k_slope_chunk_reg<D, NDF, UNI, FT, true, NWV>), grid, block, 0, st, A, r,
+                       work, n, KAH_RO_ARGS(A));
+  else if constexpr (!UNI)
+    hipLaunchKernelGGL((k_slope_chunk_reg<D, NDF, UNI, FT, false, NWV>), grid, block, 0, st, A, r,
+                       work, n, KAH_RO_ARGS(A));
   return hipGetLastError();
 }
 
-template <int D, int NDF, bool UNI, class FT, int VPT>
-inline hipError_t launch_slope_chunk_v(const DevArgs& A, const int2* work, int n, int maxh,
-                                       int wpi, hipStream_t st) {
-  return wpi == 3 ? launch_slope_chunk_w<D, NDF, UNI, FT, VPT, 3>(A, work, n, maxh, st)
-                  : launch_slope_chunk_w<D, NDF, UNI, FT, VPT, 4>(A, work, n, maxh, st);
-}
-
 template <int D, int NDF, bool UNI, class FT>
-inline hipError_t launch_slope_chunk_t(const DevArgs& A, const int2* work, int n, int maxh,
-                                       int vpt, int wpi, hipStream_t st) {
+inline hipError_t launch_slope_chunk_t(const DevArgs& A, const void* recs, const int4* work, int n,
+                                       int kind, int waves, hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  switch (vpt) {
-    case 1: return launch_slope_chunk_v<D, NDF, UNI, FT, 1>(A, work, n, maxh, wpi, st);
-    case 2: return launch_slope_chunk_v<D, NDF, UNI, FT, 2>(A, work, n, maxh, wpi, st);
-    case 3: return launch_slope_chunk_v<D, NDF, UNI, FT, 3>(A, work, n, maxh, wpi, st);
-    case 4: return launch_slope_chunk_v<D, NDF, UNI, FT, 4>(A, work, n, maxh, wpi, st);
-    case 5: return launch_slope_chunk_v<D, NDF, UNI, FT, 5>(A, work, n, maxh, wpi, st);
-    case 6: return launch_slope_chunk_v<D, NDF, UNI, FT, 6>(A, work, n, maxh, wpi, st);
+  switch (waves) {
+    case 3: return launch_slope_chunk_w<D, NDF, UNI, FT, 3>(A, recs, work, n, kind, st);
+    case 4: return launch_slope_chunk_w<D, NDF, UNI, FT, 4>(A, recs, work, n, kind, st);
     default: return hipErrorInvalidValue;
   }
 }
@@ -2632,6 +2790,13 @@ inline hipError_t launch_fr_w(const DevArgs& A, const int32_t* cells, int n, int
       return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_REG, MARCH_CIP, NWV>(A, cells, n, lds, st);
     return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_REG, MARCH_EULER, NWV>(A, cells, n, lds, st);
   }
+  if (mode == MODE_FUSED_ST) {
+    if (march == MARCH_CAIDVM)
+      return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_ST, MARCH_CAIDVM, NWV>(A, cells, n, lds, st);
+    if (march == MARCH_CIP)
+      return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_ST, MARCH_CIP, NWV>(A, cells, n, lds, st);
+    return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_ST, MARCH_EULER, NWV>(A, cells, n, lds, st);
+  }
   if constexpr (!UNI) {   // on a shared grid every neighbour is on the cell's grid
     if (mode == MODE_FUSED_REGX) {
       if (march == MARCH_CAIDVM)
@@ -2654,23 +2819,30 @@ inline hipError_t launch_fr_d(const DevArgs& A, const int32_t* cells, int n, int
   if (nwv == 2) return launch_fr_w<D, NDF, UNI, FT, 2>(A, cells, n, mode, march, lds, st);
   if (nwv == 3) return launch_fr_w<D, NDF, UNI, FT, 3>(A, cells, n, mode, march, lds, st);
   if (nwv == 4) return launch_fr_w<D, NDF, UNI, FT, 4>(A, cells, n, mode, march, lds, st);
+  if constexpr (sizeof(FT) == 8) {
+    if (nwv == 16 && march == MARCH_CAIDVM) {   // the few irregular cells of an adapted mesh
+      if (mode == MODE_FUSED_ST)
+        return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_ST, MARCH_CAIDVM, 16>(A, cells, n, lds, st);
+      if (mode == MODE_FUSED)
+        return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED, MARCH_CAIDVM, 16>(A, cells, n, lds, st);
+    }
+  }
   return launch_fr_w<D, NDF, UNI, FT, 8>(A, cells, n, mode, march, lds, st);
 }
 
 // ------------------------------------------------------------------ immersed boundary
 // update_solid_cell! and update_solid_neighbor! (src/Boundary/Immersed_boundary.jl:122-148,
-// 367-483) between the slopes and the flux, in three launches over (solid cell or IB face, chunk
-// of IB_THREADS velocity cells) work items, one velocity cell per thread: the solid cells; the
-// extrapolated wall-side f with the partial sums of the wall density; the wall Maxwellian and
-// the there-half moments. Few solid cells and faces (tens) carry grids of up to ~3*10^4
-// velocity cells, so one workgroup per cell or face left most of the chip idle behind a serial
-// chain of dependent loads (1640 us per step on a 14^3 sphere, 24 faces, grids of 4.5k to 30k
-// cells; 85 us like this, bound by the latency of the three dependent launches); sources on
-// other grids are read through the overlap maps instead of a key search per source. Arithmetic
-// in FP64.
+// 367-483) between the slopes and the flux. Few solid cells and faces (tens) carry grids of up to
+// ~3*10^4 velocity cells, so the work per velocity cell (extrapolations, wall Maxwellian) runs in
+// chunks of IB_CHUNK velocity cells, one per thread, and only the sums over a grid run in one
+// workgroup per cell or face, over terms or values already in memory: with all of it in one
+// workgroup most of the chip idled behind a serial chain of dependent loads (1640 us per
+// step on a 14^3 sphere with 24 faces; 100 us like this, bound by the latency of the five
+// dependent launches). Sources on other grids are read
+// through the overlap maps instead of a key search per source. Arithmetic in FP64.
 
-// threads per workgroup of the immersed-boundary kernels = velocity cells per work item
-constexpr int IB_THREADS = IB_CHUNK;
+// threads per workgroup of the sums over a grid
+constexpr int IB_THREADS = 512;
 
 // sum of one value over the IB_THREADS-thread workgroup (every thread gets the sum; fixed
 // order: wave sums, then the waves' partials in index order)
@@ -2683,14 +2855,6 @@ __device__ inline double block_sum_ib(double v, double* sh) {
 #pragma unroll
   for (int k = 1; k < IB_THREADS / 64; ++k) t += sh[k];
   return t;
-}
-
-// sum over the work items [w0, w1) of their partials part[w*stride]: every lane of the wave gets
-// it (lane l adds the items w0+l, w0+l+64, ..., then the fixed shuffle tree)
-__device__ inline double items_sum(const double* part, int w0, int w1, int stride) {
-  double t = 0.0;
-  for (int w = w0 + int(threadIdx.x & 63); w < w1; w += 64) t += part[int64_t(w) * stride];
-  return wave_sum<>(t);
 }
 
 // sum_j wn_j (f_j + sdf_j . (x - x_j)) over the listed cells at velocity cell i, with
@@ -2760,44 +2924,29 @@ __device__ inline void ib_extrapolate(const DevArgs& A, const int32_t* cells, co
 }
 
 // update_solid_cell!: f of one chunk of solid cell s from its fluid face neighbours, written to
-// both state buffers (this step's IB faces read it; the next step keeps it), and the chunk's
-// partial moments; k_ib_wall forms w and prim from them
+// both state buffers (this step's IB faces read it; the next step keeps it); k_ib_sum forms w and
+// prim from it
 template <int D, int NDF, bool UNI, class FT>
-__global__ __launch_bounds__(IB_THREADS) void k_ib_solid(DevArgs A, IbArgs B) {
-  constexpr int NW = D + 2;
-  __shared__ double red[IB_THREADS / 64];
+__global__ __launch_bounds__(IB_CHUNK) void k_ib_solid(DevArgs A, IbArgs B) {
   const int2 wk = B.swork[blockIdx.x];
   const int s = B.solid[wk.x];
   const int b = B.snoff[wk.x], N = B.snoff[wk.x + 1] - b;
   const Grid<D, NDF, UNI, FT> G(A, s);
   const int n = G.n;
-  const int i = wk.y * IB_THREADS + int(threadIdx.x);
-  double m[NW];
+  const int i = wk.y * IB_CHUNK + int(threadIdx.x);
+  if (i >= n) return;
+  FT* df_a = static_cast<FT*>(B.df_a);
+  FT* df_b = static_cast<FT*>(B.df_b);
+  double u[D], f[NDF];
 #pragma unroll
-  for (int r = 0; r < NW; ++r) m[r] = 0.0;
-  if (i < n) {
-    FT* df_a = static_cast<FT*>(B.df_a);
-    FT* df_b = static_cast<FT*>(B.df_b);
-    double u[D];
+  for (int t = 0; t < D; ++t) u[t] = G.u(i, t);
+  ib_extrapolate<D, NDF, UNI, FT>(A, B.snb + b, B.smap + b, N, B.cmid, &B.cmid[int64_t(s) * D], i,
+                                  G.lev(i), G.keyp(i), u, f);
 #pragma unroll
-    for (int t = 0; t < D; ++t) u[t] = G.u(i, t);
-    double f[NDF];
-    ib_extrapolate<D, NDF, UNI, FT>(A, B.snb + b, B.smap + b, N, B.cmid, &B.cmid[int64_t(s) * D],
-                                    i, G.lev(i), G.keyp(i), u, f);
-    double fs[NDF];
-#pragma unroll
-    for (int k = 0; k < NDF; ++k) {
-      const FT v = FT(f[k]);
-      df_a[G.off * NDF + int64_t(k) * n + i] = v;
-      df_b[G.off * NDF + int64_t(k) * n + i] = v;
-      fs[k] = double(v);
-    }
-    moment_terms<D, NDF, double>(G.wt(i), u, fs, m);
-  }
-#pragma unroll
-  for (int r = 0; r < NW; ++r) {
-    const double t = block_sum_ib(m[r], red);
-    if (threadIdx.x == 0) B.spart[int64_t(blockIdx.x) * NW + r] = t;
+  for (int k = 0; k < NDF; ++k) {
+    const FT v = FT(f[k]);
+    df_a[G.off * NDF + int64_t(k) * n + i] = v;
+    df_b[G.off * NDF + int64_t(k) * n + i] = v;
   }
 }
 
@@ -2815,183 +2964,201 @@ __device__ inline int ib_cut_of(const int32_t* ci, int cnt, int i) {
 
 // update_solid_neighbor! of one chunk of an IB face, first part: image_df, boundary_slope! and
 // its positivity scaling give the extrapolated df at the wall (to the pseudo cell's rows), and
-// the chunk's share of the two flux sums of the wall density
+// the terms of the two flux sums of the wall density
 template <int D, int NDF, bool UNI, class FT>
-__global__ __launch_bounds__(IB_THREADS) void k_ib_face(DevArgs A, IbArgs B) {
-  __shared__ double red[IB_THREADS / 64];
+__global__ __launch_bounds__(IB_CHUNK) void k_ib_face(DevArgs A, IbArgs B) {
   const int2 wk = B.fwork[blockIdx.x];
   const IbFaceDesc F = B.faces[wk.x];
   const Grid<D, NDF, UNI, FT> G(A, F.donor);
   const Grid<D, NDF, UNI, FT> S(A, F.solid);
   const Grid<D, NDF, UNI, FT> PS(A, F.pseudo);   // the donor's grid, copied
   const int n = G.n;
-  const int i = wk.y * IB_THREADS + int(threadIdx.x);
-  double sf = 0.0, mur = 0.0;
-  if (i < n) {
-    FT* pa = static_cast<FT*>(B.df_a) + PS.off * NDF;
-    FT* ps = reinterpret_cast<FT*>(A.sdf) + PS.off * NDF * D;
-    double u[D];
+  const int i = wk.y * IB_CHUNK + int(threadIdx.x);
+  if (i >= n) return;
+  FT* pa = static_cast<FT*>(B.df_a) + PS.off * NDF;
+  FT* ps = reinterpret_cast<FT*>(A.sdf) + PS.off * NDF * D;
+  double u[D];
 #pragma unroll
-    for (int t = 0; t < D; ++t) u[t] = G.u(i, t);
-    const int li = G.lev(i);
-    const uint32_t* kp = G.keyp(i);
-    double im[NDF];
-    ib_extrapolate<D, NDF, UNI, FT>(A, B.img + F.img_beg, B.imap + F.img_beg, F.img_cnt, B.cmid,
-                                    F.ip, i, li, kp, u, im);
-    // boundary_slope!'s one-sided difference with the solid cell, walked across the grids
-    double sLv[NDF];
+  for (int t = 0; t < D; ++t) u[t] = G.u(i, t);
+  const int li = G.lev(i);
+  const uint32_t* kp = G.keyp(i);
+  double im[NDF];
+  ib_extrapolate<D, NDF, UNI, FT>(A, B.img + F.img_beg, B.imap + F.img_beg, F.img_cnt, B.cmid,
+                                  F.ip, i, li, kp, u, im);
+  // boundary_slope!'s one-sided difference with the solid cell, walked across the grids
+  double sLv[NDF];
 #pragma unroll
-    for (int k = 0; k < NDF; ++k) sLv[k] = 0.0;
-    for_overlap_m<D, NDF, UNI, FT>(A, S, F.smap, i, li, kp, [&](int jj, double den, double rden) {
-#pragma unroll
-      for (int k = 0; k < NDF; ++k) {
-        double d = G.f(i, k) - S.f(jj, k);
-        if (den != 1.0) d = d * rden;
-        sLv[k] += d / F.dxs;
-      }
-    });
-    double aux[NDF];
+  for (int k = 0; k < NDF; ++k) sLv[k] = 0.0;
+  for_overlap_m<D, NDF, UNI, FT>(A, S, F.smap, i, li, kp, [&](int jj, double den, double rden) {
 #pragma unroll
     for (int k = 0; k < NDF; ++k) {
-      const double fc = G.f(i, k);
-      const double sL = sLv[k];
-      double sl = minmod(sL, (im[k] - fc) / F.dxf);
-      sl = jl_min(fabs((im[k] - MACH_EPS) / (sl * F.dxL + MACH_EPS)), 1.0) * sl;
-      aux[k] = im[k] + sl * F.dxL;
-      pa[k * n + i] = FT(aux[k]);
-      if (A.ib_ssdf) A.ib_ssdf[F.row * NDF + int64_t(k) * n + i] = sl;
-      // the SolidNeighbor's slopes: the limited boundary slope along the face direction,
-      // zero across it (read by the DVM flux's reconstruction of the wall side)
-#pragma unroll
-      for (int d = 0; d < D; ++d) ps[(d * NDF + k) * n + i] = d == F.dir ? FT(sl) : FT(0);
+      double d = G.f(i, k) - S.f(jj, k);
+      if (den != 1.0) d = d * rden;
+      sLv[k] += d / F.dxs;
     }
-    double vn = u[0] * F.nrm[0];
+  });
+  double aux[NDF];
 #pragma unroll
-    for (int t = 1; t < D; ++t) vn += u[t] * F.nrm[t];
-    double M[2];
-    maxwell<D>(u, F.bc, A.K, M);
-    const int j = ib_cut_of(B.cut_idx + F.cut_beg, F.cut_cnt, i);
-    if (j >= 0) {
-      const double2 gw = B.cut_w[F.cut_beg + j];
-      mur = gw.y * vn * M[0];
-      sf = gw.x * vn * aux[0];
-    } else if (vn >= 0.0) {
-      mur = G.wt(i) * vn * M[0];
-    } else {
-      sf = G.wt(i) * vn * aux[0];
-    }
+  for (int k = 0; k < NDF; ++k) {
+    const double fc = G.f(i, k);
+    const double sL = sLv[k];
+    double sl = minmod(sL, (im[k] - fc) / F.dxf);
+    sl = jl_min(fabs((im[k] - MACH_EPS) / (sl * F.dxL + MACH_EPS)), 1.0) * sl;
+    aux[k] = im[k] + sl * F.dxL;
+    pa[k * n + i] = FT(aux[k]);
+    if (A.ib_ssdf) A.ib_ssdf[F.row * NDF + int64_t(k) * n + i] = sl;
+    // the SolidNeighbor's slopes: the limited boundary slope along the face direction,
+    // zero across it (read by the DVM flux's reconstruction of the wall side)
+#pragma unroll
+    for (int d = 0; d < D; ++d) ps[(d * NDF + k) * n + i] = d == F.dir ? FT(sl) : FT(0);
   }
-  const double t0 = block_sum_ib(sf, red);
-  const double t1 = block_sum_ib(mur, red);
-  if (threadIdx.x == 0) {
-    B.fpart[int64_t(blockIdx.x) * 2] = t0;
-    B.fpart[int64_t(blockIdx.x) * 2 + 1] = t1;
+  double vn = u[0] * F.nrm[0];
+#pragma unroll
+  for (int t = 1; t < D; ++t) vn += u[t] * F.nrm[t];
+  double M[2], sf = 0.0, mur = 0.0;
+  maxwell<D>(u, F.bc, A.K, M);
+  const int j = ib_cut_of(B.cut_idx + F.cut_beg, F.cut_cnt, i);
+  if (j >= 0) {
+    const double2 gw = B.cut_w[F.cut_beg + j];
+    mur = gw.y * vn * M[0];
+    sf = gw.x * vn * aux[0];
+  } else if (vn >= 0.0) {
+    mur = G.wt(i) * vn * M[0];
+  } else {
+    sf = G.wt(i) * vn * aux[0];
   }
+  B.term[F.row + i] = make_double2(sf, mur);
 }
 
-// update_solid_neighbor! of one chunk, second part, after the face's flux sums are complete: the
-// wall Maxwellian of zero net mass flux (cvc_Mu / cvc_density) on u.n >= 0, the cut-cell mixing
-// (cvc_correction!) and the chunk's row of the face's there half (df .* u[dir] over
-// rot*u[dir] > 0, calc_flux with a solid there side, src/Flux/CAIDVM.jl:110-112), which the
-// flux kernel sums like any other. The SolidNeighbor's df goes to the pseudo cell's rows of both
-// state buffers. The workgroups after the faces' take one solid cell each: w and prim from the
-// partial moments of k_ib_solid.
-template <int D, int NDF, bool UNI, class FT>
-__global__ __launch_bounds__(IB_THREADS) void k_ib_wall(DevArgs A, IbArgs B) {
-  constexpr int NW = D + 2;
-  if (int(blockIdx.x) >= B.nfw) {
-    const int q = int(blockIdx.x) - B.nfw;
-    if (threadIdx.x >= 64) return;
-    double w[NW], p[NW];
-#pragma unroll
-    for (int r = 0; r < NW; ++r) w[r] = items_sum(B.spart + r, B.swoff[q], B.swoff[q + 1], NW);
-    w[NW - 1] = 0.5 * w[NW - 1];
-    if (threadIdx.x == 0) {
-      const int s = B.solid[q];
-      get_prim<D>(w, A.gamma, p);
-#pragma unroll
-      for (int r = 0; r < NW; ++r) {
-        A.w[int64_t(s) * NW + r] = w[r];
-        A.prim[int64_t(s) * NW + r] = p[r];
-      }
-    }
-    return;
-  }
+// the wall density of zero net mass flux (cvc_Mu / cvc_density) of one face from its terms
+template <int D, bool UNI>
+__global__ __launch_bounds__(IB_THREADS) void k_ib_rho(DevArgs A, IbArgs B) {
   __shared__ double red[IB_THREADS / 64];
+  const IbFaceDesc& F = B.faces[blockIdx.x];
+  const int n = UNI ? A.uni_n : int(A.voff[F.donor + 1] - A.voff[F.donor]);
+  double sf = 0.0, mur = 0.0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n; i += IB_THREADS) {
+    const double2 t = B.term[F.row + i];
+    sf += t.x;
+    mur += t.y;
+  }
+  const double SF = block_sum_ib(sf, red);
+  const double MuR = block_sum_ib(mur, red);
+  if (threadIdx.x == 0) B.rho[blockIdx.x] = -SF / MuR;
+}
+
+// update_solid_neighbor! of one chunk, second part: the wall Maxwellian on u.n >= 0 and the
+// cut-cell mixing (cvc_correction!). The SolidNeighbor's df goes to the pseudo cell's rows of both
+// state buffers.
+template <int D, int NDF, bool UNI, class FT>
+__global__ __launch_bounds__(IB_CHUNK) void k_ib_wall(DevArgs A, IbArgs B) {
   const int2 wk = B.fwork[blockIdx.x];
   const IbFaceDesc F = B.faces[wk.x];
   const Grid<D, NDF, UNI, FT> G(A, F.donor);
   const Grid<D, NDF, UNI, FT> PS(A, F.pseudo);
   const int n = G.n;
-  const int w0 = B.fwoff[wk.x], w1 = B.fwoff[wk.x + 1];
-  const double SF = items_sum(B.fpart, w0, w1, 2);
-  const double MuR = items_sum(B.fpart + 1, w0, w1, 2);
-  const double rho = -SF / MuR;
-  const int i = wk.y * IB_THREADS + int(threadIdx.x);
-  double hm[NW];
+  const int i = wk.y * IB_CHUNK + int(threadIdx.x);
+  if (i >= n) return;
+  const double rho = B.rho[wk.x];
+  FT* pa = static_cast<FT*>(B.df_a) + PS.off * NDF;
+  FT* pb = static_cast<FT*>(B.df_b) + PS.off * NDF;
+  double u[D];
 #pragma unroll
-  for (int r = 0; r < NW; ++r) hm[r] = 0.0;
-  if (i < n) {
-    FT* pa = static_cast<FT*>(B.df_a) + PS.off * NDF;
-    FT* pb = static_cast<FT*>(B.df_b) + PS.off * NDF;
-    double u[D];
+  for (int t = 0; t < D; ++t) u[t] = G.u(i, t);
+  double vn = u[0] * F.nrm[0];
+#pragma unroll
+  for (int t = 1; t < D; ++t) vn += u[t] * F.nrm[t];
+  double M[2];
+  maxwell<D>(u, F.bc, A.K, M);
+  const int j = ib_cut_of(B.cut_idx + F.cut_beg, F.cut_cnt, i);
+#pragma unroll
+  for (int k = 0; k < NDF; ++k) {
+    const double Mk = M[k] * rho;
+    const double g = double(pa[k * n + i]);
+    double out;
+    if (j >= 0) {
+      const double2 gw = B.cut_w[F.cut_beg + j];
+      out = (gw.x * g + gw.y * Mk) / (gw.x + gw.y);
+    } else {
+      out = vn >= 0.0 ? Mk : g;
+    }
+    const FT v = FT(out);
+    pa[k * n + i] = v;
+    pb[k * n + i] = v;
+  }
+}
+
+// The sums over a grid of values in memory, one workgroup each: of face blockIdx.x the moments of
+// its there half (df .* u[dir] over rot*u[dir] > 0, calc_flux with a solid there side,
+// src/Flux/CAIDVM.jl:110-112), to the half flux's row, which the flux kernel sums like any other;
+// after the faces, of each solid cell its w and prim.
+template <int D, int NDF, bool UNI, class FT>
+__global__ __launch_bounds__(IB_THREADS) void k_ib_sum(DevArgs A, IbArgs B) {
+  constexpr int NW = D + 2;
+  __shared__ double red[IB_THREADS / 64];
+  const int q = int(blockIdx.x) - B.nf;
+  const bool face = q < 0;
+  const int fi = face ? int(blockIdx.x) : 0;
+  const int s = face ? B.faces[fi].pseudo : B.solid[q];
+  const int dir = face ? B.faces[fi].dir : 0;
+  const double rot = face ? B.faces[fi].rot : 0.0;
+  const Grid<D, NDF, UNI, FT> V(A, s);
+  const Grid<D, NDF, UNI, FT> G(A, face ? B.faces[fi].donor : s);
+  const FT* f = static_cast<const FT*>(B.df_a) + V.off * NDF;
+  const int n = G.n;
+  double m[NW];
+#pragma unroll
+  for (int r = 0; r < NW; ++r) m[r] = 0.0;
+#pragma unroll 2
+  for (int i = threadIdx.x; i < n; i += IB_THREADS) {
+    double u[D], v[NDF], mt[NW];
 #pragma unroll
     for (int t = 0; t < D; ++t) u[t] = G.u(i, t);
-    double vn = u[0] * F.nrm[0];
 #pragma unroll
-    for (int t = 1; t < D; ++t) vn += u[t] * F.nrm[t];
-    double M[2];
-    maxwell<D>(u, F.bc, A.K, M);
-    const int j = ib_cut_of(B.cut_idx + F.cut_beg, F.cut_cnt, i);
-    double out[NDF];
+    for (int k = 0; k < NDF; ++k) v[k] = double(f[k * n + i]);
+    const double ud = pick<D>(u, dir);
+    if (face) {
+      if (!(rot * ud > 0.0)) continue;
 #pragma unroll
-    for (int k = 0; k < NDF; ++k) {
-      const double Mk = M[k] * rho;
-      const double g = double(pa[k * n + i]);
-      if (j >= 0) {
-        const double2 gw = B.cut_w[F.cut_beg + j];
-        out[k] = (gw.x * g + gw.y * Mk) / (gw.x + gw.y);
-      } else {
-        out[k] = vn >= 0.0 ? Mk : g;
-      }
-      const FT v = FT(out[k]);
-      pa[k * n + i] = v;
-      pb[k * n + i] = v;
-      out[k] = double(v);
+      for (int k = 0; k < NDF; ++k) v[k] = v[k] * ud;
     }
-    const double ud = pick<D>(u, F.dir);
-    if (F.rot * ud > 0.0) {
-      double mic[NDF];
+    moment_terms<D, NDF, double>(G.wt(i), u, v, mt);
 #pragma unroll
-      for (int k = 0; k < NDF; ++k) mic[k] = out[k] * ud;
-      moment_terms<D, NDF, double>(G.wt(i), u, mic, hm);
-    }
+    for (int r = 0; r < NW; ++r) m[r] += mt[r];
   }
+  double w[NW];
 #pragma unroll
-  for (int r = 0; r < NW; ++r) {
-    const double t = block_sum_ib(hm[r], red);
-    if (threadIdx.x == 0) A.half_fw[(A.part_off[F.slot] + wk.y) * NW + r] = t;
+  for (int r = 0; r < NW; ++r) w[r] = block_sum_ib(m[r], red);
+  if (threadIdx.x != 0) return;
+  if (face) {
+#pragma unroll
+    for (int r = 0; r < NW; ++r) A.half_fw[A.part_off[B.faces[fi].slot] * NW + r] = w[r];
+  } else {
+    double p[NW];
+    w[NW - 1] = 0.5 * w[NW - 1];
+    get_prim<D>(w, A.gamma, p);
+#pragma unroll
+    for (int r = 0; r < NW; ++r) {
+      A.w[int64_t(s) * NW + r] = w[r];
+      A.prim[int64_t(s) * NW + r] = p[r];
+    }
   }
 }
 
 template <int D, int NDF, bool UNI, class FT>
 inline hipError_t launch_ib_t(const DevArgs& A, const IbArgs& B, hipStream_t st) {
-  if (B.nsw > 0) {
-    hipLaunchKernelGGL((k_ib_solid<D, NDF, UNI, FT>), dim3(B.nsw), dim3(IB_THREADS), 0, st, A, B);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
+  const dim3 chunk(IB_CHUNK), sum(IB_THREADS);
+  if (B.nsw > 0)
+    hipLaunchKernelGGL((k_ib_solid<D, NDF, UNI, FT>), dim3(B.nsw), chunk, 0, st, A, B);
   if (B.nfw > 0) {
-    hipLaunchKernelGGL((k_ib_face<D, NDF, UNI, FT>), dim3(B.nfw), dim3(IB_THREADS), 0, st, A, B);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((k_ib_face<D, NDF, UNI, FT>), dim3(B.nfw), chunk, 0, st, A, B);
+    hipLaunchKernelGGL((k_ib_rho<D, UNI>), dim3(B.nf), sum, 0, st, A, B);
+    hipLaunchKernelGGL((k_ib_wall<D, NDF, UNI, FT>), dim3(B.nfw), chunk, 0, st, A, B);
   }
-  if (B.nfw + B.ns > 0) {
-    hipLaunchKernelGGL((k_ib_wall<D, NDF, UNI, FT>), dim3(B.nfw + B.ns), dim3(IB_THREADS), 0, st,
-                       A, B);
-    return hipGetLastError();
-  }
-  return hipSuccess;
+  if (B.nf + B.ns > 0)
+    hipLaunchKernelGGL((k_ib_sum<D, NDF, UNI, FT>), dim3(B.nf + B.ns), sum, 0, st, A, B);
+  return hipGetLastError();
 }
 
 template <int D, int NDF, bool UNI, class FT>

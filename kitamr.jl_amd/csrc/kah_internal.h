@@ -43,7 +43,9 @@ struct SlopeNb {        // one neighbour in a slope stencil
   int32_t cell;         // data cell
   int32_t proj;         // 1: project with the neighbour's transverse slopes
   int32_t map;          // overlap map id of (owner grid, neighbour grid), MAP_SAME, or -1
-  int32_t pad;
+  int32_t n;            // the neighbour's grid size
+  // its first velocity cell in the state and in the geometry table, first overlap map entry or -1
+  int64_t off, g, mbase;
   double dm[3];         // transverse offsets (dm[dir] = 0)
   float dm_f[3];        // the same rounded to float (FP32 advection form)
   float pad_f;
@@ -77,6 +79,28 @@ struct SlopeDesc {      // per (fluid cell, direction)
   float inv_cnt_f[2];
 };
 
+// What the slope kernel reads of a regular cell (one same-level neighbour per side of every
+// direction): per direction and side the neighbour, the slope's distance, the face and the row
+// of the outgoing half flux; the cell's reconstruction point x, size dsr and, per direction, the
+// transverse face midpoints fmt (alike on both sides). *_f: the FP32 advection form's copies.
+struct RegSide {
+  int64_t off, g, mbase;   // neighbour's first velocity cell (state, geometry), overlap map or -1
+  int32_t n, map;          // its grid size; MAP_SAME, a map id or -1
+  double ds, rds;
+  double fm;               // face midpoint along the direction
+  int64_t row;             // first partial row of the half flux out of this side
+  float rds_f, dx_f;
+};
+template <int D>
+struct RegCell {
+  int64_t off, g;
+  int32_t n, pad;
+  RegSide s[D][2];
+  double fmt[D][D];
+  double x[D], dsr[D];
+  float dxt_f[D][D], dsr_f[D];
+};
+
 struct HalfDesc {       // one half flux computed by its owner cell in K1
   int32_t slot;         // output row in half_fw (pair*2 + side)
   int32_t data_cell;    // cell whose f/sdf feed the micro flux
@@ -84,6 +108,7 @@ struct HalfDesc {       // one half flux computed by its owner cell in K1
   int32_t sel;          // 0: rot*u[dir] <= 0 ; 1: rot*u[dir] > 0
   int32_t dir;
   int32_t bc;           // boundary condition (domain halves) or -1
+  int64_t ofb;          // element of oflux that holds its micro flux at velocity cell 0, or -1
   double rot;
   double xrec[3];       // cell-record midpoint used for the reconstruction
   double dsrec[3];      // cell-record size used by the limiter
@@ -94,6 +119,11 @@ struct HalfDesc {       // one half flux computed by its owner cell in K1
   float ds_f[3];
   float pad_f;
 };
+
+// How the fused gather reads a face side from stored micro fluxes (EntryDesc.kind): both sides
+// stored; f*u of the cell itself on both sets (uniform outflow); own stored and f*u of the other
+// cell (an immersed boundary's wall side, a solid cell); own stored and a boundary Maxwellian
+enum : int32_t { EK_STORED = 0, EK_SELF = 1, EK_PLAIN = 2, EK_MAXWELL = 3 };
 
 struct EntryDesc {      // one face side of a fluid cell, gathered in K2
   int32_t pair;
@@ -108,6 +138,14 @@ struct EntryDesc {      // one face side of a fluid cell, gathered in K2
   double area;          // signed face area, rot*A (or rot*A/2^(DIM-1))
   int64_t row[2];       // first partial row in half_fw of the face's here / there half flux
   int32_t rows[2];      // their row counts
+  // the other cell's first velocity cell in the state and in the geometry table, its grid size,
+  // and the first entry of the overlap map (-1: none, the key search is done in place)
+  int64_t oth_off, oth_g, mbase;
+  // elements of oflux that hold the own and the other side's micro flux through this face at
+  // velocity cell 0 (stored gather)
+  int64_t own_ofb, oth_ofb;
+  int32_t oth_n;
+  int32_t kind;         // EK_*
   double fmid[3];
   double xown[3], dsown[3];
   double xoth[3], dsoth[3];
@@ -345,9 +383,9 @@ __host__ __device__ inline double get_tau(const double* prim, double mu, double 
 
 // Contribution of one velocity cell to micro_to_macro (2D2F.jl:119-126, 3D1F.jl:109-123);
 // the 1/2 of the energy row is applied after the sum.
-// Terms of type T (float in the FP32 advection form), returned as double for the FP64 sums.
-template <int D, int NDF, class T = double>
-__host__ __device__ inline void moment_terms(T wt, const T* u, const T* f, double* m) {
+// Terms of type T (float in the FP32 advection form), returned as T or widened for the FP64 sums.
+template <int D, int NDF, class T = double, class R = double>
+__host__ __device__ inline void moment_terms(T wt, const T* u, const T* f, R* m) {
   if constexpr (D == 2) {
     m[0] = wt * f[0];
     m[1] = wt * u[0] * f[0];

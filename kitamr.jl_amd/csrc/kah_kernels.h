@@ -9,8 +9,10 @@ namespace kah {
 
 // MODE_FUSED_REG / MODE_FUSED_REGX: MODE_FUSED for regular cells (2*DIM faces to fluid cells
 // on the same level, limited or plain-slope reconstruction), gathered from the stored outgoing
-// micro fluxes; REG: every neighbour on the cell's velocity grid, REGX: on any grid
-enum { MODE_FLUX = 0, MODE_ITER = 1, MODE_FUSED = 2, MODE_FUSED_REG = 3, MODE_FUSED_REGX = 4 };
+// micro fluxes; REG: every neighbour on the cell's velocity grid, REGX: on any grid.
+// MODE_FUSED_ST: MODE_FUSED from stored micro fluxes for the other cells (EK_*)
+enum { MODE_FLUX = 0, MODE_ITER = 1, MODE_FUSED = 2, MODE_FUSED_REG = 3, MODE_FUSED_REGX = 4,
+       MODE_FUSED_ST = 5 };
 enum { MARCH_CAIDVM = 0, MARCH_EULER = 1, MARCH_CIP = 2 };
 constexpr int cpre_len(int dim) { return 3 * (dim + 2) + 8; }
 
@@ -99,16 +101,17 @@ struct DevArgs {
     (B).rec_ds = ro_recds;                                                                   \
   } while (0)
 
-constexpr int SLOPE_MAX_VPT = 6;   // velocity cells per thread of the chunked slope kernel: 1..6
+constexpr int SLOPE_MAX_VPT = 6;   // KAH_OPT_SLOPE_VPT: 1..6
 constexpr int MAX_ENTRIES = 24;    // face sides per cell (2*DIM sides, up to 2^(DIM-1) each)
 
 // f32: f, sdf and the next f stored as float (FP32 form), else double
 hipError_t launch_slope(const DevArgs& A, int dim, bool uni, bool f32, const int32_t* cells,
                         int n, int maxh, hipStream_t st);
-// work = (cell, chunk) pairs, one per workgroup of wpi (3 or 4) waves; chunk = vpt*64*wpi
-// velocity cells
-hipError_t launch_slope_chunk(const DevArgs& A, int dim, bool uni, bool f32, const int2* work,
-                              int n, int maxh, int vpt, int wpi, hipStream_t st);
+// work items (cell or record index, chunk, first and end velocity position of the chunk), one per
+// workgroup of `waves` (3 or 4) waves; kind 0: general cells; 1, 2: regular cells (index into recs,
+// RegCell<dim>), with every neighbour on the cell's velocity grid (1) or some on others (2)
+hipError_t launch_slope_chunk(const DevArgs& A, int dim, bool uni, bool f32, const void* recs,
+                              const int4* work, int n, int kind, int waves, hipStream_t st);
 hipError_t launch_flux_relax(const DevArgs& A, int dim, bool uni, bool f32, const int32_t* cells,
                              int n, int mode, int march, size_t lds, int waves_per_block,
                              hipStream_t st);
@@ -153,26 +156,24 @@ hipError_t launch_overlap_map(const DevArgs& A, int dim, const OvJob* jobs, int 
                               uint32_t* map, hipStream_t st);
 hipError_t launch_macro_slope(const DevArgs& A, int dim, bool uni, bool f32, const int32_t* cells,
                               int n, double* sw, hipStream_t st);
-// Immersed boundary (shared or adapted velocity grids): ns solid cells and the IB faces, each as
-// work items of IB_CHUNK velocity cells (nsw, nfw of them; work[x] = (solid cell or face index,
-// chunk), the items of index q are [woff[q], woff[q+1])), with their overlap map ids and the
-// partial sums of each item. Both state buffers df_a (this step's) and df_b are written.
+// Immersed boundary (shared or adapted velocity grids): ns solid cells and nf IB faces, each as
+// work items of IB_CHUNK velocity cells (nsw, nfw of them: (solid cell or face index, chunk)),
+// with the overlap map ids of their sources. Both state buffers df_a (this step's) and df_b are
+// written.
 constexpr int IB_CHUNK = 256;
 struct IbArgs {
-  int32_t ns, nsw, nfw;
+  int32_t ns, nsw, nf, nfw;
   const int32_t* solid;     // [ns] cells
   const int32_t* snoff;     // [ns+1] first fluid neighbour of each
   const int32_t* snb;       // fluid neighbours
   const int32_t* smap;      // overlap map id of (solid cell's grid, neighbour's grid)
   const int2* swork;
-  const int32_t* swoff;
-  double* spart;            // [nsw*(D+2)] moments
   const IbFaceDesc* faces;
   const int32_t* img;       // image stencils
   const int32_t* imap;      // overlap map id of (donor's grid, image cell's grid)
   const int2* fwork;
-  const int32_t* fwoff;
-  double* fpart;            // [nfw*2] the two flux sums of the wall density
+  double2* term;            // per face row: the velocity cell's terms of the wall density's sums
+  double* rho;              // [nf] wall densities
   const int32_t* cut_idx;
   const double2* cut_w;
   const double* cmid;
