@@ -2049,26 +2049,20 @@ int kah_vs_resolution(kah_ctx* C, double* vr) {
   if (!vr) return C->fail(KAH_EINVAL, "null vr");
   if (!C->vs_ok) return C->fail(KAH_EINVAL, "velocity root grid (vs_trees_num / vs_lo / vs_hi) not set");
   KAH_TRY(C->hip(hipSetDevice(C->P.device), "hipSetDevice"));
-  DBuf d_res;
-  KAH_TRY(C->alloc(d_res, sizeof(double) * size_t(2 * C->nc), "vs resolution"));
+  // the maxima over the fluid cells (vs_resolution(trees), src/Velocity_space/AMR.jl:137-151) on
+  // the device, in the staging buffer
+  KAH_TRY(C->reserve(C->d_xbuf, sizeof(double) * size_t(2 * C->nc + 2), "vs resolution"));
+  double* part = C->d_xbuf.as<double>();
   DevArgs A = make_args(C, 0.0);
-  KAH_TRY(C->hip(launch_vs_res(A, C->D, C->uni, C->f32, C->vsa, int(C->nc), d_res.as<double>(),
-                               C->stream), "vs resolution launch"));
-  std::vector<double> r(size_t(2 * C->nc));
-  KAH_TRY(C->hip(hipMemcpyAsync(r.data(), d_res.p, d_res.bytes, hipMemcpyDeviceToHost, C->stream),
+  KAH_TRY(C->hip(launch_vs_res(A, C->D, C->uni, C->f32, C->vsa, int(C->nc), part, C->stream),
+                 "vs resolution launch"));
+  KAH_TRY(C->hip(launch_vs_res_max(part, C->d_benc.as<int32_t>(), int(C->nc), part + 2 * C->nc,
+                                   C->stream),
+                 "vs resolution maxima launch"));
+  KAH_TRY(C->hip(hipMemcpyAsync(vr, part + 2 * C->nc, 2 * sizeof(double), hipMemcpyDeviceToHost,
+                                C->stream),
                  "vs resolution download"));
-  KAH_TRY(C->hip(hipStreamSynchronize(C->stream), "vs resolution"));
-  // maxima over the fluid cells (vs_resolution(trees), src/Velocity_space/AMR.jl:137-151)
-  double dres = 0.0, eres = 0.0;
-  auto jmax = [](double a, double b) { return (a != a) ? a : (b != b) ? b : (b > a ? b : a); };
-  for (int64_t c = 0; c < C->nc; ++c) {
-    if (C->benc[c] < 0) continue;
-    dres = jmax(r[size_t(2 * c)], dres);
-    eres = jmax(r[size_t(2 * c + 1)], eres);
-  }
-  vr[0] = dres;
-  vr[1] = eres;
-  return KAH_OK;
+  return C->hip(hipStreamSynchronize(C->stream), "vs resolution");
 }
 
 int kah_vs_resolution_noalloc(kah_ctx* C, double* vr) {
@@ -2115,12 +2109,13 @@ int kah_vs_flags(kah_ctx* C, const kah_vs_adapt* p, const double* vr, uint8_t* f
   P.tl = p->coeff_lohner;
   P.vr[0] = vr[0];
   P.vr[1] = vr[1];
-  DBuf d_fl;
-  KAH_TRY(C->alloc(d_fl, size_t(C->np), "vs flags"));
+  // keys in LDS up to 32 KiB a workgroup (five of them per CU); larger grids search in memory
+  P.key_cap = C->max_n <= 8192 ? C->max_n : 8192;
+  KAH_TRY(C->reserve(C->d_xbuf, size_t(C->np), "vs flags"));   // the staging buffer
   DevArgs A = make_args(C, 0.0);
-  KAH_TRY(C->hip(launch_vs_flags(A, C->D, C->uni, C->f32, P, int(C->nc), d_fl.as<uint8_t>(),
+  KAH_TRY(C->hip(launch_vs_flags(A, C->D, C->uni, C->f32, P, int(C->nc), C->d_xbuf.as<uint8_t>(),
                                  C->stream), "vs flags launch"));
-  KAH_TRY(C->hip(hipMemcpyAsync(flags, d_fl.p, size_t(C->np), hipMemcpyDeviceToHost, C->stream),
+  KAH_TRY(C->hip(hipMemcpyAsync(flags, C->d_xbuf.p, size_t(C->np), hipMemcpyDeviceToHost, C->stream),
                  "vs flags download"));
   return C->hip(hipStreamSynchronize(C->stream), "vs flags");
 }

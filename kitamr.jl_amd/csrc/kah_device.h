@@ -2337,7 +2337,10 @@ inline hipError_t launch_mirror_t(const DevArgs& A, const int32_t* cells, const 
 // resolution, the per-velocity-cell criteria (Criteria.jl), the remap of the state onto the
 // rebuilt grids (Rebuild.jl) and the conservative I-projection. The face neighbours of the
 // Loehner indicator come from a binary search over the cell's keys (the grid is in key
-// order), as VsNeighborIndex locates them (Neighbor.jl:126-201).
+// order), as VsNeighborIndex locates them (Neighbor.jl:126-201): the stored keys of an adapted
+// grid, from an LDS copy where it fits (P.key_cap). Forming each probed key from the cell's
+// midpoint took three quarters of k_vs_flags (1388 -> 354 us for 6.2 M velocity cells; what is
+// left is FP64 arithmetic of the criteria and the searches' latency).
 template <int D>
 __device__ inline uint64_t vs_code(const VsArgs& P, const int64_t (&g)[D]) {
   int64_t root = 0;
@@ -2356,11 +2359,13 @@ template <int D, int NDF, bool UNI, class FT>
 struct VsGrid {
   const Grid<D, NDF, UNI, FT>& G;
   const VsArgs& P;
+  const uint32_t* keys;   // adapted grids: the cell's keys
   __device__ int lev(int j) const { return int(G.A.glev[G.goff() + j]); }
   __device__ double size(int j, int d) const {
     return P.hf[d] * double(int64_t(1) << (P.L - lev(j)));
   }
   __device__ uint64_t key(int j) const {   // _corner_index, Neighbor.jl:38-41
+    if constexpr (!UNI) return keys[j];
     int64_t g[D];
 #pragma unroll
     for (int d = 0; d < D; ++d)
@@ -2459,8 +2464,12 @@ __global__ __launch_bounds__(256) void k_vs_flags(DevArgs A, VsArgs P,
   __shared__ double scl[2];
   const int c = blockIdx.x;
   const Grid<D, NDF, UNI, FT> G(A, c);
-  const VsGrid<D, NDF, UNI, FT> X{G, P};
   const int n = G.n;
+  extern __shared__ uint32_t skeys[];
+  const bool local = !UNI && n <= P.key_cap;
+  const VsGrid<D, NDF, UNI, FT> X{G, P, local ? skeys : (UNI ? nullptr : A.gkey + G.g)};
+  if (local)   // the barriers of block_min2 below stand between this copy and its use
+    for (int i = threadIdx.x; i < n; i += 256) skeys[i] = G.key(i);
   const bool lohner = P.mode == VS_LOHNER;
   // vs_lohner_scales: peaks of |h| and |b|
   double a1 = 0.0, a2 = 0.0;
@@ -2656,7 +2665,8 @@ inline hipError_t launch_vs_t(const DevArgs& A, int which, const VsArgs& P, int 
   if (which == 0)
     hipLaunchKernelGGL((k_vs_res<D, NDF, UNI, FT>), dim3(nc), dim3(256), 0, st, A, P, out);
   else
-    hipLaunchKernelGGL((k_vs_flags<D, NDF, UNI, FT>), dim3(nc), dim3(256), 0, st, A, P, flags);
+    hipLaunchKernelGGL((k_vs_flags<D, NDF, UNI, FT>), dim3(nc), dim3(256),
+                       UNI ? 0 : sizeof(uint32_t) * size_t(P.key_cap), st, A, P, flags);
   return hipGetLastError();
 }
 template <int D, int NDF, class FT>

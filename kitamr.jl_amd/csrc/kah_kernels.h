@@ -128,6 +128,7 @@ struct VsArgs {
   int64_t tn[3], stride[3];
   int32_t L;               // vs_maxlevel
   int32_t mode;            // KAH_VS_*
+  int32_t key_cap;         // largest grid whose keys k_vs_flags copies to LDS
   double cl, cg, tl;       // ADAPT_COEFFI_VS_LOCAL / _GLOBAL / _LOHNER
   double vr[2];            // Velocity_Resolution
   double wfine;            // weight of a finest velocity cell

@@ -254,3 +254,26 @@ def test_balance_rounds_inject_on_the_device(name, precision):
         assert rel_err(g["df"], oo["df"]) < 1e-12
         o.close()
     dev.close()
+
+
+# Grids on both sides of the 8,192 velocity cells whose keys the criteria kernel copies to LDS
+# (7.8k and 8.5k), 3D ones above it, and a shared grid, whose keys it forms itself: flags are
+# whole numbers, equal bit for bit.
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["below", "above", "above3d", "shared"])
+def test_flags_key_copy_edges(name):
+    case = {"below": lambda: cases.riemann_2d(n=4, nv=44, vs_levels=2),
+            "above": lambda: cases.riemann_2d(n=4, nv=46, vs_levels=2),
+            "above3d": lambda: cases.box_3d(n=2, nv=16, vs_levels=1),
+            "shared": lambda: cases.riemann_2d(n=4, nv=12)}[name]()
+    sizes = np.diff(case.topo["vs_offset"])
+    say(f"[vs] key copy {name}: grids {sizes.min()}-{sizes.max()}")
+    dev, orc = pair(case)
+    dev.step(case.dt_xi, 0)
+    _sync_oracle(dev, orc)
+    vr = dev.vs_resolution()
+    assert np.array_equal(vr, orc.vs_resolution())
+    p = abi.vs_adapt_params("lohner")
+    assert np.array_equal(dev.vs_flags(p, vr), orc.vs_flags(p, vr))
+    dev.close()
+    orc.close()
