@@ -284,6 +284,8 @@ int kah_load_restart(kah_ctx* ctx, const int64_t* vs_nums, const int64_t* bound_
                      const double* ws, const double* vs_df);
 
 /* ---- the per-step path --------------------------------------------------------------- */
+/* These calls queue their work on the context's stream and return without waiting for the device,
+ * except where a residual is sampled; every other call on the context is ordered behind them. */
 /* slope!(p4est,ka), src/Flux/Slope.jl:1047-1070: level-ordered velocity-space slopes
  * with the transverse correction on coarse-neighbour faces. dt is status.Δt of the step
  * (limit_Δt!, src/Theory/Iterate.jl:27-39); it is needed here because the per-face
@@ -330,7 +332,8 @@ int64_t kah_device_bytes(const kah_ctx* ctx);
  * (CAIDVM flux), cells whose 2*DIM faces go to fluid cells on the same level, which read the
  * outgoing micro fluxes the slope kernel stores instead of reconstructing; 0 runs every cell
  * through the general slope and gather. Takes effect at the next kah_set_topology.
- * KAH_OPT_BRANCHES: 1..4 (default 4) streams over which the independent launches of a phase
+ * KAH_OPT_BRANCHES: 1..4 (default: 4, or 1 for a phase of fewer than 786,432 velocity cells,
+ * which forking would only delay) streams over which the independent launches of a phase
  * (slope launches of one projection depth, flux/relaxation launches) are spread, forked from
  * and joined back to the context's stream by events (parallel branches of a captured graph).
  * No counterpart in the reference. */

@@ -44,6 +44,7 @@ struct DBuf {
 };
 
 struct LevelBin {
+  int64_t cells = 0;   // velocity cells of its grids
   int level;
   int maxh;       // per-cell kernel: half fluxes; chunked kernel: its kind
   int waves = 4;  // chunked kernel: waves per workgroup
@@ -141,7 +142,15 @@ struct kah_ctx {
   // the context's stream by events (parallel branches of the captured graph), so that small
   // launches run beside large ones instead of after them; 1: in order on the context's stream
   static constexpr int MAX_BRANCHES = 4;
-  int branches = MAX_BRANCHES;   // measured: 7.95 -> 7.35 ms per step on the adapted cylinder
+  int branches = 0;   // 0: not set by the caller, branches_for decides
+  // Fork and join cost some 20 us a phase, an empty step 45 us: worth it where the launches of a
+  // phase are long enough to overlap. A step of 65 k velocity cells takes 84 us on four streams
+  // and 37 us on one, of 435 k (split calls) 193 and 136; of 1.1 M on several grid sizes 241 and
+  // 283, of 2.5 M on a refined 3D mesh 290 and 325, of 151 M on the adapted cylinder 7.35 and
+  // 7.95 ms.
+  int branches_for(int64_t cells) const {
+    return branches ? branches : (cells >= 768 * 1024 ? MAX_BRANCHES : 1);
+  }
   hipStream_t side[MAX_BRANCHES - 1] = {};
   std::vector<hipEvent_t> ev_pool;   // fork/join events, reused step after step
   size_t ev_next = 0;
@@ -839,6 +848,7 @@ int slope_bins(kah_ctx* C, const SlopeTables& t, const std::vector<char>& walled
         lb->maxh = kind;
         lb->waves = w;
         lb->n = int(it->second.size());
+        for (const int4& w4 : it->second) lb->cells += w4.w - w4.z;
         lb->chunked = true;
         KAH_TRY(C->upload(lb->items, it->second.data(), it->second.size(), "slope work items"));
       }
@@ -848,6 +858,7 @@ int slope_bins(kah_ctx* C, const SlopeTables& t, const std::vector<char>& walled
       lb->level = L;
       lb->maxh = kv.first;
       lb->n = int(kv.second.size());
+      for (int32_t c : kv.second) lb->cells += (*t.voff)[size_t(c) + 1] - (*t.voff)[size_t(c)];
       lb->chunked = false;
       KAH_TRY(C->upload(lb->items, kv.second.data(), kv.second.size(), "level cells"));
     }
@@ -1662,7 +1673,9 @@ int run_slope(kah_ctx* C, const DevArgs& A) {
   for (size_t b0 = 0; b0 < C->bins.size();) {
     size_t b1 = b0;
     while (b1 < C->bins.size() && C->bins[b1]->level == C->bins[b0]->level) ++b1;
-    const int nb = std::min<int>(C->branches, int(b1 - b0));
+    int64_t cells = 0;
+    for (size_t j = b0; j < b1; ++j) cells += C->bins[j]->cells;
+    const int nb = std::min<int>(C->branches_for(cells), int(b1 - b0));
     KAH_TRY(fork_branches(C, nb));
     for (size_t j = b0; j < b1; ++j) {
       const LevelBin* b = C->bins[j];
@@ -1723,7 +1736,7 @@ int run_flux_relax(kah_ctx* C, const DevArgs& A, int mode) {
                                    C->stream),
                    "cell prologue launch"));
   // the bins write disjoint cells and read only what the slope phase wrote
-  const int nb = std::min<int>(C->branches, int(C->frbins.size()));
+  const int nb = std::min<int>(C->branches_for(C->phase_cells), int(C->frbins.size()));
   KAH_TRY(fork_branches(C, nb));
   for (size_t j = 0; j < C->frbins.size(); ++j) {
     const kah_ctx::FrBin* b = C->frbins[j];
@@ -2223,8 +2236,7 @@ int kah_slope(kah_ctx* C, double dt) {
   if (!C) return KAH_EINVAL;
   KAH_TRY(check_ready(C, dt));
   DevArgs A = make_args(C, dt);
-  KAH_TRY(run_slope(C, A));
-  return C->hip(hipStreamSynchronize(C->stream), "slope");
+  return run_slope(C, A);   // every later call is ordered behind it on the stream
 }
 
 int kah_flux(kah_ctx* C, double dt) {
@@ -2236,8 +2248,7 @@ int kah_flux(kah_ctx* C, double dt) {
   }
   DevArgs A = make_args(C, dt);
   KAH_TRY(run_ib(C, A));
-  KAH_TRY(run_flux_relax(C, A, MODE_FLUX));
-  return C->hip(hipStreamSynchronize(C->stream), "flux");
+  return run_flux_relax(C, A, MODE_FLUX);
 }
 
 int kah_get_ib(kah_ctx* C, double* aux_df) {
@@ -2263,7 +2274,6 @@ int kah_iterate(kah_ctx* C, double dt, int64_t step, double* sum_res, double* su
   }
   DevArgs A = make_args(C, dt);
   KAH_TRY(run_flux_relax(C, A, MODE_ITER));
-  KAH_TRY(C->hip(hipStreamSynchronize(C->stream), "iterate"));
   return finish_iterate(C, step, sum_res, sum_avg);
 }
 
