@@ -814,6 +814,7 @@ template <int D, class ChunksOf>
 int slope_bins(kah_ctx* C, const SlopeTables& t, const std::vector<char>& walled,
                const std::vector<int>& depth, int Dmax, ChunksOf&& chunks_of) {
   std::vector<RegCell<D>> regs;
+  if (C->reg_mode) regs.reserve(C->fluid.size());
   for (int L = 0; L <= Dmax; ++L) {
     std::map<int, std::vector<int32_t>> lists;   // walled cells by half-flux count
     std::map<int, std::vector<int4>> works;      // 8*kind + waves
@@ -824,12 +825,13 @@ int slope_bins(kah_ctx* C, const SlopeTables& t, const std::vector<char>& walled
         lists[nh <= 4 ? 4 : (nh <= 8 ? 8 : (nh <= 16 ? 16 : 24))].push_back(c);
         continue;
       }
-      RegCell<D> r;
-      const int kind = C->reg_mode ? slope_record<D>(C, t, c, r) : 0;
+      int kind = 0;
       int32_t idx = c;
-      if (kind) {
-        idx = int32_t(regs.size());
-        regs.push_back(r);
+      if (C->reg_mode) {
+        regs.emplace_back();
+        kind = slope_record<D>(C, t, c, regs.back());
+        if (kind) idx = int32_t(regs.size()) - 1;
+        else regs.pop_back();
       }
       const int64_t n = (*t.voff)[size_t(c) + 1] - (*t.voff)[size_t(c)];
       const auto ck = chunks_of(c);
@@ -1249,6 +1251,13 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
   std::vector<int32_t> hoff(size_t(nc + 1), 0), eoff(size_t(nc + 1), 0);
   std::vector<HalfDesc> halves;
   std::vector<EntryDesc> ents;
+  size_t n_hal = 0, n_ent = 0;
+  for (int64_t c = 0; c < nc; ++c) {
+    n_hal += B.hal[c].size();
+    n_ent += B.ent[c].size();
+  }
+  halves.reserve(n_hal);
+  ents.reserve(n_ent);
   for (int64_t c = 0; c < nc; ++c) {
     hoff[c] = int32_t(halves.size());
     eoff[c] = int32_t(ents.size());
@@ -1422,27 +1431,24 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
       e.rows[sd] = pcnt[size_t(2 * e.pair + sd)];
     }
     e.mbase = e.map >= 0 ? mbase[size_t(e.map)] : -1;
-    if (e.oth_cell < 0) continue;
+    e.own_ofb = of_slot[size_t(2 * e.pair + e.side)];
+    e.oth_ofb = of_slot[size_t(2 * e.pair + 1 - e.side)];
+    e.kind = -1;   // no stored form
+    const bool same = C->uni || e.map == MAP_SAME;
+    if (e.oth_cell < 0) {
+      if (e.oth_mode == MI_SELF_PLAIN && e.own_mode == MI_PLAIN) e.kind = EK_SELF;
+      else if ((e.oth_mode == MI_MAXWELL || e.oth_mode == MI_WALL) && e.own_ofb >= 0)
+        e.kind = EK_MAXWELL;
+      continue;
+    }
     e.oth_off = voff[size_t(e.oth_cell)];
     e.oth_n = int32_t(voff[size_t(e.oth_cell) + 1] - e.oth_off);
     e.oth_g = C->uni ? 0 : gof[size_t(e.oth_cell)];
-  }
-  for (int64_t c = 0; c < nc; ++c)
-    for (int x = eoff[c]; x < eoff[c + 1]; ++x) {
-      EntryDesc& e = ents[size_t(x)];
-      e.own_ofb = of_slot[size_t(2 * e.pair + e.side)];
-      e.oth_ofb = of_slot[size_t(2 * e.pair + 1 - e.side)];
-      e.kind = -1;   // no stored form
-      const bool same = C->uni || e.map == MAP_SAME;
-      if (e.oth_cell < 0) {
-        if (e.oth_mode == MI_SELF_PLAIN && e.own_mode == MI_PLAIN) e.kind = EK_SELF;
-        else if ((e.oth_mode == MI_MAXWELL || e.oth_mode == MI_WALL) && e.own_ofb >= 0)
-          e.kind = EK_MAXWELL;
-      } else if (e.own_ofb >= 0) {
-        if (e.oth_mode == MI_PLAIN && same) e.kind = EK_PLAIN;
-        else if (e.oth_mode != MI_PLAIN && e.oth_ofb >= 0) e.kind = EK_STORED;
-      }
+    if (e.own_ofb >= 0) {
+      if (e.oth_mode == MI_PLAIN && same) e.kind = EK_PLAIN;
+      else if (e.oth_mode != MI_PLAIN && e.oth_ofb >= 0) e.kind = EK_STORED;
     }
+  }
   KAH_TRY(C->upload(C->d_ents, ents.data(), ents.size(), "entry descriptors"));
 
   // state buffers
