@@ -313,9 +313,8 @@ int64_t kah_phase_cells(const kah_ctx* ctx);
 /* Device bytes held by the context (state + topology). */
 int64_t kah_device_bytes(const kah_ctx* ctx);
 /* Launch options (autotuned schedule choices). KAH_OPT_FLUX_WAVES: waves per workgroup of
- * the flux/relaxation kernel (2, 3, 4 or 8; 0, the default, chooses per size-class launch: for
- * the 2D FP32 form on adapted velocity grids 2 when the LDS copy of f* takes at most 8 KiB
- * (grids of up to 640 cells), 4 up to 40 KiB, else 8; 8 for 3D and the other forms);
+ * the flux/relaxation kernel (2, 3, 4 or 8; default by shape: on shared grids the fewest that keep
+ * the GPU occupied, on adapted grids by the size of the LDS copy of f*, up to 16 for 3D grids);
  * a change drops captured graphs. KAH_OPT_SLOPE_VPT: velocity cells per thread of the slope
  * kernel (1..6, default 3 in 2D and 6 in 3D): in the FP32 form of 3-wave or 4-wave workgroups,
  * per cell whichever pads the grid least, in the FP64 form the number its even cut of a grid

@@ -108,24 +108,53 @@ struct kah_ctx {
   int64_t part_rows = 0;
   int cur = 0;
   bool timing = false;
-  // waves per workgroup of the flux/relaxation kernel; 0: by shape. The FP32 form on adapted
-  // grids whose LDS copy of f* leaves room for four or more workgroups per CU runs 4-wave
-  // workgroups (more of them resident: measured 1.4x on 2D grids of 1.6k cells), and 2-wave
-  // workgroups for the smallest size class (grids of up to 640 velocity cells: -7 % on the
-  // flux phase of the adapted cylinder, whose free stream has 568-cell grids); larger grids,
-  // whose LDS already limits residency, the 3D grids (8 waves: -14 % on the sphere's flux
-  // phase against 4) and the other forms run 8 waves.
+  // Waves per workgroup of the flux/relaxation kernel; 0: by shape, as follows.
+  // Every wave pays for its share of the workgroup's two or three compensated reductions (some
+  // hundred instructions each, a quarter of the kernel on 784 velocity cells with 8 waves), so
+  // few waves with many velocity cells each issue least, as long as enough of them are resident
+  // to hide the memory latency: the workgroups per CU are bounded by the LDS copy of f*, by the
+  // registers (7 waves per SIMD, 4 for irregular cells) and by the number of cells.
+  // Shared grids: the fewest waves that keep 20 of a CU's 32 resident (12 for irregular cells),
+  // else the number that keeps most. Steps against 8 waves: 64^2 leaves with 16^2, 28^2 and 40^2
+  // velocity cells 113 -> 98, 189 -> 175 and 443 -> 442 us (3, 3 and 8 waves), 32^2 refined
+  // leaves with 28^2 996 -> 890, FP32 form 145 -> 130, a 3D box with 12^3 287 -> 282. The Newton
+  // iteration of CIP_Marching is mostly reductions: half the residency does, 40^2 leaves with
+  // 24^2 130 -> 98 us on 2 waves, 40^2 with 40^2 190 -> 188 on 4; 144 cells stay on 8 (63 against
+  // 74 us on 2).
+  // Adapted grids: several size classes run side by side. 2D FP32 form: 2 waves for the smallest
+  // class (8 KiB), 4 while four or more workgroups fit, else 8. 3D: 16 waves where the LDS copy
+  // leaves one or two workgroups per CU or is in global memory (few, long workgroups that the
+  // step waits for: 14^3 sphere, FP32 form 1237 -> 1090 us per step, FP64 1443 -> 1414), else 8.
+  // 2D FP64: 8 (16 on every class above 56 KiB: 450 -> 470 us on the 75^2 cylinder), but 16 for a
+  // small launch of irregular cells with larger grids (459 -> 435).
+  // cells: those of the kind that run side by side
   int fr_waves = 0;
-  // In the FP64 form a small launch of irregular cells with larger grids runs 16 waves: too few
-  // workgroups to fill the GPU, its time is one workgroup's (75^2 adapted cylinder 0.459 -> 0.435
-  // ms per step; grids of 640 cells and fewer gain nothing).
-  int flux_waves(size_t lds, int64_t n, bool irregular, size_t cells) const {
+  int flux_waves(size_t lds, int64_t n, bool irregular, int64_t cells) const {
     if (fr_waves) return fr_waves;
-    if (!f32 && !uni && irregular && cells < 1024 && n > 640 && P.marching == KAH_MARCH_CAIDVM)
-      return 16;
-    if (D != 2 || !f32 || uni || lds == 0) return 8;   // 3D grids (4.5k cells and up): 8 waves
-    if (lds <= 8 * 1024) return 2;
-    return lds <= 40 * 1024 ? 4 : 8;
+    const bool cip = P.marching == KAH_MARCH_CIP;
+    if (!uni) {
+      if (D == 2 && f32 && lds > 0) {
+        if (lds <= 8 * 1024) return 2;
+        return lds <= 40 * 1024 ? 4 : 8;
+      }
+      if (P.marching != KAH_MARCH_CAIDVM) return 8;
+      if (D == 3) return lds == 0 || lds > 56 * 1024 ? 16 : 8;
+      return !f32 && irregular && cells < 1024 && n > 640 ? 16 : 8;
+    }
+    const int64_t by_lds = lds ? std::max<int64_t>(1, (160 * 1024) / int64_t(lds + 1536)) : 32;
+    const int regs = irregular ? 16 : 28, want = irregular || cip ? 12 : 20;
+    int at = 8;
+    int64_t most = 0;
+    for (int w : {2, 3, 4, 8}) {
+      if (w == (cip ? 3 : 2)) continue;
+      const int64_t r = std::min({by_lds * w, int64_t(regs / w * w), cells * w / 256});
+      if (r >= want) return w;
+      if (r > most) {
+        most = r;
+        at = w;
+      }
+    }
+    return at;
   }
   // launches of the flux/relaxation kernel: the fluid cells by grid size, each launch with
   // the LDS its largest grid needs (0: the global scratch area)
@@ -1520,6 +1549,7 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
     // irregular ones are launched first, as in the slope phase
     std::map<int, std::vector<int32_t>> lists;
     std::map<int, int64_t> bmax;
+    std::map<int, int64_t> bcells;   // of a size class, whatever their path
     for (int32_t c : C->fluid) {
       const int64_t n = T->vs_offset[c + 1] - T->vs_offset[c];
       int b = 0;
@@ -1529,6 +1559,7 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
       const int key = (64 * bulk + 63 - b) * 4 + (C->reg_mode ? cls : 0);   // large grids first
       lists[key].push_back(c);
       bmax[key] = std::max(bmax[key], n);
+      ++bcells[key / 4];
     }
     bool need_scratch = false;
     for (auto& kv : lists) {
@@ -1543,7 +1574,8 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
                                                                        int64_t(C->max_n));
       fb->lds = sc_elem * size_t(NDF + 1) * size_t(std::max(cap, bmax[key]));
       if (fb->lds > C->lds_limit) fb->lds = 0;
-      fb->waves = C->flux_waves(fb->lds, std::max(cap, bmax[key]), key < 256, kv.second.size());
+      fb->waves = C->flux_waves(fb->lds, std::max(cap, bmax[key]), key < 256,
+                                key < 256 ? bcells[key / 4] : int64_t(C->fluid.size()));
       need_scratch |= fb->lds == 0;
       KAH_TRY(C->upload(fb->cells, kv.second.data(), kv.second.size(), "flux cells"));
     }

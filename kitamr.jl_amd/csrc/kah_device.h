@@ -2829,12 +2829,19 @@ inline hipError_t launch_fr_d(const DevArgs& A, const int32_t* cells, int n, int
   if (nwv == 2) return launch_fr_w<D, NDF, UNI, FT, 2>(A, cells, n, mode, march, lds, st);
   if (nwv == 3) return launch_fr_w<D, NDF, UNI, FT, 3>(A, cells, n, mode, march, lds, st);
   if (nwv == 4) return launch_fr_w<D, NDF, UNI, FT, 4>(A, cells, n, mode, march, lds, st);
-  if constexpr (sizeof(FT) == 8) {
-    if (nwv == 16 && march == MARCH_CAIDVM) {   // the few irregular cells of an adapted mesh
+  // 3D grids too large for several workgroups per CU; in the 2D FP64 form irregular cells
+  if constexpr (!UNI && (D == 3 || sizeof(FT) == 8)) {
+    if (nwv == 16 && march == MARCH_CAIDVM) {
       if (mode == MODE_FUSED_ST)
         return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_ST, MARCH_CAIDVM, 16>(A, cells, n, lds, st);
       if (mode == MODE_FUSED)
         return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED, MARCH_CAIDVM, 16>(A, cells, n, lds, st);
+      if constexpr (D == 3) {
+        if (mode == MODE_FUSED_REG)
+          return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_REG, MARCH_CAIDVM, 16>(A, cells, n, lds, st);
+        if (mode == MODE_FUSED_REGX)
+          return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_REGX, MARCH_CAIDVM, 16>(A, cells, n, lds, st);
+      }
     }
   }
   return launch_fr_w<D, NDF, UNI, FT, 8>(A, cells, n, mode, march, lds, st);
