@@ -316,9 +316,9 @@ int64_t kah_device_bytes(const kah_ctx* ctx);
  * the flux/relaxation kernel (2, 3, 4 or 8; default by shape: on shared grids the fewest that keep
  * the GPU occupied, on adapted grids by the size of the LDS copy of f*, up to 16 for 3D grids);
  * a change drops captured graphs. KAH_OPT_SLOPE_VPT: velocity cells per thread of the slope
- * kernel (1..6, default 3 in 2D and 6 in 3D): in the FP32 form of 3-wave or 4-wave workgroups,
- * per cell whichever pads the grid least, in the FP64 form the number its even cut of a grid
- * into 4-wave workgroups comes nearest to. KAH_OPT_VEL_TILES: 1 (default) processes a shared tensor-product velocity grid in
+ * kernel (1..6, default 3 in 2D and 6 in 3D): in the FP64 form and on shared grids the number the
+ * even cut of a grid into 4-wave workgroups comes nearest to, in the FP32 form on adapted grids
+ * that of 3-wave or 4-wave workgroups, per cell whichever pads the grid least. KAH_OPT_VEL_TILES: 1 (default) processes a shared tensor-product velocity grid in
  * 8x8 / 4x4x4 tiles per wave, 0 in storage order. KAH_OPT_OVERLAP_MAPS: 1 (default)
  * precomputes, per distinct pair of adapted velocity grids that face each other, the
  * overlapping velocity cells of the other grid (4 bytes per velocity cell of the first), 0

@@ -1350,22 +1350,25 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
   // of 13 wave passes; 1.01 against 1.11 ms per step on 22k refined leaves with 28^2 grids, 0.29
   // against 0.33 on 3D leaves with 12^3). FP32 form: slope_vpt per thread of a 3-wave or 4-wave
   // workgroup, whichever pads the grid least (a 568-cell grid fills one 3-wave chunk of 576 at 3
-  // cells per thread; ties go to 4 waves): the even cut is no faster on its adapted grids, and
-  // a thread's plain FP64 sum of slope_vpt terms is what a chunk's bits depend on, which over
-  // some hundred steps of float rounding decide the last digits of every f.
+  // cells per thread; ties go to 4 waves). On a shared grid the FP32 form takes the even cut too
+  // wherever that is not the same number of 4-wave workgroups: 22k refined leaves with 28^2 656
+  // -> 594 us per step, 64^2 with 28^2 130 -> 122, 28^2 with 20^2 52 -> 48, 3D with 12^3 235 ->
+  // 223; with the same number it was 1 % slower (36^2, 160 -> 162). On adapted grids it is no
+  // faster.
   struct Chunks {
     int waves, count;
     int64_t cells;
   };
+  const int64_t w = 64 * C->slope_vpt;
   auto chunks_of = [&](int64_t c) {
-    const int64_t n = T->vs_offset[c + 1] - T->vs_offset[c], w = 64 * C->slope_vpt;
-    if (!C->f32) {
-      const int64_t k = std::max<int64_t>(1, (2 * n + 4 * w) / (8 * w));
-      const int64_t cells = ((n + 63) / 64 + k - 1) / k * 64;
-      return Chunks{4, int((n + cells - 1) / cells), cells};
-    }
+    const int64_t n = T->vs_offset[c + 1] - T->vs_offset[c];
+    const int64_t k = std::max<int64_t>(1, (2 * n + 4 * w) / (8 * w));
+    const int64_t even = ((n + 63) / 64 + k - 1) / k * 64;
+    const Chunks cut{4, int((n + even - 1) / even), even};
+    if (!C->f32) return cut;
     auto count = [&](int64_t v) { return (n + v * w - 1) / (v * w); };
     const int64_t v = 3 * count(3) < 4 * count(4) ? 3 : 4;
+    if (C->uni && (v == 3 || count(4) != cut.count)) return cut;
     return Chunks{int(v), int(count(v)), v * w};
   };
   // Launch order of the slopes: the reference sweeps coarse to fine levels because the
