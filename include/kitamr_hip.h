@@ -121,7 +121,9 @@ typedef struct kah_topology {
   const double*  bc_prim;     /* [n_bc*(dim+2)]  prim of the boundary state            */
 
   /* Velocity root grid (Configure.quadrature / vs_trees_num), used to key the cells of
-   * adapted grids (src/Velocity_space/Neighbor.jl:9-24). */
+   * adapted grids (src/Velocity_space/Neighbor.jl:9-24). The reference has v = 0 on a root corner
+   * (check_vs_setting, src/Solver/Types.jl:335-353); on another lattice cells with neighbours on
+   * other grids do not gather from stored micro fluxes (KAH_OPT_REGULAR). */
   int32_t vs_trees_num[3];
   int32_t reserved;
   double  vs_lo[3];

@@ -1129,6 +1129,9 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
   // on the same grid then needs no overlap map (velocity cell i meets velocity cell i), and
   // cells of one grid read its geometry from the caches.
   std::vector<int64_t> gof;
+  // v = 0 inside a root cell: a velocity cell at rest there overlaps finer ones of other grids on
+  // both sides of zero, which leave their cells through opposite faces
+  bool zero_in_root = false;
   std::vector<int64_t> voff(T->vs_offset, T->vs_offset + nc + 1);
   for (int64_t h : C->ib_donor) voff.push_back(voff.back() + (T->vs_offset[h + 1] - T->vs_offset[h]));
   C->n_grids = 1;
@@ -1161,6 +1164,7 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
     };
     std::vector<int64_t> rep_of(size_t(nc), -1);   // representative cell of each cell's grid
     int64_t ndistinct = 0;
+    std::vector<uint8_t> signs;   // of the velocity components of each root's cells: 1 > 0, 2 < 0, 4 = 0
     for (int64_t c = 0; c < nc; ++c) {
       const int64_t o = T->vs_offset[c], n = T->vs_offset[c + 1] - o;
       uint64_t h = 1469598103934665603ull;
@@ -1182,6 +1186,14 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
         gw.insert(gw.end(), T->vs_weight + o, T->vs_weight + o + n);
         gl.insert(gl.end(), T->vs_level + o, T->vs_level + o + n);
         gk.insert(gk.end(), keys.begin() + o, keys.begin() + o + n);
+        for (int d = 0; d < D; ++d) {
+          const double* u = T->vs_mid + o * D + d * n;
+          for (int64_t i = 0; i < n; ++i) {
+            const size_t r = size_t(uint64_t(keys[size_t(o + i)]) >> (D * C->lmax)) * D + d;
+            if (r >= signs.size()) signs.resize(r + D, 0);
+            signs[r] |= u[i] > 0.0 ? 1 : (u[i] < 0.0 ? 2 : 4);
+          }
+        }
         ++ndistinct;
       } else {
         gof[size_t(c)] = gof[size_t(rep)];
@@ -1190,6 +1202,7 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
     }
     for (size_t k = 0; k < C->ib_donor.size(); ++k)
       gof[size_t(nc) + k] = gof[size_t(C->ib_donor[k])];
+    for (uint8_t x : signs) zero_in_root |= (x & (x - 1)) != 0;
     C->n_grids = ndistinct;
     C->grid_cells = int64_t(gw.size());
     KAH_TRY(C->upload(C->d_gu, gu.data(), gu.size(), "vs_mid"));
@@ -1527,6 +1540,10 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
     // gathers in FP64 while the slope kernel reconstructs in FP32)
     const bool caidvm = C->P.flux_kind == KAH_FLUX_CAIDVM;
     const bool same_arith = !(C->f32 && C->P.marching == KAH_MARCH_CIP);
+    // Across grids the stored fluxes serve only where no root contains both signs of a velocity
+    // component: the face a neighbour's velocity cell leaves through is then that of every cell it
+    // overlaps. Else (v = 0 inside a root: a lattice the solver's own configurations refuse) the
+    // general gather reconstructs at the neighbour's own velocities.
     // 0: not regular; 1: every neighbour on the cell's velocity grid; 2: some on other grids;
     // 3: any other cell that gathers from stored micro fluxes
     auto fr_class = [&](int32_t c) {
@@ -1544,7 +1561,10 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
             (ed.own_mode != MI_LIMITED && ed.own_mode != MI_UNLIMITED) ||
             (ed.oth_mode != MI_LIMITED && ed.oth_mode != MI_UNLIMITED))
           reg = false;
-        if (!C->uni && ed.map != MAP_SAME) cls = 2;
+        if (!C->uni && ed.map != MAP_SAME) {
+          cls = 2;
+          if (inner && zero_in_root) return 0;
+        }
       }
       return reg ? cls : (stored ? 3 : 0);
     };
