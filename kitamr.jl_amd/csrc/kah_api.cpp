@@ -311,22 +311,35 @@ namespace {
     if (_rc) return _rc;      \
   } while (0)
 
-// Key of a velocity cell (src/Velocity_space/Neighbor.jl:61-124): root lattice index times
+// Keys of velocity cells (src/Velocity_space/Neighbor.jl:61-124): root lattice index times
 // 2^(D*Lmax) plus the Morton code of the cell's lower corner inside its root.
-uint64_t cell_key(int D, int L, int lmax, const double* mid, const double* lo,
-                  const double* root_ds, const int32_t* ntree) {
-  uint64_t root_lin = 0, stride = 1, morton = 0;
-  for (int d = 0; d < D; ++d) {
-    double hf = root_ds[d] / std::ldexp(1.0, lmax);
-    double cell = hf * double(int64_t(1) << (lmax - L));
-    int64_t g = std::llround((mid[d] - 0.5 * cell - lo[d]) / hf);
-    root_lin += uint64_t(g >> lmax) * stride;
-    stride *= uint64_t(ntree[d]);
-    int64_t q = g & ((int64_t(1) << lmax) - 1);
-    for (int b = 0; b < lmax; ++b) morton |= uint64_t((q >> b) & 1) << (b * D + d);
+struct CellKeys {
+  int D, lmax;
+  double hf[3], lo[3];   // finest cell size, lower corner
+  uint64_t stride[3];
+  CellKeys(int dim, int lmax_, const double* lo_, const double* root_ds, const int32_t* ntree)
+      : D(dim), lmax(lmax_) {
+    uint64_t st = 1;
+    for (int d = 0; d < D; ++d) {
+      hf[d] = root_ds[d] / std::ldexp(1.0, lmax);
+      lo[d] = lo_[d];
+      stride[d] = st;
+      st *= uint64_t(ntree[d]);
+    }
   }
-  return (root_lin << (D * lmax)) | morton;
-}
+  uint64_t key(int L, const double* mid) const {
+    uint64_t root_lin = 0, morton = 0;
+    const double size = double(int64_t(1) << (lmax - L));
+    for (int d = 0; d < D; ++d) {
+      double cell = hf[d] * size;
+      int64_t g = std::llround((mid[d] - 0.5 * cell - lo[d]) / hf[d]);
+      root_lin += uint64_t(g >> lmax) * stride[d];
+      int64_t q = g & ((int64_t(1) << lmax) - 1);
+      for (int b = 0; b < lmax; ++b) morton |= uint64_t((q >> b) & 1) << (b * D + d);
+    }
+    return (root_lin << (D * lmax)) | morton;
+  }
+};
 
 struct Builder {
   kah_ctx& C;
@@ -335,8 +348,11 @@ struct Builder {
   int64_t nc, nrec;
   std::vector<SlopeDesc> sl;
   std::vector<SlopeNb> slnb;
-  std::vector<std::vector<HalfDesc>> hal;
-  std::vector<std::vector<EntryDesc>> ent;
+  // half fluxes and face sides of cell c: [hoff[c], hoff[c+1]) and [eoff[c], eoff[c+1]), in face-list
+  // order; counted first, then written in place
+  std::vector<int32_t> hoff, eoff;
+  std::vector<HalfDesc> halves;
+  std::vector<EntryDesc> ents;
 
   Builder(kah_ctx& c, const kah_topology& t) : C(c), T(t), D(c.D), NW(c.NW) {
     nc = t.n_cells;
@@ -485,6 +501,7 @@ struct Builder {
     e.own_mode = om;
     e.oth_mode = tm;
     e.oth_cell = oth;
+    e.map = -1;
     e.dir = int8_t(dir);
     e.bc = bc;
     e.rot = rot;
@@ -508,8 +525,7 @@ struct Builder {
   int build() {
     const bool caidvm = C.P.flux_kind == KAH_FLUX_CAIDVM;
     sl.assign(size_t(nc * D), SlopeDesc{});
-    hal.assign(size_t(nc), {});
-    ent.assign(size_t(nc), {});
+    slnb.reserve(size_t(T.nb_offset[nc * 2 * D]));
     int Lmin = 1 << 30;
     for (int64_t c = 0; c < nc; ++c)
       if (T.bound_enc[c] >= 0) Lmin = std::min(Lmin, int(T.ps_level[c]));
@@ -524,6 +540,39 @@ struct Builder {
         else KAH_TRY(plain(c, d, s));
       }
     }
+    // an IB face reads its there side from the SolidNeighbor rows (cell nc + k), whose half flux the
+    // IB kernel writes after the slopes
+    auto ib_face = [&](int64_t p) {
+      return C.ib_of_pair.empty() ? int64_t(-1) : C.ib_of_pair[size_t(p)];
+    };
+    // the counts leave out what the loop below refuses
+    hoff.assign(size_t(nc + 1), 0);
+    eoff.assign(size_t(nc + 1), 0);
+    for (int64_t p = 0; p < T.n_pairs; ++p) {
+      const int64_t h = T.pair_here[p], trec = T.pair_there[p];
+      if (h < 0 || h >= nc || trec >= nrec) continue;
+      ++eoff[size_t(h) + 1];
+      if (trec < 0) {
+        if (caidvm) hoff[size_t(h) + 1] += 2;
+        continue;
+      }
+      const int64_t t = src(trec);
+      const bool solid = T.bound_enc[t] < 0;
+      if (!solid) ++eoff[size_t(t) + 1];
+      if (!caidvm) continue;
+      ++hoff[size_t(h) + 1];
+      if (!solid) ++hoff[size_t(t) + 1];
+      else if (ib_face(p) < 0) ++hoff[size_t(h) + 1];
+    }
+    for (int64_t c = 0; c < nc; ++c) {
+      hoff[size_t(c) + 1] += hoff[size_t(c)];
+      eoff[size_t(c) + 1] += eoff[size_t(c)];
+    }
+    halves.resize(size_t(hoff[size_t(nc)]));
+    ents.resize(size_t(eoff[size_t(nc)]));
+    std::vector<int32_t> hat(hoff.begin(), hoff.end() - 1), eat(eoff.begin(), eoff.end() - 1);
+    auto add_half = [&](int64_t c, const HalfDesc& x) { halves[size_t(hat[size_t(c)]++)] = x; };
+    auto add_entry = [&](int64_t c, const EntryDesc& x) { ents[size_t(eat[size_t(c)]++)] = x; };
     for (int64_t p = 0; p < T.n_pairs; ++p) {
       int64_t h = T.pair_here[p], trec = T.pair_there[p];
       if (h < 0 || h >= nc || T.bound_enc[h] < 0)
@@ -554,17 +603,15 @@ struct Builder {
             return C.fail(KAH_EINVAL, "unknown boundary condition kind " + std::to_string(kind));
         }
         if (caidvm) {
-          hal[h].push_back(half(s0, int32_t(h), m0, 0, dir, rot, h, fm, bc));
-          hal[h].push_back(half(s1, int32_t(h), m1, 1, dir, rot, h, fm, bc));
+          add_half(h, half(s0, int32_t(h), m0, 0, dir, rot, h, fm, bc));
+          add_half(h, half(s1, int32_t(h), m1, 1, dir, rot, h, fm, bc));
         }
-        ent[h].push_back(entry(int32_t(p), 0, m0, mo, -1, dir, rot, area, fm, h, -1, bc));
+        add_entry(h, entry(int32_t(p), 0, m0, mo, -1, dir, rot, area, fm, h, -1, bc));
       } else {
         if (trec >= nrec) return C.fail(KAH_EINVAL, "pair there out of range");
         int64_t t = src(trec);
         bool solid = T.bound_enc[t] < 0;
-        // an IB face reads its there side from the SolidNeighbor rows (cell nc + k), whose
-        // half flux the IB kernel writes after the slopes
-        const int64_t ibk = C.ib_of_pair.empty() ? -1 : C.ib_of_pair[size_t(p)];
+        const int64_t ibk = ib_face(p);
         if (solid && !C.uni && ibk < 0)
           return C.fail(KAH_EUNSUPPORTED,
                         "faces with solid cells outside an immersed boundary need a shared "
@@ -572,16 +619,16 @@ struct Builder {
         int8_t mh = solid ? MI_UNLIMITED : MI_LIMITED;
         int8_t mt = solid ? (caidvm ? MI_PLAIN : MI_UNLIMITED) : MI_LIMITED;
         if (caidvm) {
-          hal[h].push_back(half(s0, int32_t(h), mh, 0, dir, rot, h, fm, -1));
+          add_half(h, half(s0, int32_t(h), mh, 0, dir, rot, h, fm, -1));
           if (solid && ibk < 0)
-            hal[h].push_back(half(s1, int32_t(t), MI_PLAIN, 1, dir, rot, trec, fm, -1));
+            add_half(h, half(s1, int32_t(t), MI_PLAIN, 1, dir, rot, trec, fm, -1));
           else if (!solid)
-            hal[t].push_back(half(s1, int32_t(t), MI_LIMITED, 1, dir, rot, trec, fm, -1));
+            add_half(t, half(s1, int32_t(t), MI_LIMITED, 1, dir, rot, trec, fm, -1));
         }
         const int32_t oth = ibk >= 0 ? int32_t(nc + ibk) : int32_t(t);
-        ent[h].push_back(entry(int32_t(p), 0, mh, mt, oth, dir, rot, area, fm, h, trec, -1));
+        add_entry(h, entry(int32_t(p), 0, mh, mt, oth, dir, rot, area, fm, h, trec, -1));
         if (!solid)
-          ent[t].push_back(entry(int32_t(p), 1, MI_LIMITED, MI_LIMITED, int32_t(h), dir, rot, area,
+          add_entry(t, entry(int32_t(p), 1, MI_LIMITED, MI_LIMITED, int32_t(h), dir, rot, area,
                                  fm, trec, h, -1));
       }
     }
@@ -1105,6 +1152,7 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
     if (rootbits + D * lmax > 32)
       return C->fail(KAH_EUNSUPPORTED, "velocity cell keys exceed 32 bits");
     keys.resize(size_t(ng));
+    const CellKeys maker(D, lmax, T->vs_lo, root_ds, T->vs_trees_num);
     for (int64_t c = 0; c < nc; ++c) {
       int64_t off = T->vs_offset[c], n = T->vs_offset[c + 1] - off;
       for (int64_t i = 0; i < n; ++i) {
@@ -1112,8 +1160,7 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
         for (int d = 0; d < D; ++d) m[d] = T->vs_mid[off * D + d * n + i];
         int L = T->vs_level[off + i];
         if (L < 0 || L > lmax) return C->fail(KAH_EINVAL, "velocity level out of range");
-        uint64_t k = cell_key(D, L, lmax, m, T->vs_lo, root_ds, T->vs_trees_num);
-        keys[size_t(off + i)] = uint32_t(k);
+        keys[size_t(off + i)] = uint32_t(maker.key(L, m));
         if (i > 0 && keys[size_t(off + i)] <= keys[size_t(off + i - 1)])
           return C->fail(KAH_EINVAL, "velocity grid of cell " + std::to_string(c) +
                                          " is not in key order");
@@ -1186,13 +1233,13 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
         gw.insert(gw.end(), T->vs_weight + o, T->vs_weight + o + n);
         gl.insert(gl.end(), T->vs_level + o, T->vs_level + o + n);
         gk.insert(gk.end(), keys.begin() + o, keys.begin() + o + n);
+        const int root = D * C->lmax;   // (the keys ascend)
+        signs.resize(std::max(signs.size(), size_t((uint64_t(keys[size_t(o + n - 1)]) >> root) + 1) * D), 0);
         for (int d = 0; d < D; ++d) {
           const double* u = T->vs_mid + o * D + d * n;
-          for (int64_t i = 0; i < n; ++i) {
-            const size_t r = size_t(uint64_t(keys[size_t(o + i)]) >> (D * C->lmax)) * D + d;
-            if (r >= signs.size()) signs.resize(r + D, 0);
-            signs[r] |= u[i] > 0.0 ? 1 : (u[i] < 0.0 ? 2 : 4);
-          }
+          for (int64_t i = 0; i < n; ++i)
+            signs[size_t(uint64_t(keys[size_t(o + i)]) >> root) * D + d] |=
+                u[i] > 0.0 ? 1 : (u[i] < 0.0 ? 2 : 4);
         }
         ++ndistinct;
       } else {
@@ -1223,6 +1270,9 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
   // descriptors
   Builder B(*C, *T);
   KAH_TRY(B.build());
+  const std::vector<int32_t>&hoff = B.hoff, &eoff = B.eoff;
+  std::vector<HalfDesc>& halves = B.halves;
+  std::vector<EntryDesc>& ents = B.ents;
 
   // Overlap maps of adapted grids: one map per distinct ordered pair (owner grid, neighbour
   // grid) that a fluid cell's slope stencil or face gather reads across grids (see OvJob); a
@@ -1250,9 +1300,8 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
       map_id.emplace(key, id);
       return id;
     };
-    for (auto& e : B.slnb) e.map = -1;
-    for (int64_t c = 0; c < nc; ++c) {
-      for (auto& ed : B.ent[c]) ed.map = -1;
+    // (a shared grid needs none)
+    for (int64_t c = 0; c < (C->uni ? 0 : nc); ++c) {
       if (T->bound_enc[c] < 0) continue;
       for (int d = 0; d < D; ++d) {
         const SlopeDesc& sd = B.sl[size_t(c * D + d)];
@@ -1263,10 +1312,12 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
             nbr.map = assign(c, nbr.cell);
           }
       }
-      for (auto& ed : B.ent[c])
+      for (int32_t e = eoff[size_t(c)]; e < eoff[size_t(c) + 1]; ++e) {
+        EntryDesc& ed = ents[size_t(e)];
         if (ed.oth_cell >= 0 &&
             (ed.oth_mode == MI_LIMITED || ed.oth_mode == MI_UNLIMITED || ed.oth_mode == MI_PLAIN))
           ed.map = assign(c, ed.oth_cell);
+      }
     }
     KAH_TRY(upload_ib(C, T->vs_offset, assign));
     C->map_entries = next;
@@ -1290,26 +1341,9 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
     }
     KAH_TRY(C->hip(hipStreamSynchronize(C->stream), "overlap maps"));
   }
-  std::vector<int32_t> hoff(size_t(nc + 1), 0), eoff(size_t(nc + 1), 0);
-  std::vector<HalfDesc> halves;
-  std::vector<EntryDesc> ents;
-  size_t n_hal = 0, n_ent = 0;
-  for (int64_t c = 0; c < nc; ++c) {
-    n_hal += B.hal[c].size();
-    n_ent += B.ent[c].size();
-  }
-  halves.reserve(n_hal);
-  ents.reserve(n_ent);
-  for (int64_t c = 0; c < nc; ++c) {
-    hoff[c] = int32_t(halves.size());
-    eoff[c] = int32_t(ents.size());
-    if (B.hal[c].size() > 24)
+  for (int64_t c = 0; c < nc; ++c)
+    if (hoff[size_t(c) + 1] - hoff[size_t(c)] > 24)
       return C->fail(KAH_EUNSUPPORTED, "cell " + std::to_string(c) + " owns more than 24 half fluxes");
-    halves.insert(halves.end(), B.hal[c].begin(), B.hal[c].end());
-    ents.insert(ents.end(), B.ent[c].begin(), B.ent[c].end());
-  }
-  hoff[nc] = int32_t(halves.size());
-  eoff[nc] = int32_t(ents.size());
   // float copies for the FP32 advection form
   for (auto& sd : B.sl)
     for (int k = 0; k < 2; ++k) {
