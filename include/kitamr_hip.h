@@ -333,10 +333,11 @@ int64_t kah_device_bytes(const kah_ctx* ctx);
  * (CAIDVM flux), cells whose 2*DIM faces go to fluid cells on the same level, which read the
  * outgoing micro fluxes the slope kernel stores instead of reconstructing; 0 runs every cell
  * through the general slope and gather. Takes effect at the next kah_set_topology.
- * KAH_OPT_BRANCHES: 1..4 (default: 4, or 1 for a phase of fewer than 786,432 velocity cells,
- * which forking would only delay) streams over which the independent launches of a phase
- * (slope launches of one projection depth, flux/relaxation launches) are spread, forked from
- * and joined back to the context's stream by events (parallel branches of a captured graph).
+ * KAH_OPT_BRANCHES: 1..4 streams over which the independent launches of a phase (slope launches
+ * of one projection depth, flux/relaxation launches) are spread, forked from and joined back to
+ * the context's stream by events (parallel branches of a captured graph). 1 to 3 hold for every
+ * phase; 4, the default, is up to four where the shape of the case makes it pay (large meshes, and
+ * adapted grids of some hundred velocity cells and up), else one.
  * No counterpart in the reference. */
 enum { KAH_OPT_FLUX_WAVES = 1, KAH_OPT_SLOPE_VPT = 2, KAH_OPT_VEL_TILES = 3,
        KAH_OPT_OVERLAP_MAPS = 4, KAH_OPT_GRAPHS = 5, KAH_OPT_REGULAR = 6,

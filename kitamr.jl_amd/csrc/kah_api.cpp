@@ -44,7 +44,6 @@ struct DBuf {
 };
 
 struct LevelBin {
-  int64_t cells = 0;   // velocity cells of its grids
   int level;
   int maxh;       // per-cell kernel: half fluxes; chunked kernel: its kind
   int waves = 4;  // chunked kernel: waves per workgroup
@@ -167,18 +166,28 @@ struct kah_ctx {
   };
   int reg_mode = 1;   // KAH_OPT_REGULAR: 0 every cell through the general slope and gather
   // KAH_OPT_BRANCHES: independent launches of one phase (the slope bins of one projection
-  // depth, the flux/relaxation bins) spread over this many streams, forked from and joined to
-  // the context's stream by events (parallel branches of the captured graph), so that small
+  // depth, the flux/relaxation bins) spread over up to this many streams, forked from and joined
+  // to the context's stream by events (parallel branches of the captured graph), so that small
   // launches run beside large ones instead of after them; 1: in order on the context's stream
   static constexpr int MAX_BRANCHES = 4;
-  int branches = 0;   // 0: not set by the caller, branches_for decides
-  // Fork and join cost some 20 us a phase, an empty step 45 us: worth it where the launches of a
-  // phase are long enough to overlap. A step of 65 k velocity cells takes 84 us on four streams
-  // and 37 us on one, of 435 k (split calls) 193 and 136; of 1.1 M on several grid sizes 241 and
-  // 283, of 2.5 M on a refined 3D mesh 290 and 325, of 151 M on the adapted cylinder 7.35 and
-  // 7.95 ms.
-  int branches_for(int64_t cells) const {
-    return branches ? branches : (cells >= 768 * 1024 ? MAX_BRANCHES : 1);
+  int branches = MAX_BRANCHES;
+  // Below MAX_BRANCHES the caller's number holds for every phase; at MAX_BRANCHES, the default, the
+  // shape decides for the whole step. Fork and join cost 8 to 20 us a phase and give back what the
+  // launches beside the longest one would have taken alone. Steps forked / in order, us:
+  // Shared grids have 10 to 30 us of irregular cells beside the bulk, so it takes a GPU that is busy
+  // for longer: 2D 0.44 M velocity cells 94 / 85, 1.4 M 137 / 127, 2.1 M 126 / 118, 2.3 M with walls
+  // 138 / 151, 3.2 M 177 / 174 and with walls 197 / 223, 11 M 776 / 779; 3D 0.70 M 125 / 122, 0.72 M
+  // 155 / 161, 2.4 M 254 / 264, 4.0 M 281 / 316.
+  // Adapted grids: a launch lasts as long as its largest grid takes, however few the cells, and the
+  // FP32 form has a launch per number of waves. 2D FP64 with grids up to 316 velocity cells 75 / 66,
+  // 520 79 / 74, 594 113 / 120, 811 341 / 361, 1651 107 / 120; FP32 form 316 76 / 74, 403 86 / 89,
+  // 520 87 / 90, 594 127 / 157; 3D 552 96 / 116, 1247 133 / 176 and in the FP32 form 154 / 272. Large
+  // meshes of small grids: 1.1 M 167 / 161, 1.6 M 182 / 197, 1.9 M 291 / 284, 2.1 M 151 / 164.
+  int step_branches() const {
+    if (branches < MAX_BRANCHES) return branches;
+    const bool large = phase_cells >= (D == 2 ? 2000 : 768) * int64_t(1024);
+    const bool grids = !uni && max_n >= (D == 3 ? 512 : f32 ? 384 : 768);
+    return large || grids ? MAX_BRANCHES : 1;
   }
   hipStream_t side[MAX_BRANCHES - 1] = {};
   std::vector<hipEvent_t> ev_pool;   // fork/join events, reused step after step
@@ -931,7 +940,6 @@ int slope_bins(kah_ctx* C, const SlopeTables& t, const std::vector<char>& walled
         lb->maxh = kind;
         lb->waves = w;
         lb->n = int(it->second.size());
-        for (const int4& w4 : it->second) lb->cells += w4.w - w4.z;
         lb->chunked = true;
         KAH_TRY(C->upload(lb->items, it->second.data(), it->second.size(), "slope work items"));
       }
@@ -941,7 +949,6 @@ int slope_bins(kah_ctx* C, const SlopeTables& t, const std::vector<char>& walled
       lb->level = L;
       lb->maxh = kv.first;
       lb->n = int(kv.second.size());
-      for (int32_t c : kv.second) lb->cells += (*t.voff)[size_t(c) + 1] - (*t.voff)[size_t(c)];
       lb->chunked = false;
       KAH_TRY(C->upload(lb->items, kv.second.data(), kv.second.size(), "level cells"));
     }
@@ -1773,9 +1780,7 @@ int run_slope(kah_ctx* C, const DevArgs& A) {
   for (size_t b0 = 0; b0 < C->bins.size();) {
     size_t b1 = b0;
     while (b1 < C->bins.size() && C->bins[b1]->level == C->bins[b0]->level) ++b1;
-    int64_t cells = 0;
-    for (size_t j = b0; j < b1; ++j) cells += C->bins[j]->cells;
-    const int nb = std::min<int>(C->branches_for(cells), int(b1 - b0));
+    const int nb = std::min<int>(C->step_branches(), int(b1 - b0));
     KAH_TRY(fork_branches(C, nb));
     for (size_t j = b0; j < b1; ++j) {
       const LevelBin* b = C->bins[j];
@@ -1836,7 +1841,7 @@ int run_flux_relax(kah_ctx* C, const DevArgs& A, int mode) {
                                    C->stream),
                    "cell prologue launch"));
   // the bins write disjoint cells and read only what the slope phase wrote
-  const int nb = std::min<int>(C->branches_for(C->phase_cells), int(C->frbins.size()));
+  const int nb = std::min<int>(C->step_branches(), int(C->frbins.size()));
   KAH_TRY(fork_branches(C, nb));
   for (size_t j = 0; j < C->frbins.size(); ++j) {
     const kah_ctx::FrBin* b = C->frbins[j];

@@ -24,7 +24,7 @@ SPACE = {
     "flux_waves": [0, 8, 4, 2],      # 0: the library's choice by shape
     "vel_tiles": [1, 0],
     "overlap_maps": [1, 0],
-    "branches": [4, 1, 2],           # streams for the independent launches of a phase
+    "branches": [4, 1, 2],           # streams of a phase's independent launches; 4: by shape
 }
 
 
