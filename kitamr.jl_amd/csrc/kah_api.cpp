@@ -1053,6 +1053,7 @@ const char* kah_last_error(const kah_ctx* ctx) {
 int kah_set_topology(kah_ctx* C, const kah_topology* T) {
   if (!C) return KAH_EINVAL;
   C->drop_graphs();   // captured launches refer to the buffers replaced below
+  C->d_xbuf.release();   // sized for the grids replaced below (a byte per velocity cell for the flags)
   if (!T) return C->fail(KAH_EINVAL, "null topology");
   KAH_TRY(C->hip(hipSetDevice(C->P.device), "hipSetDevice"));
   C->have_topo = C->have_state = false;

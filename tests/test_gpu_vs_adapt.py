@@ -277,3 +277,27 @@ def test_flags_key_copy_edges(name):
     assert np.array_equal(dev.vs_flags(p, vr), orc.vs_flags(p, vr))
     dev.close()
     orc.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("remap", [False, True])
+def test_flags_staging_does_not_outlive_the_grids(remap):
+    """The staging memory of the criteria (a byte per velocity cell) is given back when the grids are
+    replaced, so that a remap has as much room as without the flags."""
+    case = cases.riemann_2d(n=6, nv=12, vs_levels=1)
+    say(f"[vs] staging remap={remap}")
+    held = []
+    for flags in (False, True):
+        dev, orc = pair(case)
+        orc.close()
+        if flags:
+            dev.vs_flags(abi.vs_adapt_params("lohner"), dev.vs_resolution())
+        if remap:   # onto the same grids
+            sizes = np.diff(np.asarray(case.topo["vs_offset"]))
+            src = np.concatenate([np.arange(n) for n in sizes]).astype(np.int32)
+            dev.vs_remap(case.topo, src, np.zeros(len(sizes), dtype=np.uint8))
+        else:
+            dev.set_topology(case.topo)
+        held.append(dev.device_bytes())
+        dev.close()
+    assert held[0] == held[1]
