@@ -45,3 +45,43 @@ def test_waves_by_shape(name, precision):
         assert rel_err_rows(g["w"].reshape(-1, nw), other["w"].reshape(-1, nw), nw) <= tol
     for k in ("w", "prim", "qf", "df"):
         assert np.array_equal(g[k], r[k]), k
+
+
+# 16-wave workgroups in the FP64 form with the copy of f* in LDS: 2D cells with neighbours on other
+# levels or at the domain's edge whose grids lie above 640 velocity cells (and below the 6,485 that
+# fit 152 KiB), 3D grids whose copy takes more than 56 KiB and fits (3,585 to 9,728).
+WIDE = {
+    "2d": (lambda: cases.riemann_2d(n=6, nv=16, vs_levels=2), 641, 6485),
+    "2d-hanging": (lambda: cases.riemann_2d(n=6, nv=16, ps_levels=1, vs_levels=2, vs_variants=5),
+                   641, 6485),
+    "3d": (lambda: cases.box_3d(n=3, nv=14, vs_levels=1), 3585, 9728),
+}
+
+
+@pytest.mark.parametrize("name", list(WIDE))
+def test_wide_shapes(name):
+    make, lo, hi = WIDE[name]
+    sizes = np.diff(np.asarray(make().topo["vs_offset"]))
+    assert lo <= sizes.min() and sizes.max() <= hi, (sizes.min(), sizes.max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(WIDE))
+def test_wide_workgroups(name):
+    case = WIDE[name][0]()
+    say(f"[flux waves] wide {name}: cells={case.n_cells} P={case.phase_cells}")
+    dev, orc = pair(case)
+    eight, _ = pair(case, options={"flux_waves": 8})
+    general, _ = pair(case, options={"regular": 0})
+    for s in range(2):
+        for d in (dev, eight, general, orc):
+            d.step(case.dt_xi, s)
+    g, e, r, o = dev.get_state(), eight.get_state(), general.get_state(), orc.get_state()
+    for d in (dev, eight, general):
+        d.close()
+    nw = case.config.solver.DIM + 2
+    for other in (o, e):   # sums of a few thousand terms in another order, as above
+        assert rel_err(g["df"], other["df"]) <= 1e-12
+        assert rel_err_rows(g["w"].reshape(-1, nw), other["w"].reshape(-1, nw), nw) <= 1e-12
+    for k in ("w", "prim", "qf", "df"):
+        assert np.array_equal(g[k], r[k]), k

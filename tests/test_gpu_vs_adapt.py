@@ -301,3 +301,12 @@ def test_flags_staging_does_not_outlive_the_grids(remap):
         held.append(dev.device_bytes())
         dev.close()
     assert held[0] == held[1]
+
+
+@pytest.mark.parametrize("dim,nv,vs,below", [(2, 44, 2, True), (2, 46, 2, False), (3, 16, 1, False)])
+def test_key_copy_shapes(dim, nv, vs, below):
+    """The meshes of test_flags_key_copy_edges lie on their side of the 8,192 keys."""
+    case = (cases.riemann_2d(n=4, nv=nv, vs_levels=vs) if dim == 2 else
+            cases.box_3d(n=2, nv=nv, vs_levels=vs))
+    sizes = np.diff(np.asarray(case.topo["vs_offset"]))
+    assert (sizes.max() <= 8192) if below else (sizes.min() > 8192), (sizes.min(), sizes.max())

@@ -80,3 +80,17 @@ def test_per_step_kernels_use_no_scratch_memory():
     walled = [k for k in res if "7k_slopeI" in k and res[k].get("ScratchSize", 0) > 0]
     for k in walled:
         assert re.search(r"Li(16|24)ELi4EEEv", k), k
+
+
+def test_immersed_boundary_sums_use_no_scratch_memory():
+    """The same for the immersed-boundary kernels of the wall density and of the sums over a grid."""
+    import json
+    from kitamr_hip import build as B
+    if not B.RESOURCES.exists():
+        pytest.skip("library built without the resource report")
+    res = json.loads(B.RESOURCES.read_text())
+    for name in ("k_ib_rho", "k_ib_wall", "k_ib_sum"):
+        hot = [k for k in res if name in k]
+        assert hot, name
+        spilled = sorted(k for k in hot if res[k].get("ScratchSize", 0) > 0)
+        assert not spilled, spilled
