@@ -48,12 +48,12 @@ def test_waves_by_shape(name, precision):
 
 
 # 16-wave workgroups in the FP64 form with the copy of f* in LDS: 2D cells with neighbours on other
-# levels or at the domain's edge whose grids lie above 640 velocity cells (and below the 6,485 that
+# levels or at the domain's edge whose grids lie above 2,048 velocity cells (and below the 6,485 that
 # fit 152 KiB), 3D grids whose copy takes more than 56 KiB and fits (3,585 to 9,728).
 WIDE = {
-    "2d": (lambda: cases.riemann_2d(n=6, nv=16, vs_levels=2), 641, 6485),
-    "2d-hanging": (lambda: cases.riemann_2d(n=6, nv=16, ps_levels=1, vs_levels=2, vs_variants=5),
-                   641, 6485),
+    "2d": (lambda: cases.riemann_2d(n=6, nv=26, vs_levels=2), 2049, 6485),
+    "2d-hanging": (lambda: cases.riemann_2d(n=5, nv=26, ps_levels=1, vs_levels=2, vs_variants=5),
+                   2049, 6485),
     "3d": (lambda: cases.box_3d(n=3, nv=14, vs_levels=1), 3585, 9728),
 }
 
