@@ -316,7 +316,6 @@ struct Grid {
   const FT* fb;
   const FT* sb;
   FT* swb;
-  FT* ofb;
   FT* ob;
   const double* gub;
   const double* gwb;
@@ -333,7 +332,6 @@ struct Grid {
     fb = reinterpret_cast<const FT*>(a.df) + off * NDF;
     sb = reinterpret_cast<const FT*>(a.sdf_r) + off * NDF * D;
     swb = reinterpret_cast<FT*>(a.sdf) + off * NDF * D;
-    ofb = reinterpret_cast<FT*>(a.oflux) + off * NDF * D;
     ob = reinterpret_cast<FT*>(a.df_out) + off * NDF;
     gub = a.gu + goff() * D;
     gwb = a.gw + goff();
@@ -377,10 +375,6 @@ struct Grid {
   // accessors widen to double, and the FP32 form's arithmetic narrows where it advects
   __device__ double f(int i, int k) const { return double(at(fb, k * n + i)); }
   __device__ double s(int i, int k, int d) const { return double(at(sb, (d * NDF + k) * n + i)); }
-  // the outgoing micro flux of velocity cell i through the cell's face in direction d
-  __device__ void set_of(int i, int k, int d, double v) const {
-    at(ofb, (d * NDF + k) * n + i) = FT(v);
-  }
   __device__ void set_s(int i, int k, int d, double v) const {
     at(swb, (d * NDF + k) * n + i) = FT(v);
   }
@@ -638,9 +632,9 @@ __device__ inline T div_ds(T a, double ds, double rds, float rds_f) {
 }
 
 template <int D, int NDF, bool UNI, class FT, class T>
-__device__ inline void side_sum(const DevArgs& A, int c, int n_own, int beg, int cnt,
-                                double dsx, double rdsx, float rdsx_f, int i, int li,
-                                const uint32_t* kp, const T (&f)[NDF], T (&a)[NDF]) {
+__device__ inline void side_sum(const DevArgs& A, int beg, int cnt, double dsx, double rdsx,
+                                float rdsx_f, int i, int li, const uint32_t* kp, const T (&f)[NDF],
+                                T (&a)[NDF]) {
   using GR = Grid<D, NDF, UNI, FT>;
 #pragma unroll
   for (int k = 0; k < NDF; ++k) a[k] = T(0);
@@ -689,12 +683,12 @@ __device__ inline void slope_dir(const DevArgs& A, const Grid<D, NDF, UNI, FT>& 
     return;
   }
   T aL[NDF];
-  side_sum<D, NDF, UNI, FT, T>(A, c, G.n, sd.nb_beg[0], sd.nb_cnt[0], sd.ds[0], sd.rds[0],
+  side_sum<D, NDF, UNI, FT, T>(A, sd.nb_beg[0], sd.nb_cnt[0], sd.ds[0], sd.rds[0],
                                sd.rds_f[0], i, li, kp, f, aL);
   const T ic0 = desc_val<T>(sd.inv_cnt[0], sd.inv_cnt_f[0]);
   if (sd.mode == SL_INNER) {
     T aR[NDF];
-    side_sum<D, NDF, UNI, FT, T>(A, c, G.n, sd.nb_beg[1], sd.nb_cnt[1], sd.ds[1], sd.rds[1],
+    side_sum<D, NDF, UNI, FT, T>(A, sd.nb_beg[1], sd.nb_cnt[1], sd.ds[1], sd.rds[1],
                                  sd.rds_f[1], i, li, kp, f, aR);
     const T ic1 = desc_val<T>(sd.inv_cnt[1], sd.inv_cnt_f[1]);
 #pragma unroll
@@ -1090,7 +1084,7 @@ __global__ __launch_bounds__(NWV * 64) void k_slope_chunk_reg(DevArgs A0,
 // Micro flux into velocity cell i of cell c through all its faces, in face-list order
 // (update_flux!/update_domain_flux!/update_micro_flux!, src/Flux/Flux.jl:64-281).
 template <int D, int NDF, bool UNI, class FT, class T>
-__device__ inline void gather_flux(const DevArgs& A, int c, int n_own, int eb, int ne, int i,
+__device__ inline void gather_flux(const DevArgs& A, int eb, int ne, int i,
                                    const T (&u)[D], const T (&f)[NDF], const T (&s)[D][NDF],
                                    int li, const uint32_t* kp, T (&fl)[NDF]) {
   const T dt = T(A.dt);
@@ -1896,7 +1890,7 @@ __global__ __launch_bounds__(NWV * 64) void k_flux_relax(DevArgs A0,
         for (int d = 0; d < D; ++d) s[d][k] = CT(G.s(i, k, d));
         fl[k] = CT(A.vflux[G.off * NDF + int64_t(k) * n + i]);
       }
-      gather_flux<D, NDF, UNI, FT, CT>(A, c, n, eb, ne, i, u, f, s, G.lev(i), G.keyp(i), fl);
+      gather_flux<D, NDF, UNI, FT, CT>(A, eb, ne, i, u, f, s, G.lev(i), G.keyp(i), fl);
 #pragma unroll
       for (int k = 0; k < NDF; ++k) A.vflux[G.off * NDF + int64_t(k) * n + i] = fl[k];
     }
@@ -2002,7 +1996,7 @@ __global__ __launch_bounds__(NWV * 64) void k_flux_relax(DevArgs A0,
 #pragma unroll
           for (int d = 0; d < D; ++d) s[d][k] = CT(G.s(i, k, d));
         }
-        gather_flux<D, NDF, UNI, FT, CT>(A, c, n, eb, ne, i, u, f, s, G.lev(i), G.keyp(i), fl);
+        gather_flux<D, NDF, UNI, FT, CT>(A, eb, ne, i, u, f, s, G.lev(i), G.keyp(i), fl);
       } else {
 #pragma unroll
         for (int k = 0; k < NDF; ++k) {
@@ -2759,11 +2753,10 @@ template <int D, int NDF, bool UNI, class FT>
 inline hipError_t launch_slope_chunk_t(const DevArgs& A, const void* recs, const int4* work, int n,
                                        int kind, int waves, hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  switch (waves) {
-    case 3: return launch_slope_chunk_w<D, NDF, UNI, FT, 3>(A, recs, work, n, kind, st);
-    case 4: return launch_slope_chunk_w<D, NDF, UNI, FT, 4>(A, recs, work, n, kind, st);
-    default: return hipErrorInvalidValue;
-  }
+  if constexpr (!UNI && sizeof(FT) == 4)   // 3 waves: adapted grids of the FP32 form
+    if (waves == 3) return launch_slope_chunk_w<D, NDF, UNI, FT, 3>(A, recs, work, n, kind, st);
+  if (waves != 4) return hipErrorInvalidValue;
+  return launch_slope_chunk_w<D, NDF, UNI, FT, 4>(A, recs, work, n, kind, st);
 }
 
 template <int D, int NDF, bool UNI, class FT, int MODE, int MARCH, int NWV>
@@ -2781,46 +2774,36 @@ inline hipError_t launch_fr_t(const DevArgs& A, const int32_t* cells, int n, siz
   return hipGetLastError();
 }
 
+template <int D, int NDF, bool UNI, class FT, int MODE, int NWV>
+inline hipError_t launch_fr_m(const DevArgs& A, const int32_t* cells, int n, int march, size_t lds,
+                              hipStream_t st) {
+  // CIP_Marching of the FP32 form gathers in FP64, never from fluxes stored in FP32
+  constexpr bool stored = MODE != MODE_FUSED && MODE != MODE_ITER;
+  if (march == MARCH_CAIDVM)
+    return launch_fr_t<D, NDF, UNI, FT, MODE, MARCH_CAIDVM, NWV>(A, cells, n, lds, st);
+  if (march == MARCH_EULER)
+    return launch_fr_t<D, NDF, UNI, FT, MODE, MARCH_EULER, NWV>(A, cells, n, lds, st);
+  if constexpr (!stored || sizeof(FT) == 8)
+    return launch_fr_t<D, NDF, UNI, FT, MODE, MARCH_CIP, NWV>(A, cells, n, lds, st);
+  else
+    return hipErrorInvalidValue;
+}
+
 template <int D, int NDF, bool UNI, class FT, int NWV>
 inline hipError_t launch_fr_w(const DevArgs& A, const int32_t* cells, int n, int mode,
                               int march, size_t lds, hipStream_t st) {
   if (mode == MODE_FLUX)
     return launch_fr_t<D, NDF, UNI, FT, MODE_FLUX, MARCH_CAIDVM, NWV>(A, cells, n, 0, st);
-  if (mode == MODE_ITER) {
-    if (march == MARCH_CAIDVM)
-      return launch_fr_t<D, NDF, UNI, FT, MODE_ITER, MARCH_CAIDVM, NWV>(A, cells, n, lds, st);
-    if (march == MARCH_CIP)
-      return launch_fr_t<D, NDF, UNI, FT, MODE_ITER, MARCH_CIP, NWV>(A, cells, n, lds, st);
-    return launch_fr_t<D, NDF, UNI, FT, MODE_ITER, MARCH_EULER, NWV>(A, cells, n, lds, st);
-  }
-  if (mode == MODE_FUSED_REG) {
-    if (march == MARCH_CAIDVM)
-      return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_REG, MARCH_CAIDVM, NWV>(A, cells, n, lds, st);
-    if (march == MARCH_CIP)
-      return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_REG, MARCH_CIP, NWV>(A, cells, n, lds, st);
-    return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_REG, MARCH_EULER, NWV>(A, cells, n, lds, st);
-  }
-  if (mode == MODE_FUSED_ST) {
-    if (march == MARCH_CAIDVM)
-      return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_ST, MARCH_CAIDVM, NWV>(A, cells, n, lds, st);
-    if (march == MARCH_CIP)
-      return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_ST, MARCH_CIP, NWV>(A, cells, n, lds, st);
-    return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_ST, MARCH_EULER, NWV>(A, cells, n, lds, st);
-  }
-  if constexpr (!UNI) {   // on a shared grid every neighbour is on the cell's grid
-    if (mode == MODE_FUSED_REGX) {
-      if (march == MARCH_CAIDVM)
-        return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_REGX, MARCH_CAIDVM, NWV>(A, cells, n, lds, st);
-      if (march == MARCH_CIP)
-        return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_REGX, MARCH_CIP, NWV>(A, cells, n, lds, st);
-      return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED_REGX, MARCH_EULER, NWV>(A, cells, n, lds, st);
-    }
-  }
-  if (march == MARCH_CAIDVM)
-    return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED, MARCH_CAIDVM, NWV>(A, cells, n, lds, st);
-  if (march == MARCH_CIP)
-    return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED, MARCH_CIP, NWV>(A, cells, n, lds, st);
-  return launch_fr_t<D, NDF, UNI, FT, MODE_FUSED, MARCH_EULER, NWV>(A, cells, n, lds, st);
+  if (mode == MODE_ITER)
+    return launch_fr_m<D, NDF, UNI, FT, MODE_ITER, NWV>(A, cells, n, march, lds, st);
+  if (mode == MODE_FUSED_REG)
+    return launch_fr_m<D, NDF, UNI, FT, MODE_FUSED_REG, NWV>(A, cells, n, march, lds, st);
+  if (mode == MODE_FUSED_ST)
+    return launch_fr_m<D, NDF, UNI, FT, MODE_FUSED_ST, NWV>(A, cells, n, march, lds, st);
+  if constexpr (!UNI)   // on a shared grid every neighbour is on the cell's grid
+    if (mode == MODE_FUSED_REGX)
+      return launch_fr_m<D, NDF, UNI, FT, MODE_FUSED_REGX, NWV>(A, cells, n, march, lds, st);
+  return launch_fr_m<D, NDF, UNI, FT, MODE_FUSED, NWV>(A, cells, n, march, lds, st);
 }
 
 template <int D, int NDF, bool UNI, class FT>
