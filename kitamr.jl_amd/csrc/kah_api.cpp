@@ -73,6 +73,7 @@ struct kah_ctx {
   int max_n = 0;
   size_t lds_bytes = 0;
   size_t lds_limit = 56 * 1024;   // dynamic LDS per workgroup (set from the device)
+  int64_t lds_cu = 160 * 1024, cus = 256;   // LDS of a CU, CUs of the device (the same)
   int64_t phase_cells = 0;
   std::vector<int32_t> fluid;
   std::vector<int32_t> benc;
@@ -116,10 +117,11 @@ struct kah_ctx {
   // Shared grids: the fewest waves that keep 20 of a CU's 32 resident (12 for irregular cells),
   // else the number that keeps most. Steps against 8 waves: 64^2 leaves with 16^2, 28^2 and 40^2
   // velocity cells 113 -> 98, 189 -> 175 and 443 -> 442 us (3, 3 and 8 waves), 32^2 refined
-  // leaves with 28^2 996 -> 890, FP32 form 145 -> 130, a 3D box with 12^3 287 -> 282. The Newton
-  // iteration of CIP_Marching is mostly reductions: half the residency does, 40^2 leaves with
-  // 24^2 130 -> 98 us on 2 waves, 40^2 with 40^2 190 -> 188 on 4; 144 cells stay on 8 (63 against
-  // 74 us on 2).
+  // leaves with 28^2 996 -> 890, FP32 form 145 -> 130, a 3D box with 12^3 287 -> 282. 2 waves are
+  // not offered (64^2 leaves with 24^2 136 us against 131 on 3, with 28^2 182 against 178; with 16^2
+  // 82 against 85). The Newton iteration of CIP_Marching is mostly reductions: half the residency
+  // does, and 2 waves come before 3 (64^2 leaves with 16^2 111 us on 2, 125 on 3, 177 on 8; with 28^2
+  // 199, 206, 253), so 3 is not offered there; 40^2 with 36^2 136 us on 4, 151 on 8.
   // Adapted grids: several size classes run side by side. 2D FP32 form: 2 waves for the smallest
   // class (8 KiB), 4 while four or more workgroups fit, else 8. 3D: 16 waves where the LDS copy
   // leaves one or two workgroups per CU or is in global memory (few, long workgroups that the
@@ -142,15 +144,15 @@ struct kah_ctx {
       }
       if (P.marching != KAH_MARCH_CAIDVM) return 8;
       if (D == 3) return lds == 0 || lds > 56 * 1024 ? 16 : 8;
-      return !f32 && irregular && cells < 1024 && n > 640 && max_n > 2048 ? 16 : 8;
+      return !f32 && irregular && cells < 4 * cus && n > 640 && max_n > 2048 ? 16 : 8;
     }
-    const int64_t by_lds = lds ? std::max<int64_t>(1, (160 * 1024) / int64_t(lds + 1536)) : 32;
+    const int64_t by_lds = lds ? std::max<int64_t>(1, lds_cu / int64_t(lds + 1536)) : 32;
     const int regs = irregular ? 16 : 28, want = irregular || cip ? 12 : 20;
     int at = 8;
     int64_t most = 0;
     for (int w : {2, 3, 4, 8}) {
       if (w == (cip ? 3 : 2)) continue;
-      const int64_t r = std::min({by_lds * w, int64_t(regs / w * w), cells * w / 256});
+      const int64_t r = std::min({by_lds * w, int64_t(regs / w * w), cells * w / cus});
       if (r >= want) return w;
       if (r > most) {
         most = r;
@@ -1036,8 +1038,14 @@ int kah_create(const kah_params* params, kah_ctx** out) {
   // static LDS
   int lds_max = 0;
   if (hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock,
-                            params->device) == hipSuccess && lds_max > 16 * 1024)
+                            params->device) == hipSuccess && lds_max > 16 * 1024) {
     C->lds_limit = size_t(lds_max) - 8 * 1024;
+    C->lds_cu = lds_max;
+  }
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, params->device) ==
+          hipSuccess && cus > 0)
+    C->cus = cus;
   *out = C;
   return KAH_OK;
 }
@@ -1409,16 +1417,15 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
       return C->fail(KAH_EUNSUPPORTED, "cell " + std::to_string(c) + " has more than " +
                                            std::to_string(MAX_ENTRIES) + " face sides");
   // Chunks of the slope kernel, by grid size alone (alike for regular and general cells, whose
-  // sums so run in the same order). FP64 form: 4-wave workgroups, as many chunks as come nearest
-  // to slope_vpt velocity cells per thread, cut evenly at multiples of 64 (784 cells: one chunk
-  // of 13 wave passes; 1.01 against 1.11 ms per step on 22k refined leaves with 28^2 grids, 0.29
-  // against 0.33 on 3D leaves with 12^3). FP32 form: slope_vpt per thread of a 3-wave or 4-wave
-  // workgroup, whichever pads the grid least (a 568-cell grid fills one 3-wave chunk of 576 at 3
-  // cells per thread; ties go to 4 waves). On a shared grid the FP32 form takes the even cut too
-  // wherever that is not the same number of 4-wave workgroups: 22k refined leaves with 28^2 656
-  // -> 594 us per step, 64^2 with 28^2 130 -> 122, 28^2 with 20^2 52 -> 48, 3D with 12^3 235 ->
-  // 223; with the same number it was 1 % slower (36^2, 160 -> 162). On adapted grids it is no
-  // faster.
+  // sums so run in the same order). FP64 form and shared grids: 4-wave workgroups, as many chunks as
+  // come nearest to slope_vpt velocity cells per thread, cut evenly at multiples of 64 (784 cells:
+  // one chunk of 13 wave passes; 1.01 against 1.11 ms per step on 22k refined leaves with 28^2 grids,
+  // 0.29 against 0.33 on 3D leaves with 12^3; FP32 form 656 -> 594 us on the refined leaves, 64^2 with
+  // 28^2 130 -> 122, 40^2 with 34^2 93 -> 90, with 36^2 100 and 100). FP32 form on adapted grids,
+  // where the even cut is no faster: slope_vpt per thread of a 3-wave or 4-wave workgroup, whichever
+  // pads the grid least (a 568-cell grid fills one 3-wave chunk of 576 at 3 cells per thread; ties
+  // go to 4 waves). A thread so adds up to about 1.5 slope_vpt terms of a half flux before the
+  // compensated sum over the workgroup.
   struct Chunks {
     int waves, count;
     int64_t cells;
@@ -1428,11 +1435,9 @@ int kah_set_topology(kah_ctx* C, const kah_topology* T) {
     const int64_t n = T->vs_offset[c + 1] - T->vs_offset[c];
     const int64_t k = std::max<int64_t>(1, (2 * n + 4 * w) / (8 * w));
     const int64_t even = ((n + 63) / 64 + k - 1) / k * 64;
-    const Chunks cut{4, int((n + even - 1) / even), even};
-    if (!C->f32) return cut;
+    if (!C->f32 || C->uni) return Chunks{4, int((n + even - 1) / even), even};
     auto count = [&](int64_t v) { return (n + v * w - 1) / (v * w); };
     const int64_t v = 3 * count(3) < 4 * count(4) ? 3 : 4;
-    if (C->uni && (v == 3 || count(4) != cut.count)) return cut;
     return Chunks{int(v), int(count(v)), v * w};
   };
   // Launch order of the slopes: the reference sweeps coarse to fine levels because the
