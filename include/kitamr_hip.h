@@ -315,8 +315,9 @@ int64_t kah_phase_cells(const kah_ctx* ctx);
 /* Device bytes held by the context (state + topology). */
 int64_t kah_device_bytes(const kah_ctx* ctx);
 /* Launch options (autotuned schedule choices). KAH_OPT_FLUX_WAVES: waves per workgroup of
- * the flux/relaxation kernel (2, 3, 4 or 8; default by shape: on shared grids the fewest that keep
- * the GPU occupied, on adapted grids by the size of the LDS copy of f*, up to 16 for 3D grids);
+ * the flux/relaxation kernel (2, 3, 4 or 8; 0, the default, by shape: on shared grids the fewest
+ * that keep the GPU occupied, on adapted grids by the size of the LDS copy of f*, up to 16 for 3D
+ * grids and for few irregular cells of the 2D FP64 form);
  * a change drops captured graphs. KAH_OPT_SLOPE_VPT: velocity cells per thread of the slope
  * kernel (1..6, default 3 in 2D and 6 in 3D): in the FP64 form and on shared grids the number the
  * even cut of a grid into 4-wave workgroups comes nearest to, in the FP32 form on adapted grids

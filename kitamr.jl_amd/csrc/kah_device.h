@@ -1713,8 +1713,8 @@ __device__ inline double cell_update(const DevArgs& A, int c, int eb, int ne, bo
 // half fluxes, one thread per component adds the faces in order, one per cell does the rest, and
 // the face records hold their rows, which takes a lookup out of the chain. One thread per cell
 // walked faces, sides and rows one after the other: 23 us against 10 on 64^2 leaves, 53 against
-// 15 on 2k refined 3D leaves, 240 against 25 on a 14^3 sphere (whose wall faces have up to 118
-// rows).
+// 15 on 2k refined 3D leaves, 240 against 25 on a 14^3 sphere (whose wall faces then had a row per
+// chunk, up to 118; they have one).
 template <int D>
 __global__ __launch_bounds__(256) void k_cell_pre(DevArgs A, const int32_t* __restrict__ cells,
                                                   int ncells) {

@@ -31,8 +31,9 @@ struct DevArgs {
   double* df_out;           // f of the next step
   double* sdf;
   // outgoing micro flux of every velocity cell per direction, written by K1 for the face of
-  // the cell's outgoing side (the cell's own reconstruction times u[dir]); the gather of
-  // regular cells reads it instead of reconstructing (layout of sdf, storage type of f)
+  // the cell's outgoing side (the cell's own reconstruction times u[dir]); the stored gathers
+  // read it instead of reconstructing. Layout of sdf, storage type of f; after the cells' rows
+  // a block [NDF][n] for each face side that shares its side of the cell (HalfDesc.ofb)
   double* oflux;
   double* vflux;            // VsData.flux accumulators (split flux/iterate calls)
   double* psflux;           // PsData.flux accumulators
