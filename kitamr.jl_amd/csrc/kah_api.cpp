@@ -383,26 +383,30 @@ struct Builder {
   }
   int64_t nb(int64_t c, int f, int64_t j) const { return T.nb_cell[T.nb_offset[c * 2 * D + f] + j]; }
 
-  // proj: with the neighbours' transverse slopes, where the neighbours are offset at all
+  // A midpoint x of a neighbour is offset from cell c along t: by half the cell's size for a coarser
+  // neighbour, a quarter for a finer one. Midpoints on one level may differ in the last bits (a size
+  // of the mesh that is no power of two); that is no offset, and a projection over 10^-17 would read
+  // slopes that the same launch writes.
+  bool apart(int64_t c, int t, double x) const {
+    return std::fabs(x - mid(c)[t]) > 0.125 * dsr(c)[t];
+  }
+  // proj: with the transverse slopes of the neighbours that are offset
   void add_side(SlopeDesc& s, int side, int64_t c, int f, int dir, bool proj) {
-    proj = proj && offset(c, f, dir);
     s.nb_beg[side] = int32_t(slnb.size());
     s.nb_cnt[side] = int32_t(nbn(c, f));
     for (int64_t j = 0; j < nbn(c, f); ++j) {
       SlopeNb e{};
       e.cell = int32_t(nb(c, f, j));
-      e.proj = proj ? 1 : 0;
       e.map = -1;
-      for (int t = 0; t < 3; ++t) e.dm[t] = 0.0;
-      if (proj)
-        for (int t = 0; t < D; ++t) e.dm[t] = (t == dir) ? 0.0 : (mid(c)[t] - mid(e.cell)[t]);
+      for (int t = 0; proj && t < D; ++t)
+        if (t != dir && apart(c, t, mid(e.cell)[t])) {
+          e.proj = 1;
+          e.dm[t] = mid(c)[t] - mid(e.cell)[t];
+        }
       slnb.push_back(e);
     }
   }
-  // _ps_has_transverse_offset, src/Flux/Slope.jl:177-199, up to rounding: a coarser neighbour is
-  // offset by half the cell's size, a neighbour on the level or the mean of finer ones not at all.
-  // Their midpoints may differ in the last bits (a size of the mesh that is no power of two), and
-  // a projection over 10^-17 would read slopes that the same launch writes.
+  // _ps_has_transverse_offset, src/Flux/Slope.jl:177-199, up to rounding
   bool offset(int64_t c, int f, int dir) const {
     int64_t n = nbn(c, f);
     if (n == 0) return false;
@@ -411,7 +415,7 @@ struct Builder {
       double avg = 0.0;
       for (int64_t j = 0; j < n; ++j) avg += mid(nb(c, f, j))[t];
       avg /= double(n);
-      if (std::fabs(avg - mid(c)[t]) > 0.125 * dsr(c)[t]) return true;
+      if (apart(c, t, avg)) return true;
     }
     return false;
   }
@@ -479,7 +483,7 @@ struct Builder {
       double dsL = xm - mid(L0)[dir], dsR = xm - mid(R0)[dir];
       if (benc(L0) < 0) bound(s, c, fR, dir, dsR, true);
       else if (benc(R0) < 0) bound(s, c, fL, dir, dsL, true);
-      else inner(s, c, dir, dsL, dsR, true, true);
+      else inner(s, c, dir, dsL, dsR, offset(c, fL, dir), offset(c, fR, dir));
     } else if (sR == 0 && sL == -1) {
       int64_t L0 = nb(c, fL, 0);
       if (benc(L0) < 0) s.mode = SL_SKIP;

@@ -5,8 +5,10 @@ Against the oracle, which projects over the rounding: 1e-12 as in the parity tes
 import numpy as np
 import pytest
 
+import oracle as O
 from _util import pair, rel_err, rel_err_rows, say
 from kitamr_hip import cases
+from kitamr_hip.solver import kah_params
 
 SHAPES = {
     "box": lambda: cases.box_3d(n=6, nv=12, ps_levels=1),
@@ -39,3 +41,35 @@ def test_steps_repeat(name):
     nw = case.config.solver.DIM + 2
     assert rel_err(g["df"], o["df"]) <= 1e-12
     assert rel_err_rows(g["w"].reshape(-1, nw), o["w"].reshape(-1, nw), nw) <= 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [6, 8, 12])
+def test_narrow_levels(n):
+    """Cells with a coarser neighbour on one side and finer ones on the other: the mean of the finer
+    midpoints is the cell's own up to rounding, so there is no projection on that side. Measured
+    against the oracle on the same mesh in units of its cells, where every midpoint is exact: slopes
+    to 1e-12 of the largest (differences of values alike in both, divided by sizes that round)."""
+    case = cases.riemann_2d(n=n, nv=8, ps_levels=2, halo=(2.0, 1.5, 1.0))
+    state = np.asarray(case.topo["nb_state"]).reshape(-1, 2, 2)
+    narrow = int(np.sum(np.any(state == -1, axis=2) & np.any(state == 2, axis=2)))
+    say(f"[slope order] narrow n={n}: cells={case.n_cells}, {narrow} between coarse and fine")
+    assert narrow > 0
+    # a factor per cell that is curved along both directions: slopes across the faces and along them
+    x, y = np.asarray(case.topo["cell_mid"]).reshape(-1, 2)[:case.n_cells].T
+    size = np.diff(np.asarray(case.topo["vs_offset"])) * 2
+    case.df = case.df * np.repeat(1.0 + 0.3 * np.sin(3.0 * x + 2.0 * y) + 0.2 * x * y, size)
+    dev, orc = pair(case)
+    for _ in range(2):   # the second sweep finds slopes in the finer cells
+        dev.slope(case.dt_xi)
+    g = dev.get_state(sdf=True)
+    dev.close()
+    orc.close()
+    topo = dict(case.topo)
+    for k in ("cell_mid", "cell_ds", "pair_mid"):
+        topo[k] = np.round(np.asarray(topo[k]) * n * 1024) / 1024
+    exact = O.Oracle(kah_params(case.config), topo)
+    exact.set_state(case.w, case.prim, case.df)
+    for _ in range(2):
+        exact.slope()
+    assert rel_err(g["sdf"], exact.get_state()["sdf"] * n) <= 1e-12
