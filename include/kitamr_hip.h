@@ -338,7 +338,8 @@ int64_t kah_device_bytes(const kah_ctx* ctx);
  * of one projection depth, flux/relaxation launches) are spread, forked from and joined back to
  * the context's stream by events (parallel branches of a captured graph). 1 to 3 hold for every
  * phase; 4, the default, is up to four where the shape of the case makes it pay (large meshes, and
- * adapted grids of some hundred velocity cells and up), else one.
+ * adapted grids of some hundred velocity cells and up; two for a small step outside a graph), else
+ * one.
  * No counterpart in the reference. */
 enum { KAH_OPT_FLUX_WAVES = 1, KAH_OPT_SLOPE_VPT = 2, KAH_OPT_VEL_TILES = 3,
        KAH_OPT_OVERLAP_MAPS = 4, KAH_OPT_GRAPHS = 5, KAH_OPT_REGULAR = 6,

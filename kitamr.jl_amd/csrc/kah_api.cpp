@@ -189,12 +189,19 @@ struct kah_ctx {
   // 520 79 / 74, 594 113 / 120, 811 341 / 361, 1651 107 / 120; FP32 form 316 76 / 74, 403 86 / 89,
   // 520 87 / 90, 594 127 / 157; 3D 552 96 / 116, 1247 133 / 176 and in the FP32 form 154 / 272. Large
   // meshes of small grids: 1.1 M 167 / 161, 1.6 M 182 / 197, 1.9 M 291 / 284, 2.1 M 151 / 164.
-  int step_branches() const {
+  // Launched one by one, a small step also waits for the host's calls of fork and join (ten for four
+  // streams): 12^2 leaves with grids of up to 1425 velocity cells (0.19 M) 142 us on four streams, 110
+  // on two, 125 in order. Below 0.8 M velocity cells it takes two streams, and the flux and iterate
+  // phases of a split step, which are short, none.
+  int step_branches(bool fused = true) const {
     if (branches < MAX_BRANCHES) return branches;
     const bool large = phase_cells >= (D == 2 ? 2000 : 768) * int64_t(1024);
     const bool grids = !uni && max_n >= (D == 3 ? 512 : f32 ? 384 : 768);
-    return large || grids ? MAX_BRANCHES : 1;
+    if (!large && !grids) return 1;
+    if (capturing || phase_cells >= 768 * int64_t(1024)) return MAX_BRANCHES;
+    return fused ? 2 : 1;
   }
+  bool capturing = false;   // the launches go into a graph
   hipStream_t side[MAX_BRANCHES - 1] = {};
   std::vector<hipEvent_t> ev_pool;   // fork/join events, reused step after step
   size_t ev_next = 0;
@@ -1855,7 +1862,7 @@ int run_flux_relax(kah_ctx* C, const DevArgs& A, int mode) {
                                    C->stream),
                    "cell prologue launch"));
   // the bins write disjoint cells and read only what the slope phase wrote
-  const int nb = std::min<int>(C->step_branches(), int(C->frbins.size()));
+  const int nb = std::min<int>(C->step_branches(mode == MODE_FUSED), int(C->frbins.size()));
   KAH_TRY(fork_branches(C, nb));
   for (size_t j = 0; j < C->frbins.size(); ++j) {
     const kah_ctx::FrBin* b = C->frbins[j];
@@ -2410,9 +2417,11 @@ int kah_step(kah_ctx* C, double dt, int64_t step, double* sum_res, double* sum_a
       hipGraph_t g = nullptr;
       KAH_TRY(C->hip(hipStreamBeginCapture(C->stream, hipStreamCaptureModeThreadLocal),
                      "hipStreamBeginCapture"));
+      C->capturing = true;
       int rc = run_slope(C, A);
       if (!rc) rc = run_ib(C, A);
       if (!rc) rc = run_flux_relax(C, A, MODE_FUSED);
+      C->capturing = false;
       hipError_t ec = hipStreamEndCapture(C->stream, &g);
       if (rc) {
         if (g) (void)hipGraphDestroy(g);
