@@ -130,8 +130,9 @@ struct kah_ctx {
   // launch of fewer than four irregular cells a CU, above the smallest class, on meshes whose largest
   // grids (above 2048 velocity cells) make the step wait for it: steps on 16 and on 8 waves 450 / 472
   // us on the 75^2 cylinder, 366 / 390 on 64^2, 170 / 181 on 16^2 leaves with 3.6k velocity cells, 203
-  // / 209 with 2.7k and 142 / 146 with 2.3k; with smaller ones the bulk beside it fills the GPU: 283 /
-  // 273 with 1.6k, 217 / 214 with 1.0k.
+  // / 209 with 2.7k and 142 / 146 with 2.3k. With smaller ones the bulk beside it fills the GPU (283 /
+  // 273 with 1.6k, 217 / 214 with 1.0k), unless the mesh has fewer than two cells a CU (400 leaves
+  // with 1.4k 103 / 104, 81 with 0.7k 102 / 104).
   // cells: those of the kind that run side by side
   int fr_waves = 0;
   int flux_waves(size_t lds, int64_t n, bool irregular, int64_t cells) const {
@@ -144,7 +145,8 @@ struct kah_ctx {
       }
       if (P.marching != KAH_MARCH_CAIDVM) return 8;
       if (D == 3) return lds == 0 || lds > 56 * 1024 ? 16 : 8;
-      return !f32 && irregular && cells < 4 * cus && n > 640 && max_n > 2048 ? 16 : 8;
+      return !f32 && irregular && cells < 4 * cus && n > 640 &&
+                     (max_n > 2048 || int64_t(fluid.size()) < 2 * cus) ? 16 : 8;
     }
     const int64_t by_lds = lds ? std::max<int64_t>(1, lds_cu / int64_t(lds + 1536)) : 32;
     const int regs = irregular ? 16 : 28, want = irregular || cip ? 12 : 20;
